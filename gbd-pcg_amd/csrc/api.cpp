@@ -132,8 +132,10 @@ struct Layout {
   bool reg = false;    // register-resident kernel
   bool bc = false;     // ... in the row-broadcast layout
   bool pair = false;   // ... running forward and adjoint together
+  int any = kAnyNone;  // ... for any stateSize (which instance)
   bool fused = true;   // its recurrence (the LDS kernel takes it from the flags)
   int nt = 256;        // threads per workgroup
+  RegVariant variant() const { return RegVariant{fused, bc, pair, any}; }
 };
 
 // A layout chosen for (dtype, n, N, recurrence, pairing, the config fields that
@@ -298,29 +300,56 @@ static int plan_single(int dtype, uint32_t n, uint32_t N, bool fused, uint32_t w
   return GBDPCG_OK;
 }
 
-// Register-resident kernel (either recurrence): reg_lpr(n) lanes per matrix row of
-// the owned knots plus one ghost knot each side.  Prefers 256 threads (one wave
-// per SIMD: every wave runs the uniform scalar work, so fewer waves cost less)
-// with up to 8 knots per workgroup; 512 threads when the knots need it, or when
-// only then do all workgroups fit one XCD (shared L2: XCD-local exchanges).
-// Returns GBDPCG_ERR_UNSUPPORTED when the shape does not suit this kernel.
-static int plan_single_reg(int dtype, uint32_t n, uint32_t N, uint32_t want_G, uint32_t kcap, Layout *L,
-                           int only_nt = 0, bool fused = true, bool bc = false, bool pair = false) {
-  const RegVariant rv{fused, bc, pair && fused && n <= 14};
-  if (!reg_supported((int)n, bc) || N < 4) return GBDPCG_ERR_UNSUPPORTED;
+// The instance for any stateSize that takes n at nt threads.
+static int any_set(uint32_t n, int nt) { return nt == 64 ? kAnyTiny : n <= 16 ? kAnyNarrow : kAnyWide; }
+
+// Checks that a register layout of G workgroups (c: kernel, threads, G, stride 0 =
+// one XCD when they fit there) can run co-resident and completes it.
+static int finish_reg_layout(int dtype, uint32_t n, uint32_t N, Layout *c) {
   DeviceInfo di;
   int rc = device_info(cur_dev(), &di);
   if (rc < 0) return rc;
+  const RegVariant rv = c->variant();
+  c->reg = true;
+  c->lds = reg_lds_bytes(dtype, n, ceil_div(N, c->G), c->nt, rv);
+  if (c->lds > di.max_lds) return GBDPCG_ERR_UNSUPPORTED;
+  HIPCHK(reg_prepare(dtype, (int)n, c->nt, c->lds, rv));
+  int occ = 0;
+  HIPCHK(reg_occupancy(dtype, (int)n, c->nt, c->lds, &occ, rv));
+  const uint32_t per_xcd = (uint32_t)(di.cus / kXcds) * (uint32_t)occ;
+  if (occ <= 0 || c->G > (uint32_t)di.cus * (uint32_t)occ || (c->stride == (uint32_t)kXcds && c->G > per_xcd))
+    return GBDPCG_ERR_UNSUPPORTED;
+  if (!c->stride) c->stride = c->G <= per_xcd ? (uint32_t)kXcds : 1u;
+  c->grid = c->G * c->stride;
+  return GBDPCG_OK;
+}
+
+// Register-resident kernel (either recurrence): two lanes (some layouts one) per
+// matrix row of the owned knots plus one ghost knot each side.  Prefers 256
+// threads (one wave per SIMD: every wave runs the uniform scalar work, so fewer
+// waves cost less) with up to 8 knots per workgroup; 512 threads when the knots
+// need it, or when only then do all workgroups fit one XCD (shared L2: XCD-local
+// exchanges).  any: the instances for any stateSize up to 32 instead of the fixed
+// sizes.  Returns GBDPCG_ERR_UNSUPPORTED when the shape does not suit this kernel.
+static int plan_single_reg(int dtype, uint32_t n, uint32_t N, uint32_t want_G, uint32_t kcap, Layout *L,
+                           int only_nt = 0, bool fused = true, bool bc = false, bool pair = false, bool any = false) {
+  if (any ? n > 32 : !reg_supported((int)n, bc) || N < 4) return GBDPCG_ERR_UNSUPPORTED;
   Layout spread;  // first layout found whose workgroups span several XCDs
   bool have_spread = false;
   for (int nt : {256, 512, 64}) {
     if (only_nt && nt != only_nt) continue;
     if (nt == 64 && (!bc || !only_nt)) continue;  // one-wave ranks: on request (or tuned)
-    if (!fused && nt == 512) continue;  // reference-recurrence instances: 64 and 256 threads
+    if (!any && !fused && nt == 512) continue;  // reference-recurrence instances: 64 and 256 threads
     // FP64 rows of n = 28 (and whole FP64 rows in the row-broadcast layout) need
     // more VGPRs than two waves per SIMD leave: one wave per SIMD only
-    if (dtype == GBDPCG_F64 && (n > 14 || bc) && nt > 256) continue;
-    const uint32_t kmax = reg_max_knots(dtype, n, nt, bc);
+    if (!any && dtype == GBDPCG_F64 && (n > 14 || bc) && nt > 256) continue;
+    Layout c;
+    c.bc = bc;
+    c.pair = pair && fused && n <= 14 && !any;
+    c.any = any ? any_set(n, nt) : kAnyNone;
+    c.fused = fused;
+    c.nt = nt;
+    const uint32_t kmax = reg_max_knots(dtype, n, nt, c.variant());
     if (kmax < 2) continue;
     uint32_t G = want_G;
     if (!G) {  // about 8 knots (or the cap) per workgroup, never fewer than 2
@@ -328,23 +357,11 @@ static int plan_single_reg(int dtype, uint32_t n, uint32_t N, uint32_t want_G, u
       G = std::min(ceil_div(N, target), N / 2);
     }
     if (G < 1 || N / G < 2 || ceil_div(N, G) > kmax || G > (uint32_t)kMaxWgsPerSystem) continue;
-    const size_t lds = reg_lds_bytes(dtype, n, ceil_div(N, G), nt, rv);
-    if (lds > di.max_lds) continue;
-    HIPCHK(reg_prepare(dtype, (int)n, nt, lds, rv));
-    int occ = 0;
-    HIPCHK(reg_occupancy(dtype, (int)n, nt, lds, &occ, rv));
-    const uint32_t per_xcd = (uint32_t)(di.cus / kXcds) * (uint32_t)occ;
-    if (occ <= 0 || G > (uint32_t)di.cus * (uint32_t)occ) continue;
-    Layout c;
     c.G = G;
-    c.lds = lds;
-    c.reg = true;
-    c.bc = bc;
-    c.pair = rv.pair;
-    c.fused = fused;
-    c.nt = nt;
-    c.stride = G <= per_xcd ? (uint32_t)kXcds : 1u;
-    c.grid = G * c.stride;
+    c.stride = 0;
+    const int rc = finish_reg_layout(dtype, n, N, &c);
+    if (rc == GBDPCG_ERR_UNSUPPORTED) continue;
+    if (rc < 0) return rc;
     if (c.stride == (uint32_t)kXcds) {
       *L = c;
       return GBDPCG_OK;
@@ -359,6 +376,39 @@ static int plan_single_reg(int dtype, uint32_t n, uint32_t N, uint32_t want_G, u
   return GBDPCG_OK;
 }
 
+// One workgroup for the whole system, the smallest that holds it: no exchange at
+// all, which is more than the smaller matvecs of several workgroups save at every
+// size that fits (microseconds per iteration, one workgroup against the best of
+// several, FP32: n = 14 N = 16 fused 0.96 / 1.36 and reference form 1.33 / 2.28,
+// n = 32 N = 8 1.28 / 1.90 and 1.60 / 2.69, n = 2 N = 30 on one wave 0.42 / 1.13
+// and 0.67 / 1.99; FP64 n = 28 N = 9 2.50 / 3.40 and 2.84 / 4.48).
+// GBDPCG_ERR_UNSUPPORTED when no workgroup holds it.
+static int plan_one_workgroup(int dtype, uint32_t n, uint32_t N, bool fused, bool pair, Layout *L) {
+  if (n > 32 || (fused && N < 2)) return GBDPCG_ERR_UNSUPPORTED;
+  for (int nt : {64, 256, 512}) {
+    const bool fixed = reg_supported((int)n) && N >= 4 && nt != 64 && (fused || nt == 256) &&
+                       !(dtype == GBDPCG_F64 && n > 14 && nt > 256);
+    Layout c;
+    // FP64 rows of n = 12 and 14 broadcast by DPP: 1.13 us per fused iteration at
+    // N = 14 where two lanes per row at 512 threads take 1.56 (reference form
+    // 1.41 against 2.13)
+    c.bc = fixed && nt == 256 && dtype == GBDPCG_F64 && reg_supported((int)n, true);
+    c.pair = pair && fused && n <= 14 && fixed;
+    c.any = fixed ? kAnyNone : any_set(n, nt);
+    c.fused = fused;
+    c.nt = nt;
+    if (c.any && !any_supported(n, nt, c.any)) continue;
+    if (N > reg_max_knots(dtype, n, nt, c.variant(), true)) continue;
+    c.G = 1;
+    c.stride = 0;
+    const int rc = finish_reg_layout(dtype, n, N, &c);
+    if (rc == GBDPCG_ERR_UNSUPPORTED) continue;
+    if (rc == GBDPCG_OK) *L = c;
+    return rc;
+  }
+  return GBDPCG_ERR_UNSUPPORTED;
+}
+
 // Layout of a single solve: the autotuner's choice for this shape when the config
 // leaves everything automatic, else the planners (register kernel first when the
 // recurrence is fused).
@@ -367,39 +417,52 @@ static std::string single_key(int dev, int dtype, uint32_t n, uint32_t N, bool f
          std::to_string(N) + ":" + std::to_string(fused ? 1 : 0) + ":" + std::to_string(exit_mode);
 }
 
-// Rebuilds a layout from its (kernel, threads, workgroups, stride); checks that it
+// Kinds of layout, as the tuner's choices name them (TuneChoice.a).
+enum : uint32_t { kKindLds = 0, kKindReg = 1, kKindRowcast = 2, kKindAny = 3 };
+static uint32_t kind_of(const Layout &L) {
+  return !L.reg ? kKindLds : L.bc ? kKindRowcast : L.any ? kKindAny : kKindReg;
+}
+
+// Rebuilds a layout from its (kind, threads, workgroups, stride); checks that it
 // still fits the device.
-static int layout_from(int dtype, uint32_t n, uint32_t N, bool reg, bool bc, int nt, uint32_t G,
-                       uint32_t stride, Layout *L, bool fused, bool pair = false) {
+static int layout_from(int dtype, uint32_t n, uint32_t N, uint32_t kind, int nt, uint32_t G, uint32_t stride,
+                       Layout *L, bool fused, bool pair = false) {
   DeviceInfo di;
   int rc = device_info(cur_dev(), &di);
   if (rc < 0) return rc;
-  if (G == 0 || G > N || (stride != 1 && stride != (uint32_t)kXcds)) return GBDPCG_ERR_UNSUPPORTED;
+  if (kind > kKindAny || G == 0 || G > N || (stride != 1 && stride != (uint32_t)kXcds)) return GBDPCG_ERR_UNSUPPORTED;
   Layout t;
   t.G = G;
   t.stride = stride;
   t.grid = G * stride;
-  t.reg = reg;
-  t.bc = reg && bc;
-  t.pair = reg && fused && pair && n <= 14;
+  t.reg = kind != kKindLds;
+  t.bc = kind == kKindRowcast;
+  t.any = kind == kKindAny ? any_set(n, nt) : kAnyNone;
+  t.pair = t.reg && !t.any && fused && pair && n <= 14;
   t.fused = fused;
-  const RegVariant rv{fused, t.bc, t.pair};
-  t.nt = reg ? nt : kThreads;
-  int occ = 0;
-  if (reg) {
-    if (!reg_supported((int)n, t.bc) || ceil_div(N, G) > reg_max_knots(dtype, n, nt, t.bc) || N / G < 2 ||
-        (!fused && nt == 512) || (nt == 64 && (!t.bc || t.pair)) || (t.bc && dtype == GBDPCG_F64 && nt == 512))
+  t.nt = t.reg ? nt : kThreads;
+  if (t.any) {
+    if (!any_supported(n, nt, t.any) || (nt == 64 && G != 1) || (fused && N < 2) || (G > 1 && N / G < 2) ||
+        ceil_div(N, G) > reg_max_knots(dtype, n, nt, t.variant(), G == 1))
       return GBDPCG_ERR_UNSUPPORTED;
-    t.lds = reg_lds_bytes(dtype, n, ceil_div(N, G), nt, rv);
-    if (t.lds > di.max_lds) return GBDPCG_ERR_UNSUPPORTED;
-    HIPCHK(reg_prepare(dtype, (int)n, nt, t.lds, rv));
-    HIPCHK(reg_occupancy(dtype, (int)n, nt, t.lds, &occ, rv));
-  } else {
-    t.lds = item_lds_bytes(n, ceil_div(N, G), G, tsize(dtype));
-    if (t.lds > di.max_lds) return GBDPCG_ERR_UNSUPPORTED;
-    rc = occupancy(dtype, t.lds, &occ);
-    if (rc < 0) return rc;
+    rc = finish_reg_layout(dtype, n, N, &t);
+    if (rc == GBDPCG_OK) *L = t;
+    return rc;
   }
+  if (t.reg) {
+    if (!reg_supported((int)n, t.bc) || ceil_div(N, G) > reg_max_knots(dtype, n, nt, t.variant(), G == 1) ||
+        N / G < 2 || (!fused && nt == 512) || (nt == 64 && (!t.bc || t.pair)) ||
+        (t.bc && dtype == GBDPCG_F64 && nt == 512))
+      return GBDPCG_ERR_UNSUPPORTED;
+    rc = finish_reg_layout(dtype, n, N, &t);
+    if (rc == GBDPCG_OK) *L = t;
+    return rc;
+  }
+  int occ = 0;
+  t.lds = item_lds_bytes(n, ceil_div(N, G), G, tsize(dtype));
+  if (t.lds > di.max_lds) return GBDPCG_ERR_UNSUPPORTED;
+  rc = occupancy(dtype, t.lds, &occ);
+  if (rc < 0) return rc;
   const uint32_t per_xcd = (uint32_t)(di.cus / kXcds) * (uint32_t)occ;
   if (occ <= 0 || G > (uint32_t)di.cus * (uint32_t)occ || (stride == (uint32_t)kXcds && G > per_xcd))
     return GBDPCG_ERR_UNSUPPORTED;
@@ -407,20 +470,25 @@ static int layout_from(int dtype, uint32_t n, uint32_t N, bool reg, bool bc, int
   return GBDPCG_OK;
 }
 
-static int choose_layout(int dev, int dtype, uint32_t n, uint32_t N, bool fused, const gbdpcg_config *cfg,
-                         Layout *L, bool pair = false) {
-  if (cfg->grid[0] == 0 && cfg->knots_per_wg == 0 && cfg->kernel == GBDPCG_KERNEL_AUTO) {
-    TuneChoice c;
-    if (cfg->threads == 0 && tune_lookup(single_key(dev, dtype, n, N, fused, cfg->exit_mode), &c) &&
-        layout_from(dtype, n, N, c.a != 0, c.a == 2, (int)c.b, c.c, c.d, L, fused, pair) == GBDPCG_OK)
-      return GBDPCG_OK;
-  }
-  // automatic: the row-broadcast layout first for FP64 (measured faster there),
-  // the column-chunk register layout first for FP32.  cfg->threads asks the
-  // register kernels for that many threads per workgroup.
+static int untuned_layout(int dtype, uint32_t n, uint32_t N, bool fused, const gbdpcg_config *cfg, Layout *L,
+                          bool pair) {
+  const bool open = cfg->grid[0] == 0 && cfg->knots_per_wg == 0;
+  // automatic: one workgroup when it holds the system; then the row-broadcast
+  // layout first for FP64 (measured faster there), the column-chunk register
+  // layout first for FP32; other stateSizes on the instances for any size.
+  // cfg->threads asks the register kernels for that many threads per workgroup.
   const int req_nt = (int)cfg->threads;
+  const bool fixed = reg_supported((int)n) && N >= 4;
+  if (cfg->kernel == GBDPCG_KERNEL_AUTO && !fixed) {
+    // every size the LDS-resident kernel takes, and no other: its plan decides
+    // what is refused and which solves run the reference iteration
+    const int rc = plan_single(dtype, n, N, fused, cfg->grid[0], cfg->knots_per_wg, L);
+    if (rc < 0) return rc;
+  }
   int rc = GBDPCG_ERR_UNSUPPORTED;
-  if ((cfg->kernel == GBDPCG_KERNEL_AUTO && dtype == GBDPCG_F64) || cfg->kernel == GBDPCG_KERNEL_ROWCAST)
+  if (cfg->kernel == GBDPCG_KERNEL_AUTO && open && req_nt == 0) rc = plan_one_workgroup(dtype, n, N, fused, pair, L);
+  if (rc == GBDPCG_ERR_UNSUPPORTED &&
+      ((cfg->kernel == GBDPCG_KERNEL_AUTO && dtype == GBDPCG_F64) || cfg->kernel == GBDPCG_KERNEL_ROWCAST))
     rc = plan_single_reg(dtype, n, N, cfg->grid[0], cfg->knots_per_wg, L, req_nt, fused, true, pair);
   if (rc == GBDPCG_ERR_UNSUPPORTED && cfg->kernel == GBDPCG_KERNEL_ROWCAST) {
     set_error("row-broadcast kernel needs n in {12,14}, N >= 4 and a fitting layout");
@@ -432,8 +500,21 @@ static int choose_layout(int dev, int dtype, uint32_t n, uint32_t N, bool fused,
     set_error("register kernel needs n in {2,6,12,14,28}, N >= 4 and a fitting layout");
     return GBDPCG_ERR_UNSUPPORTED;
   }
+  if (rc == GBDPCG_ERR_UNSUPPORTED && cfg->kernel == GBDPCG_KERNEL_AUTO && !fixed)
+    rc = plan_single_reg(dtype, n, N, cfg->grid[0], cfg->knots_per_wg, L, req_nt, fused, false, false, true);
   if (rc == GBDPCG_ERR_UNSUPPORTED) rc = plan_single(dtype, n, N, fused, cfg->grid[0], cfg->knots_per_wg, L);
   return rc;
+}
+
+static int choose_layout(int dev, int dtype, uint32_t n, uint32_t N, bool fused, const gbdpcg_config *cfg,
+                         Layout *L, bool pair = false) {
+  if (cfg->grid[0] == 0 && cfg->knots_per_wg == 0 && cfg->kernel == GBDPCG_KERNEL_AUTO && cfg->threads == 0) {
+    TuneChoice c;
+    if (tune_lookup(single_key(dev, dtype, n, N, fused, cfg->exit_mode), &c) &&
+        layout_from(dtype, n, N, c.a, (int)c.b, c.c, c.d, L, fused, pair) == GBDPCG_OK)
+      return GBDPCG_OK;
+  }
+  return untuned_layout(dtype, n, N, fused, cfg, L, pair);
 }
 
 // Whether the LDS-resident kernel cannot give every workgroup the 2 knots the
@@ -610,7 +691,7 @@ static int solve_locked(Workspace *ws, int dtype, uint32_t n, uint32_t N, const 
               exchange_flags(cfg);
   if (L.reg) {
     HIPCHK(reg_launch(dtype, (int)n, L.nt, one, nullptr, nullptr, 0, L.stride, L.grid, L.lds, stream,
-                      RegVariant{fused, L.bc, L.pair}));
+                      L.variant()));
   } else {
     HIPCHK(pcg_launch(dtype, one, nullptr, nullptr, 0, L.stride, L.grid, L.lds, stream));
   }
@@ -724,7 +805,13 @@ int solve_on_scratch(int dtype, uint32_t n, uint32_t N, const void *S, const voi
     rc = choose_layout(dev, dtype, n, N, false, cfg, &L, false);
   }
   if (rc < 0) return rc;
-  const size_t words = 2 * (size_t)L.G * rec_words(n, (uint32_t)(tsize(dtype) / 4));
+  size_t words = 2 * (size_t)L.G * rec_words(n, (uint32_t)(tsize(dtype) / 4));
+  if (L.any && words > scratch_words - kScratchHeaderWords) {
+    // long horizons: the LDS-resident kernel takes fewer workgroups, hence records
+    rc = plan_single(dtype, n, N, fused, cfg->grid[0], cfg->knots_per_wg, &(L = Layout()));
+    if (rc < 0) return rc;
+    words = 2 * (size_t)L.G * rec_words(n, (uint32_t)(tsize(dtype) / 4));
+  }
   if (words > scratch_words - kScratchHeaderWords) {
     set_error("n=%u N=%u needs %zu words of exchange records on %u workgroups; the no-allocation scratch holds "
               "%zu", n, N, words, L.G, scratch_words - kScratchHeaderWords);
@@ -751,7 +838,7 @@ int solve_on_scratch(int dtype, uint32_t n, uint32_t N, const void *S, const voi
               exchange_flags(cfg);
   if (L.reg) {
     HIPCHK(reg_launch(dtype, (int)n, L.nt, one, nullptr, nullptr, 0, L.stride, L.grid, L.lds, stream,
-                      RegVariant{fused, L.bc, false}));
+                      L.variant()));
   } else {
     HIPCHK(pcg_launch(dtype, one, nullptr, nullptr, 0, L.stride, L.grid, L.lds, stream));
   }
@@ -1030,24 +1117,23 @@ int gbdpcg_tune_single(int dtype, uint32_t n, uint32_t N, const void *d_S, const
   // candidates: the untuned default first, then every (kernel, threads, knots per
   // workgroup, XCD placement) that fits
   std::vector<Layout> cands;
+  bool unfit = false;
   auto add = [&](const Layout &L) {
     for (const Layout &c : cands)
-      if (c.reg == L.reg && c.bc == L.bc && c.nt == L.nt && c.G == L.G && c.stride == L.stride) return;
+      if (kind_of(c) == kind_of(L) && c.nt == L.nt && c.G == L.G && c.stride == L.stride) return;
     cands.push_back(L);
   };
   {
     Layout def;
-    rc = GBDPCG_ERR_UNSUPPORTED;
-    if ((cfg->kernel == GBDPCG_KERNEL_AUTO && dtype == GBDPCG_F64) || cfg->kernel == GBDPCG_KERNEL_ROWCAST)
-      rc = plan_single_reg(dtype, n, N, 0, 0, &def, 0, fused, true);
-    if (rc == GBDPCG_ERR_UNSUPPORTED && (cfg->kernel == GBDPCG_KERNEL_AUTO || cfg->kernel == GBDPCG_KERNEL_REGISTER))
-      rc = plan_single_reg(dtype, n, N, 0, 0, &def, 0, fused);
-    if (rc == GBDPCG_ERR_UNSUPPORTED && (cfg->kernel == GBDPCG_KERNEL_AUTO || cfg->kernel == GBDPCG_KERNEL_LDS))
-      rc = plan_single(dtype, n, N, fused, 0, 0, &def);
+    gbdpcg_config c = *cfg;  // the layout an untuned solve would take
+    c.grid[0] = 0;
+    c.knots_per_wg = c.threads = 0;
+    rc = untuned_layout(dtype, n, N, fused, &c, &def, false);
     if (rc == GBDPCG_ERR_TOO_LARGE && fused && lds_fused_unfit(dtype, n, N)) {
       // solves of this config run the reference iteration (solve_locked): tune
       // those layouts, cached under that recurrence's key, which they look up
       fused = false;
+      unfit = true;
       rc = plan_single(dtype, n, N, false, 0, 0, &def);
     }
     if (rc < 0) return rc;
@@ -1062,7 +1148,7 @@ int gbdpcg_tune_single(int dtype, uint32_t n, uint32_t N, const void *d_S, const
     TuneChoice c;
     Layout L;
     if (tune_lookup(single_key(dev, dtype, n, N, fused, cfg->exit_mode), &c) &&
-        layout_from(dtype, n, N, c.a != 0, c.a == 2, (int)c.b, c.c, c.d, &L, fused) == GBDPCG_OK) {
+        layout_from(dtype, n, N, c.a, (int)c.b, c.c, c.d, &L, fused) == GBDPCG_OK) {
       if (report) {
         gbdpcg_tune_report r{};
         r.from_cache = 1;
@@ -1077,20 +1163,25 @@ int gbdpcg_tune_single(int dtype, uint32_t n, uint32_t N, const void *d_S, const
   }
 
   const uint32_t Ks[] = {1, 2, 3, 4, 5, 6, 7, 8, 10, 12, 14, 16, 20, 24, 28, 32, 40, 48, 64};
-  // kind 2: row-broadcast register layout, 1: register, 0: LDS
-  for (int kind = 2; kind >= 0; --kind) {
-    const uint32_t kid = kind == 2 ? GBDPCG_KERNEL_ROWCAST : kind == 1 ? GBDPCG_KERNEL_REGISTER : GBDPCG_KERNEL_LDS;
+  for (const uint32_t kind : {(uint32_t)kKindRowcast, (uint32_t)kKindReg, (uint32_t)kKindAny, (uint32_t)kKindLds}) {
+    const uint32_t kid = kind == kKindRowcast ? GBDPCG_KERNEL_ROWCAST
+                         : kind == kKindLds   ? GBDPCG_KERNEL_LDS
+                                              : GBDPCG_KERNEL_REGISTER;
     if (cfg->kernel != GBDPCG_KERNEL_AUTO && cfg->kernel != kid) continue;
-    if (kind == 0 && cfg->threads) continue;  // a thread request names a register kernel
+    if (kind == kKindLds && cfg->threads) continue;  // a thread request names a register kernel
+    // the instances for any size: automatic solves of the sizes without instances
+    // of their own, and systems of one workgroup
+    if (kind == kKindAny && (cfg->kernel != GBDPCG_KERNEL_AUTO || unfit)) continue;
     for (int nt : {256, 512, 64}) {
-      if (!kind && nt != kThreads) continue;
-      if (nt == 64 && kind != 2) continue;  // one-wave ranks: row-broadcast layout only
+      if (kind == kKindLds && nt != kThreads) continue;
+      if (nt == 64 && kind != kKindRowcast && kind != kKindAny) continue;  // one-wave workgroups
       for (uint32_t K : Ks) {
         const uint32_t G = ceil_div(N, K);
         if (G > (uint32_t)kMaxWgsPerSystem || (fused && N / G < 2)) continue;
+        if (kind == kKindAny && G > 1 && reg_supported((int)n) && N >= 4) continue;
         for (uint32_t stride : {(uint32_t)kXcds, 1u}) {
           Layout L;
-          if (layout_from(dtype, n, N, kind != 0, kind == 2, nt, G, stride, &L, fused) == GBDPCG_OK) add(L);
+          if (layout_from(dtype, n, N, kind, nt, G, stride, &L, fused) == GBDPCG_OK) add(L);
         }
       }
     }
@@ -1161,7 +1252,7 @@ int gbdpcg_tune_single(int dtype, uint32_t n, uint32_t N, const void *d_S, const
       if ((e = hipMemsetAsync(lam, 0, (size_t)n * N * ts, st)) != hipSuccess) return fail("hipMemsetAsync", e);
       if ((e = hipEventRecord(ea, st)) != hipSuccess) return fail("hipEventRecord", e);
       e = L.reg ? reg_launch(dtype, (int)n, L.nt, one, nullptr, nullptr, 0, L.stride, L.grid, L.lds, st,
-                             RegVariant{fused, L.bc, false})
+                             L.variant())
                 : pcg_launch(dtype, one, nullptr, nullptr, 0, L.stride, L.grid, L.lds, st);
       if (e != hipSuccess) return fail("solve launch", e);
       if ((e = hipEventRecord(eb, st)) != hipSuccess) return fail("hipEventRecord", e);
@@ -1197,7 +1288,7 @@ int gbdpcg_tune_single(int dtype, uint32_t n, uint32_t N, const void *d_S, const
   const Layout &B = cands[best];
   if (open_cfg)
     tune_store(single_key(dev, dtype, n, N, fused, cfg->exit_mode),
-               TuneChoice{B.bc ? 2u : B.reg ? 1u : 0u, (uint32_t)B.nt, B.G, B.stride});
+               TuneChoice{kind_of(B), (uint32_t)B.nt, B.G, B.stride});
   if (report) {
     gbdpcg_tune_report r{};
     r.candidates = timed;

@@ -40,12 +40,15 @@ struct BatchLaunch {
   bool reg = false;    // register-resident kernel (else LDS-resident)
   bool bc = false;     // ... in the row-broadcast layout
   bool pair = false;   // ... with forward + adjoint systems iterated together
+  int any = kAnyNone;  // ... for any stateSize (which instance)
+  bool fused = true;   // recurrence of a register launch
   int kn = 0;          // stateSize specialisation (0 = runtime dispatch)
   int nt = 256;        // threads per workgroup
   uint32_t grid = 0, rounds = 0, occ = 0, items = 0, systems = 0;
   size_t lds = 0;
   size_t item_off = 0;  // offset of this launch's rounds x grid items in d_items
   double makespan = 0.0;
+  RegVariant variant() const { return RegVariant{fused, bc, pair, any}; }
 };
 
 struct gbdpcg_batch {
@@ -155,27 +158,30 @@ int plan_launch(int dtype, const gbdpcg_system_desc *systems, const std::vector<
                 std::vector<uint32_t> &G, std::vector<uint8_t> &fused, std::vector<uint32_t> &items) {
   const size_t ts = tsize(dtype);
   const bool fused_cfg = cfg->recurrence == GBDPCG_RECUR_FUSED;
-  const RegVariant rv{true, L.bc, L.pair};
+  const RegVariant rv = L.variant();
   size_t lds = 0;
   // cfg->knots_per_wg caps the knots per workgroup (the autotuner's main knob)
   const uint32_t kcap = cfg->knots_per_wg ? std::max<uint32_t>(cfg->knots_per_wg, 1u) : 0u;
   for (uint32_t i : idx) {
     const gbdpcg_system_desc &d = systems[i];
     if (L.reg) {
-      const uint32_t kmax = reg_max_knots(dtype, d.n, L.nt, L.bc);
+      const uint32_t kmax = reg_max_knots(dtype, d.n, L.nt, rv);
+      const uint32_t alone = reg_max_knots(dtype, d.n, L.nt, rv, true);
       const uint32_t target = kcap ? std::min(kmax, std::max<uint32_t>(kcap, 2u)) : kmax;
       uint32_t g = d.wgs;
-      if (!g) {  // the cap is a target: every workgroup keeps at least 2 knots
+      if (!g && d.N <= alone && (!kcap || d.N <= std::max<uint32_t>(kcap, 2u))) g = 1;  // no exchange
+      if (!g && target) {  // the cap is a target: every workgroup keeps at least 2 knots
         g = (d.N + target - 1) / target;
         g = std::min(g, std::max<uint32_t>(d.N / 2, 1u));
       }
-      if (g == 0 || (d.N + g - 1) / g > kmax || d.N / g < 2 || g > (uint32_t)kMaxWgsPerSystem) {
+      if (g == 0 || (d.N + g - 1) / g > (g == 1 ? alone : kmax) || (d.N / g < 2 && (rv.fused || g > 1)) ||
+          g > (uint32_t)kMaxWgsPerSystem) {
         set_error("system %u: %u workgroups do not suit the register kernel (N=%u, 2..%u knots each)", i, g, d.N,
                   kmax);
         return GBDPCG_ERR_TOO_LARGE;
       }
       G[i] = g;
-      fused[i] = 1;
+      fused[i] = rv.fused;
       lds = std::max(lds, reg_lds_bytes(dtype, d.n, (d.N + g - 1) / g, L.nt, rv));
     } else {
       uint32_t kmax = max_knots(d.n, d.N, ts, budget);
@@ -433,8 +439,32 @@ int gbdpcg_batch_create(gbdpcg_batch **out, int dtype, const gbdpcg_system_desc 
   std::vector<uint32_t> G(count, 0), items;
   std::vector<uint8_t> fused(count, 0);
   for (size_t li = 0; li < launches.size(); ++li) {
+    const size_t at = items.size();
     const int rc = plan_launch(dtype, systems, members[li], cfg, prop, budget, launches[li], G, fused, items);
     if (rc < 0) return rc;
+    if (launches[li].reg || cfg->kernel != GBDPCG_KERNEL_AUTO) continue;
+    // What the LDS-resident kernel takes (its plan decides what is refused and
+    // which recurrence a system runs) goes to the register kernel for any
+    // stateSize when that holds every system of the launch with the recurrence
+    // asked for: rows in registers, several times the LDS kernel's rate.
+    BatchLaunch R;
+    R.reg = true;
+    R.fused = fused_cfg;
+    bool fits = true, narrow = true;
+    for (uint32_t i : members[li]) {
+      fits = fits && systems[i].n <= 32 && (fused[i] != 0) == fused_cfg;
+      narrow = narrow && systems[i].n <= 16;
+    }
+    R.any = narrow ? kAnyNarrow : kAnyAll;
+    R.nt = narrow && want256 ? 256 : 512;
+    if (!fits) continue;
+    std::vector<uint32_t> rG = G, ritems(items.begin(), items.begin() + at);
+    std::vector<uint8_t> rfused = fused;
+    if (plan_launch(dtype, systems, members[li], cfg, prop, budget, R, rG, rfused, ritems) != GBDPCG_OK) continue;
+    launches[li] = R;
+    G.swap(rG);
+    fused.swap(rfused);
+    items.swap(ritems);
   }
 
   // device state
@@ -528,7 +558,7 @@ int gbdpcg_batch_run(gbdpcg_batch *plan, void *stream) {
   for (const BatchLaunch &L : plan->launches) {
     if (L.reg) {
       HIPCHK(reg_launch(plan->dtype, L.kn, L.nt, dummy, plan->d_sys, plan->d_items + L.item_off, L.rounds, 1, L.grid,
-                        L.lds, st, RegVariant{true, L.bc, L.pair}));
+                        L.lds, st, L.variant()));
     } else {
       HIPCHK(pcg_launch(plan->dtype, dummy, plan->d_sys, plan->d_items + L.item_off, L.rounds, 1, L.grid, L.lds,
                         st));

@@ -71,6 +71,19 @@ __host__ __device__ constexpr uint32_t reg_chunk(uint32_t n, uint32_t lpr) {
   return 4u * ((3u * padded_n(n) + 4u * lpr - 1u) / (4u * lpr));
 }
 
+// Register kernels for any stateSize up to 32 (pcg_any_kernel): the classes of
+// padded stateSizes one instance holds, and its lanes per row.
+enum : int {
+  kAnyNone = 0,
+  kAnyTiny = 1,    // n <= 8, one lane per row, 64 threads: systems of one wave
+  kAnyNarrow = 2,  // n <= 16, two lanes per row
+  kAnyWide = 3,    // 16 < n <= 32, two lanes per row
+  kAnyAll = 4,     // n <= 32: batches of mixed sizes
+};
+__host__ __device__ constexpr int any_lpr(int set, int tsize) {
+  return set == kAnyTiny || (set == kAnyAll && tsize == 4) ? 1 : 2;
+}
+
 // Words (64-bit) of one exchange record: kRecScalars scalar slots (3 per wave of
 // the publishing workgroup, up to 8 waves) + two edge blocks, each a left edge
 // (2 knots of n) + a right edge (2 knots of n); single solves use the first
@@ -159,10 +172,14 @@ struct RegVariant {
   bool fused = true;  // fused recurrence; false: reference recurrence (256 threads only)
   bool bc = false;    // row-broadcast layout (pcg_rowcast_kernel.hip, n in {12, 14})
   bool pair = false;  // forward + adjoint items iterated together (pcg_pair_kernel_*.hip)
+  int any = kAnyNone; // any stateSize up to 32 (pcg_any_*.hip): which instance
 };
 bool reg_supported(int n, bool bc = false);
+bool any_supported(uint32_t n, int nt, int set);
 size_t reg_lds_bytes(int dtype, uint32_t n, uint32_t K, int nt, RegVariant v = {});
-uint32_t reg_max_knots(int dtype, uint32_t n, int nt, bool bc = false);
+// Largest knots per workgroup of a layout; of a system's only workgroup when
+// alone (no ghost rows then).
+uint32_t reg_max_knots(int dtype, uint32_t n, int nt, RegVariant v = {}, bool alone = false);
 hipError_t reg_prepare(int dtype, int n, int nt, size_t lds, RegVariant v = {});
 hipError_t reg_occupancy(int dtype, int n, int nt, size_t lds, int *wgs_per_cu, RegVariant v = {});
 hipError_t reg_launch(int dtype, int n, int nt, const KSys &one, const KSys *systems, const uint32_t *items,
@@ -171,6 +188,10 @@ hipError_t reg_launch(int dtype, int n, int nt, const KSys &one, const KSys *sys
 const void *rowcast_kernel_ptr(int dtype, int n, int nt, bool fused);
 const void *pair_kernel_ptr_f32(int n, int nt, bool bc);
 const void *pair_kernel_ptr_f64(int n, int nt, bool bc);
+const void *any_fused_kernel_ptr_f32(int nt, int set);
+const void *any_fused_kernel_ptr_f64(int nt, int set);
+const void *any_ref_kernel_ptr_f32(int nt, int set);
+const void *any_ref_kernel_ptr_f64(int nt, int set);
 // pcg_reg_ref_kernel.hip: reference-recurrence kernel for (dtype, n, threads), or null
 const void *reg_ref_kernel_ptr(int dtype, int n, int nt);
 // tune.cpp: autotuner choice cache (a..d: meaning fixed by the key's kind)

@@ -1,0 +1,27 @@
+// Register-resident PCG kernels for any stateSize up to 32, float reference-recurrence
+// instances (the kernel is in pcg_reg_impl.h): 64 threads (systems of one wave),
+// 256 and 512 (single solves and batches).
+#include "pcg_reg_impl.h"
+
+namespace gbdpcg {
+
+namespace {
+template <int NT, int SET>
+const void *ap() {
+  return reinterpret_cast<const void *>(&pcg_any_kernel<float, NT, false, SET>);
+}
+}  // namespace
+
+const void *any_ref_kernel_ptr_f32(int nt, int set) {
+  if (nt == 64) return set == kAnyTiny ? ap<64, kAnyTiny>() : nullptr;
+  if (nt == 256) return set == kAnyNarrow ? ap<256, kAnyNarrow>() : set == kAnyWide ? ap<256, kAnyWide>() : nullptr;
+  if (nt != 512) return nullptr;
+  switch (set) {
+    case kAnyNarrow: return ap<512, kAnyNarrow>();
+    case kAnyWide: return ap<512, kAnyWide>();
+    case kAnyAll: return ap<512, kAnyAll>();
+    default: return nullptr;
+  }
+}
+
+}  // namespace gbdpcg

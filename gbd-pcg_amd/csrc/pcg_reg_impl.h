@@ -60,17 +60,33 @@ __device__ __forceinline__ T waves_total(const T *wsum, int l) {
   }
 }
 
+// stateSize of an item: a constant (RT false), or read from the system.
+template <int NS, bool RT>
+struct StateSize {
+  static constexpr int n = NS;
+  __device__ __forceinline__ void set_n(int) {}
+};
+template <int NS>
+struct StateSize<NS, true> {
+  int n;
+  __device__ __forceinline__ void set_n(int v) { n = v; }
+};
+
 // Status of one exchange within the item (all threads agree after a gather).
 // BC: row-broadcast layout (one lane per matrix row, 16 lanes per knot, every
 // lane holding its whole row of 3n columns).
-template <typename T, int NS, int NT, bool BC = false>
-struct RegItem {
-  static constexpr int n = NS;
+// LP > 0: any stateSize n <= NS with padded_n(n) == NS (a multiple of 4), LP
+// lanes per row.  Vectors and chunks have the compile-time stride NS, so the
+// matvecs are those of a fixed size; lanes, records and HBM offsets follow n.
+template <typename T, int NS, int NT, bool BC = false, int LP = 0>
+struct RegItem : StateSize<NS, (LP > 0)> {
+  static constexpr bool RT = LP > 0;
+  using StateSize<NS, RT>::n;
   static constexpr int nP = (int)padded_n(NS);
-  static constexpr int LPR = BC ? 1 : (int)reg_lpr(NS, NT, (int)sizeof(T));  // lanes per matrix row
+  static_assert(!RT || (nP == NS && !BC), "runtime stateSizes: column chunks, NS a multiple of 4");
+  static constexpr int LPR = BC ? 1 : RT ? LP : (int)reg_lpr(NS, NT, (int)sizeof(T));  // lanes per matrix row
   static constexpr int CW = BC ? 3 * NS : (int)reg_chunk(NS, LPR);           // columns per lane
   static constexpr int WPV = (int)(sizeof(T) / 4);
-  static constexpr int RW = (int)rec_words(NS, WPV);
   static constexpr int NWAVES = NT / 64;
 
   // geometry
@@ -90,7 +106,7 @@ struct RegItem {
   int *ctl;
 
   __device__ __forceinline__ uint64_t *rec(int type, int g) const {
-    return slots + (size_t)(type * G + g) * RW;
+    return slots + (size_t)(type * G + g) * rec_words((uint32_t)n, WPV);
   }
 
   // Owner lanes publish their value into the edge slots of the current exchange
@@ -188,13 +204,13 @@ struct RegItem {
                                             uint32_t *&dst) const {
     if (i < nleft) {  // left neighbour's right edge: knot a-1-e = local 1-e
       const int vi = i / WPV, qq = i - vi * WPV;
-      const int e = vi / n, rr = vi - e * n;
+      const int e = vi >= n ? 1 : 0, rr = vi - e * n;
       src = rec(type, rank - 1) + (kRecScalars + voff + 2 * n + e * n + rr) * WPV + qq;
       dst = reinterpret_cast<uint32_t *>(vec + (1 - e) * nP + rr) + qq;
     } else {  // right neighbour's left edge: knot b+e = local K+2+e
       const int ii = i - nleft;
       const int vi = ii / WPV, qq = ii - vi * WPV;
-      const int e = vi / n, rr = vi - e * n;
+      const int e = vi >= n ? 1 : 0, rr = vi - e * n;
       src = rec(type, rank + 1) + (kRecScalars + voff + e * n + rr) * WPV + qq;
       dst = reinterpret_cast<uint32_t *>(vec + (K + 2 + e) * nP + rr) + qq;
     }
@@ -551,7 +567,7 @@ __device__ __forceinline__ T group_sum(T v) {
 
 // Loads this lane's chunk of row `row` of block row kg of a cbtd matrix
 // (padded row-major columns [c*CW, (c+1)*CW) of the n x 3nP block row).
-constexpr int kLoadTables = 0, kLoadArith = 1, kLoadGuarded = 2, kLoadRows = 3;
+constexpr int kLoadTables = 0, kLoadArith = 1, kLoadGuarded = 2, kLoadRows = 3, kLoadAny = 4;
 
 // Per-chunk column tables of a block row (lane chunk c of CW padded columns):
 // the element offset of each column (0 for a padded column) and bit masks of
@@ -589,16 +605,44 @@ __host__ __device__ constexpr ChunkTables<NS, CW> chunk_tables() {
 // than they save (the paired kernel's 128-VGPR allocation, the runtime-n
 // instances); kLoadRows: whole rows (one lane per row, CW = 3 nP), whose guards
 // are uniform over each block of n columns: one branch per block (the n = 28
-// one-lane-per-row instances).
+// one-lane-per-row instances).  kLoadAny: branch-free for a stateSize known at
+// run time only: the offsets are uniform per column and chunk, the masks combine
+// per-lane flags with uniform column tests.
 template <typename T, int NS, int CW, int MODE = kLoadTables>
 __device__ __forceinline__ void load_chunk(T (&dst)[CW], const T *__restrict__ A, int kg, int row, int c, int N,
-                                           bool active) {
+                                           bool active, int n_rt = 0) {
   constexpr int n = NS, nP = (int)padded_n(NS);
   // opaque copies: keeps the per-lane offsets below from being hoisted out of the
   // batched item loop (they would stay live, in registers, for the whole solve)
   int cl = c, rl = row;
   asm volatile("" : "+v"(cl), "+v"(rl));
-  if constexpr (MODE == kLoadRows) {
+  if constexpr (MODE == kLoadAny) {
+    // one or two chunks per row: the block and the column within it of element j
+    // are constants of the chunk
+    static_assert(3 * nP <= 2 * CW, "at most two chunks per row");
+    const bool mid = active && kg >= 0 && kg < N;
+    const bool ok3[3] = {mid && kg > 0, mid, mid && kg < N - 1};
+    const uint32_t base = mid ? (uint32_t)kg * (uint32_t)(3 * n_rt * n_rt) + (uint32_t)rl : 0u;
+    const bool c1 = cl != 0;
+#pragma unroll
+    for (int j = 0; j < CW; ++j) {
+      const int s0 = j / nP, k0 = j % nP, s1 = (CW + j) / nP, k1 = (CW + j) % nP;
+      const bool v0 = s0 < 3 && k0 < n_rt, v1 = s1 < 3 && k1 < n_rt;  // uniform
+      const uint32_t o0 = v0 ? (uint32_t)((s0 * n_rt + k0) * n_rt) : 0u;
+      const uint32_t o1 = v1 ? (uint32_t)((s1 * n_rt + k1) * n_rt) : 0u;
+      bool ok;
+      uint32_t off;
+      if constexpr (CW >= 3 * nP) {  // one lane per row
+        ok = v0 && ok3[s0 < 3 ? s0 : 2];
+        off = o0;
+      } else {
+        ok = c1 ? (v1 && ok3[s1 < 3 ? s1 : 2]) : (v0 && ok3[s0 < 3 ? s0 : 2]);
+        off = c1 ? o1 : o0;
+      }
+      const T v = gptr(A)[ok ? base + off : 0u];
+      dst[j] = ok ? v : (T)0;
+    }
+  } else if constexpr (MODE == kLoadRows) {
     static_assert(CW == 3 * nP, "whole-row loads");
     const bool rowok = active && kg >= 0 && kg < N;
 #pragma unroll
@@ -761,9 +805,9 @@ __device__ __forceinline__ bool finite_t(double v) { return __builtin_isfinite(v
 
 // One matvec row pass: this lane's row of a resident block row times the vector
 // window of knots m-1..m+1 (local knots m..m+2) of `vec`; 0 on inactive lanes.
-template <typename T, int NS, int NT, bool BC, int CW>
-__device__ __forceinline__ T row_mv(const RegItem<T, NS, NT, BC> &it, const T (&mat)[CW], const T *vec, bool act) {
-  using R = RegItem<T, NS, NT, BC>;
+template <typename T, int NS, int NT, bool BC, int LP, int CW>
+__device__ __forceinline__ T row_mv(const RegItem<T, NS, NT, BC, LP> &it, const T (&mat)[CW], const T *vec, bool act) {
+  using R = RegItem<T, NS, NT, BC, LP>;
   if constexpr (BC) {
     // every lane of the 16-lane row takes part in the broadcasts; lanes past the
     // window read (and discard) the last knot's entries
@@ -894,11 +938,14 @@ __device__ __forceinline__ void write_gS(T *gS, const T *gg, const T *lam, int a
 // own set-up reads together).
 // BF: the matrix chunks loaded branch-free (load_chunk), for the fixed-size
 // instances; the runtime-n instances keep the guarded loads.
-template <typename T, int NS, int NT, bool FUSED, bool BC = false, bool PRE = true, bool BF = PRE>
+// LP: lanes per row of the runtime-stateSize items (RegItem), 0 for fixed sizes.
+template <typename T, int NS, int NT, bool FUSED, bool BC = false, bool PRE = true, bool BF = PRE, int LP = 0>
 __device__ __forceinline__ void reg_item(const KSys &d, uint32_t rank, T *lds) {
-  using R = RegItem<T, NS, NT, BC>;
-  constexpr int n = R::n, nP = R::nP, CW = R::CW;
+  using R = RegItem<T, NS, NT, BC, LP>;
+  constexpr int nP = R::nP, CW = R::CW;
   R it;
+  it.set_n((int)d.n);
+  const int n = it.n;
   it.N = (int)d.N;
   it.G = (int)d.G;
   it.rank = (int)rank;
@@ -921,14 +968,16 @@ __device__ __forceinline__ void reg_item(const KSys &d, uint32_t rank, T *lds) {
     it.m = t >> 4;
     it.row = t & 15;
   } else {
-    it.m = it.q / n;
-    it.row = it.q - it.m * n;
+    const int kq = it.q / n;
+    it.row = it.q - kq * n;
+    // one rank has no neighbours: no lanes for ghost rows, so it holds two knots more
+    it.m = kq + (it.G == 1 ? 1 : 0);
   }
   it.kg = it.a - 1 + it.m;
   it.act_u = it.m < K + 2 && (!BC || it.row < n);
   it.act_w = it.m >= 1 && it.m <= K && (!BC || it.row < n);
   it.owner = it.act_w && it.c == 0;
-  it.ghost = it.c == R::LPR - 1 && it.q < 4 * n;
+  it.ghost = it.c == R::LPR - 1 && it.q < 4 * n && it.G > 1;
   it.set_edge_slots();
   {
     const int gk = it.q / n, gr = it.q - (it.q / n) * n;  // ghost element q: knot slot 0..3
@@ -991,7 +1040,7 @@ __device__ __forceinline__ void reg_item(const KSys &d, uint32_t rank, T *lds) {
   // layouts); the runtime-n and n = 28 instances keep the guarded form, whose
   // fewer live masks leave their batches faster
   constexpr bool kGuarded = !(BF && NS <= 14);
-  constexpr int kMode = kGuarded ? (R::LPR == 1 && CW == 3 * nP ? kLoadRows : kLoadGuarded)
+  constexpr int kMode = R::RT ? kLoadAny : kGuarded ? (R::LPR == 1 && CW == 3 * nP ? kLoadRows : kLoadGuarded)
                                  : (sizeof(T) == 4 && NT == 256) ? kLoadTables : kLoadArith;
   // S first: loads complete in issue order, so the first product r = b - S x
   // (and the first exchange) can start while the Pinv chunks are in flight
@@ -999,8 +1048,8 @@ __device__ __forceinline__ void reg_item(const KSys &d, uint32_t rank, T *lds) {
     load_row<T, NS, kGuarded>(mS, static_cast<const T *>(d.S), kg, row, it.N, it.act_w);
     load_row<T, NS, kGuarded>(mM, static_cast<const T *>(d.Pinv), kg, row, it.N, it.act_u);
   } else {
-    load_chunk<T, NS, CW, kMode>(mS, static_cast<const T *>(d.S), kg, row, c, it.N, it.act_w);
-    load_chunk<T, NS, CW, kMode>(mM, static_cast<const T *>(d.Pinv), kg, row, c, it.N, it.act_u);
+    load_chunk<T, NS, CW, kMode>(mS, static_cast<const T *>(d.S), kg, row, c, it.N, it.act_w, n);
+    load_chunk<T, NS, CW, kMode>(mM, static_cast<const T *>(d.Pinv), kg, row, c, it.N, it.act_u, n);
   }
   __syncthreads();
   it.base = (uint32_t)it.ctl[1];
@@ -1878,6 +1927,63 @@ pcg_pair_kernel(KSys one, const KSys *__restrict__ systems,
     __syncthreads();
     const KSys d = systems[item >> 12];
     pair_dispatch<T, NS, NT, BC>(d, item & 0xFFFu, lds);
+  }
+}
+
+// Any stateSize up to 32: an item runs as the class of its padded size (n
+// rounded up to 4), any_lpr lanes per row.  Bound by the same chain of on-chip
+// latencies as the fixed sizes; a class costs the multiply-adds and registers of
+// its padding only.  Against the LDS-resident kernel, which ran these sizes (one
+// solve, microseconds per iteration): n = 13 N = 50 FP32 reference form 2.35
+// (4.1), fused 1.61 (2.9), FP64 3.31 (4.2) and 2.15 (3.2); n = 24 N = 60 FP32
+// 2.65 (4.1) and 1.78 (3.5); a batch of 96 systems of ten sizes n <= 31, FP32
+// reference form, 168 us (1,081).  SET names the classes one kernel
+// holds and with them its registers: the tiny and narrow ones serve systems of
+// n <= 8 and n <= 16, the wide one larger ones, kAnyAll batches of mixed sizes.
+template <typename T, int NT, bool FUSED, int SET>
+__device__ __forceinline__ void any_dispatch(const KSys &d, uint32_t rank, T *lds) {
+  constexpr int LP = any_lpr(SET, (int)sizeof(T));
+  constexpr bool kLow = SET != kAnyWide, kMid = SET == kAnyNarrow || SET == kAnyAll,
+                 kHigh = SET == kAnyWide || SET == kAnyAll;
+  switch (padded_n(d.n)) {
+    case 4: if constexpr (kLow) reg_item<T, 4, NT, FUSED, false, true, true, LP>(d, rank, lds); break;
+    case 8: if constexpr (kLow) reg_item<T, 8, NT, FUSED, false, true, true, LP>(d, rank, lds); break;
+    case 12: if constexpr (kMid) reg_item<T, 12, NT, FUSED, false, true, true, LP>(d, rank, lds); break;
+    case 16: if constexpr (kMid) reg_item<T, 16, NT, FUSED, false, true, true, LP>(d, rank, lds); break;
+    case 20: if constexpr (kHigh) reg_item<T, 20, NT, FUSED, false, true, true, LP>(d, rank, lds); break;
+    case 24: if constexpr (kHigh) reg_item<T, 24, NT, FUSED, false, true, true, LP>(d, rank, lds); break;
+    case 28: if constexpr (kHigh) reg_item<T, 28, NT, FUSED, false, true, true, LP>(d, rank, lds); break;
+    case 32: if constexpr (kHigh) reg_item<T, 32, NT, FUSED, false, true, true, LP>(d, rank, lds); break;
+    default: break;  // the planner only admits the sizes above
+  }
+}
+
+// Waves per SIMD as for the fixed sizes: FP32 rows of n <= 16 at 512 threads
+// leave room for a second workgroup on the CU.
+template <typename T, int NT, int SET>
+constexpr int any_waves_per_eu() {
+  return (sizeof(T) == 4 && NT == 512 && SET == kAnyNarrow) ? 4 : 1;
+}
+
+template <typename T, int NT, bool FUSED, int SET>
+__global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(any_waves_per_eu<T, NT, SET>())))
+pcg_any_kernel(KSys one, const KSys *__restrict__ systems, const uint32_t *__restrict__ items, uint32_t rounds,
+               uint32_t stride) {
+  extern __shared__ __attribute__((aligned(16))) unsigned char lds_raw[];
+  T *lds = reinterpret_cast<T *>(lds_raw);
+  if (systems == nullptr) {
+    if (blockIdx.x % stride) return;
+    const uint32_t rank = blockIdx.x / stride;
+    if (rank >= one.G) return;
+    any_dispatch<T, NT, FUSED, SET>(one, rank, lds);
+    return;
+  }
+  for (uint32_t rd = 0; rd < rounds; ++rd) {
+    const uint32_t item = items[(size_t)rd * gridDim.x + blockIdx.x];
+    if (item == kNoItem) continue;
+    __syncthreads();
+    const KSys d = systems[item >> 12];
+    any_dispatch<T, NT, FUSED, SET>(d, item & 0xFFFu, lds);
   }
 }
 

@@ -35,6 +35,9 @@ const void *reg_ptr_n(int n) {
 }
 
 const void *reg_kernel(int dtype, int n, int nt, RegVariant v) {
+  if (v.any && dtype == GBDPCG_F64)
+    return v.fused ? any_fused_kernel_ptr_f64(nt, v.any) : any_ref_kernel_ptr_f64(nt, v.any);
+  if (v.any) return v.fused ? any_fused_kernel_ptr_f32(nt, v.any) : any_ref_kernel_ptr_f32(nt, v.any);
   if (v.pair) {
     if (!v.fused) return nullptr;
     return dtype == GBDPCG_F64 ? pair_kernel_ptr_f64(n, nt, v.bc) : pair_kernel_ptr_f32(n, nt, v.bc);
@@ -52,11 +55,27 @@ bool reg_supported(int n, bool bc) {
   return n == 2 || n == 6 || n == 12 || n == 14 || n == 28;
 }
 
+// Whether an instance for any stateSize takes n at nt threads per workgroup.
+bool any_supported(uint32_t n, int nt, int set) {
+  switch (set) {
+    case kAnyTiny: return n <= 8 && nt == 64;
+    case kAnyNarrow: return n <= 16 && (nt == 256 || nt == 512);
+    case kAnyWide: return n > 16 && n <= 32 && (nt == 256 || nt == 512);
+    case kAnyAll: return n <= 32 && nt == 512;
+    default: return false;
+  }
+}
+
+static uint32_t lanes_per_row(int dtype, uint32_t n, int nt, const RegVariant &v) {
+  const int ts = dtype == GBDPCG_F64 ? 8 : 4;
+  return v.any ? (uint32_t)any_lpr(v.any, ts) : reg_lpr(n, nt, ts);
+}
+
 // LDS of one workgroup: ghost-extended vectors (5, paired: 8), the per-wave
 // partials (3 per wave, paired: 6), the totals and the control words.
 size_t reg_lds_bytes(int dtype, uint32_t n, uint32_t K, int nt, RegVariant v) {
   const size_t ts = dtype == GBDPCG_F64 ? 8 : 4;
-  const uint32_t lpr = reg_lpr(n, nt, (int)ts);
+  const uint32_t lpr = lanes_per_row(dtype, n, nt, v);
   // paired instances that keep their S chunks in LDS: pair_s_slots chunks ahead
   // of the vectors, whose read-ahead is then 8 values
   const bool slds = v.pair && pair_s_lds(ts, nt, v.bc, (int)n);
@@ -68,12 +87,14 @@ size_t reg_lds_bytes(int dtype, uint32_t n, uint32_t K, int nt, RegVariant v) {
   return (5 * VL + 3 * (size_t)(nt / 64) + 4 + 4) * ts;
 }
 
-// Largest knots per workgroup the lane layout allows: reg_lpr(n) lanes per row
-// of the owned knots plus one ghost knot each side, and 4n ghost lanes (row
-// broadcast: 16 lanes per knot).
-uint32_t reg_max_knots(int dtype, uint32_t n, int nt, bool bc) {
-  if (bc) return n <= 16 && (uint32_t)nt >= 4 * n ? (uint32_t)nt / 16 - 2 : 0;
-  const uint32_t rows = (uint32_t)nt / reg_lpr(n, nt, dtype == GBDPCG_F64 ? 8 : 4);
+// Largest knots per workgroup the lane layout allows: lanes_per_row lanes per
+// row of the owned knots plus one ghost knot each side, and 4n ghost lanes (row
+// broadcast: 16 lanes per knot).  A system's only workgroup (alone) has no ghost
+// rows; the row-broadcast and paired items keep theirs.
+uint32_t reg_max_knots(int dtype, uint32_t n, int nt, RegVariant v, bool alone) {
+  if (v.bc) return n <= 16 && (uint32_t)nt >= 4 * n ? (uint32_t)nt / 16 - 2 : 0;
+  const uint32_t rows = (uint32_t)nt / lanes_per_row(dtype, n, nt, v);
+  if (alone && !v.pair) return rows / n;
   if (rows < 4 * n) return 0;
   return rows / n - 2;
 }
