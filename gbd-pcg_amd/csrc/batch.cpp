@@ -165,8 +165,12 @@ int plan_launch(int dtype, const gbdpcg_system_desc *systems, const std::vector<
   for (uint32_t i : idx) {
     const gbdpcg_system_desc &d = systems[i];
     if (L.reg) {
-      const uint32_t kmax = reg_max_knots(dtype, d.n, L.nt, rv);
-      const uint32_t alone = reg_max_knots(dtype, d.n, L.nt, rv, true);
+      uint32_t kmax = reg_max_knots(dtype, d.n, L.nt, rv);
+      uint32_t alone = reg_max_knots(dtype, d.n, L.nt, rv, true);
+      if (L.any) {  // fewer knots each where the budget asks for it
+        while (kmax > 2 && reg_lds_bytes(dtype, d.n, kmax, L.nt, rv) > (budget & ~(size_t)255)) --kmax;
+        while (alone > 1 && reg_lds_bytes(dtype, d.n, alone, L.nt, rv) > (budget & ~(size_t)255)) --alone;
+      }
       const uint32_t target = kcap ? std::min(kmax, std::max<uint32_t>(kcap, 2u)) : kmax;
       uint32_t g = d.wgs;
       if (!g && d.N <= alone && (!kcap || d.N <= std::max<uint32_t>(kcap, 2u))) g = 1;  // no exchange
@@ -399,8 +403,8 @@ int gbdpcg_batch_create(gbdpcg_batch **out, int dtype, const gbdpcg_system_desc 
     bool has_wide = false;
     for (uint32_t i : small)
       if (systems[i].n > 14) has_wide = true;
-    // runtime-n instances: 0 = every specialised size, -1 = sizes up to 14
-    L.kn = one_n ? (int)systems[small[0]].n : has_wide ? 0 : -1;
+    // runtime-n instance: sizes up to 14 (larger ones: the instances for any size, below)
+    L.kn = one_n ? (int)systems[small[0]].n : -1;
     // FP64 whole rows (row broadcast) and FP64 rows of n = 28: 256 threads, but
     // for a launch of forward + adjoint systems of n = 28 only, 512 (S in LDS)
     const bool pair_only = all_paired(systems, small);
@@ -414,6 +418,21 @@ int gbdpcg_batch_create(gbdpcg_batch **out, int dtype, const gbdpcg_system_desc 
     for (uint32_t i : small)
       if ((systems[i].flags & GBDPCG_SYS_FORWARD) && (systems[i].flags & GBDPCG_SYS_ADJOINT)) L.pair = true;
     if (has_wide && !(one_n && pair28(dtype, L.nt, pair_only))) L.pair = false;
+    if (!one_n && !L.pair && dtype == GBDPCG_F32) {
+      // Mixed sizes in FP32: one lane per row (kAnyAll).  Twice the knots of two
+      // lanes per row share a workgroup, so a system has half the ranks to
+      // exchange with (or none): 512 systems of n in {6, 12, 14, 28}, N 16..256:
+      // 1,043 us against 1,415 us with two lanes for n <= 14; 60 of n <= 14,
+      // N 8..60: 105 against 111.  A budget too small for two lanes is refused.
+      L.any = kAnyAll;
+      for (uint32_t i : small) {
+        const uint32_t K = reg_max_knots(dtype, systems[i].n, L.nt), g = (systems[i].N + K - 1) / K;
+        if (reg_lds_bytes(dtype, systems[i].n, (systems[i].N + g - 1) / g, L.nt) > (budget & ~(size_t)255)) {
+          set_error("the register kernel's layout does not fit the LDS budget of %zu B", budget);
+          return GBDPCG_ERR_TOO_LARGE;
+        }
+      }
+    }
     launches.push_back(L);
     members.push_back(small);
   }
@@ -440,31 +459,55 @@ int gbdpcg_batch_create(gbdpcg_batch **out, int dtype, const gbdpcg_system_desc 
   std::vector<uint8_t> fused(count, 0);
   for (size_t li = 0; li < launches.size(); ++li) {
     const size_t at = items.size();
-    const int rc = plan_launch(dtype, systems, members[li], cfg, prop, budget, launches[li], G, fused, items);
+    const std::vector<uint32_t> &mem = members[li];
+    const int rc = plan_launch(dtype, systems, mem, cfg, prop, budget, launches[li], G, fused, items);
     if (rc < 0) return rc;
-    if (launches[li].reg || cfg->kernel != GBDPCG_KERNEL_AUTO) continue;
-    // What the LDS-resident kernel takes (its plan decides what is refused and
-    // which recurrence a system runs) goes to the register kernel for any
-    // stateSize when that holds every system of the launch with the recurrence
-    // asked for: rows in registers, several times the LDS kernel's rate.
-    BatchLaunch R;
-    R.reg = true;
-    R.fused = fused_cfg;
+    if (cfg->kernel != GBDPCG_KERNEL_AUTO || launches[li].pair) continue;
     bool fits = true, narrow = true;
-    for (uint32_t i : members[li]) {
+    for (uint32_t i : mem) {
       fits = fits && systems[i].n <= 32 && (fused[i] != 0) == fused_cfg;
       narrow = narrow && systems[i].n <= 16;
     }
-    R.any = narrow ? kAnyNarrow : kAnyAll;
-    R.nt = narrow && want256 ? 256 : 512;
+    // Plans the launch as R instead; keep(R) decides whether that replaces it.
+    auto instead = [&](int any, int nt, auto keep) {
+      BatchLaunch R;
+      R.reg = true;
+      R.fused = fused_cfg;
+      R.any = any;
+      R.nt = nt;
+      std::vector<uint32_t> rG = G, ritems(items.begin(), items.begin() + at);
+      std::vector<uint8_t> rfused = fused;
+      if (plan_launch(dtype, systems, mem, cfg, prop, budget, R, rG, rfused, ritems) != GBDPCG_OK || !keep(R)) return;
+      launches[li] = R;
+      G.swap(rG);
+      fused.swap(rfused);
+      items.swap(ritems);
+    };
     if (!fits) continue;
-    std::vector<uint32_t> rG = G, ritems(items.begin(), items.begin() + at);
-    std::vector<uint8_t> rfused = fused;
-    if (plan_launch(dtype, systems, members[li], cfg, prop, budget, R, rG, rfused, ritems) != GBDPCG_OK) continue;
-    launches[li] = R;
-    G.swap(rG);
-    fused.swap(rfused);
-    items.swap(ritems);
+    // What the LDS-resident kernel takes (its plan decides what is refused and
+    // which recurrence a system runs) goes to the register kernel for any
+    // stateSize when that holds every system of the launch with the recurrence
+    // asked for: rows in registers, several times the LDS kernel's rate.  FP32
+    // on one lane per row, FP64 of n <= 16 on two (40 systems of n 3 and 13, N 5..40,
+    // 278 against 297 us with the instance that also holds larger sizes).
+    if (!launches[li].reg)
+      instead(narrow && dtype == GBDPCG_F64 ? kAnyNarrow : kAnyAll, 512, [](const BatchLaunch &) { return true; });
+    if (!launches[li].reg || !narrow) continue;
+    // Systems of one workgroup each have no exchange: worth a change of layout
+    // (100 systems of n = 12, N 10..40, FP32: 69 against 99 us on several).
+    const uint32_t n_sys = (uint32_t)mem.size();
+    if (launches[li].rounds == 1 && launches[li].items > n_sys && dtype == GBDPCG_F32 && !launches[li].any &&
+        cfg->threads == 0)
+      instead(kAnyAll, 512, [&](const BatchLaunch &R) { return R.items == n_sys && R.rounds == 1; });
+    // More work than one round: small workgroups of one lane per row, two (FP64)
+    // or three (FP32) to a CU, hold as many knots as the CU's registers and hide
+    // each other's latencies.  384 systems of n in {6, 12, 14}, N 16..256: FP32 433
+    // us against 570 (one 512-thread workgroup per CU) and 624 (two of two lanes
+    // per row), FP64 1,659 against 2,446; reference form 581 / 782 and 2,272 /
+    // 3,821.  With one round the fewer, larger workgroups win (60 systems: 105
+    // against 113, FP64 218 against 292).
+    if (launches[li].rounds > 1 && cfg->threads != 512)
+      instead(kAnyRows, 256, [](const BatchLaunch &) { return true; });
   }
 
   // device state

@@ -77,11 +77,12 @@ enum : int {
   kAnyNone = 0,
   kAnyTiny = 1,    // n <= 8, one lane per row, 64 threads: systems of one wave
   kAnyNarrow = 2,  // n <= 16, two lanes per row
-  kAnyWide = 3,    // 16 < n <= 32, two lanes per row
-  kAnyAll = 4,     // n <= 32: batches of mixed sizes
+  kAnyWide = 3,    // 16 < n <= 32, two lanes per row: single solves
+  kAnyAll = 4,     // n <= 32, one (FP32) or two (FP64) lanes per row: batches
+  kAnyRows = 5,    // n <= 16, one lane per row, 256 threads: batches of several rounds
 };
 __host__ __device__ constexpr int any_lpr(int set, int tsize) {
-  return set == kAnyTiny || (set == kAnyAll && tsize == 4) ? 1 : 2;
+  return set == kAnyTiny || set == kAnyRows || (set == kAnyAll && tsize == 4) ? 1 : 2;
 }
 
 // Words (64-bit) of one exchange record: kRecScalars scalar slots (3 per wave of

@@ -14,7 +14,14 @@ const void *ap() {
 
 const void *any_ref_kernel_ptr_f32(int nt, int set) {
   if (nt == 64) return set == kAnyTiny ? ap<64, kAnyTiny>() : nullptr;
-  if (nt == 256) return set == kAnyNarrow ? ap<256, kAnyNarrow>() : set == kAnyWide ? ap<256, kAnyWide>() : nullptr;
+  if (nt == 256) {
+    switch (set) {
+      case kAnyNarrow: return ap<256, kAnyNarrow>();
+      case kAnyWide: return ap<256, kAnyWide>();
+      case kAnyRows: return ap<256, kAnyRows>();
+      default: return nullptr;
+    }
+  }
   if (nt != 512) return nullptr;
   switch (set) {
     case kAnyNarrow: return ap<512, kAnyNarrow>();

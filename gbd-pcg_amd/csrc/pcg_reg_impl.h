@@ -1781,10 +1781,8 @@ __device__ __forceinline__ void reg_item_pair(const KSys &d, uint32_t rank, T *l
 
 }  // namespace
 
-// NS > 0: the kernel is specialised for stateSize NS.  Runtime dispatch for
-// batches of uneven stateSize: NS == 0 over every specialised size, NS == -1
-// over those up to 14 (plans that give rows of n = 28 a launch of their own;
-// the instance then needs the registers of n <= 14 only).
+// NS > 0: the kernel is specialised for stateSize NS.  NS == -1: runtime dispatch
+// over the specialised sizes up to 14 (FP64 batches that mix them).
 template <typename T, int NS, int NT, bool FUSED, bool BC>
 __device__ __forceinline__ void reg_dispatch(const KSys &d, uint32_t rank, T *lds) {
   if constexpr (NS > 0) {
@@ -1801,9 +1799,6 @@ __device__ __forceinline__ void reg_dispatch(const KSys &d, uint32_t rank, T *ld
       case 6: reg_item<T, 6, NT, FUSED, false, true, false>(d, rank, lds); break;
       case 12: reg_item<T, 12, NT, FUSED, false, true, false>(d, rank, lds); break;
       case 14: reg_item<T, 14, NT, FUSED, false, true, false>(d, rank, lds); break;
-      case 28:
-        if constexpr (NS == 0) reg_item<T, 28, NT, FUSED, false, true, false>(d, rank, lds);
-        break;
       default: break;  // the planner only admits the sizes above
     }
   }
@@ -1943,7 +1938,7 @@ pcg_pair_kernel(KSys one, const KSys *__restrict__ systems,
 template <typename T, int NT, bool FUSED, int SET>
 __device__ __forceinline__ void any_dispatch(const KSys &d, uint32_t rank, T *lds) {
   constexpr int LP = any_lpr(SET, (int)sizeof(T));
-  constexpr bool kLow = SET != kAnyWide, kMid = SET == kAnyNarrow || SET == kAnyAll,
+  constexpr bool kLow = SET != kAnyWide, kMid = SET == kAnyNarrow || SET == kAnyAll || SET == kAnyRows,
                  kHigh = SET == kAnyWide || SET == kAnyAll;
   switch (padded_n(d.n)) {
     case 4: if constexpr (kLow) reg_item<T, 4, NT, FUSED, false, true, true, LP>(d, rank, lds); break;
@@ -1958,10 +1953,12 @@ __device__ __forceinline__ void any_dispatch(const KSys &d, uint32_t rank, T *ld
   }
 }
 
-// Waves per SIMD as for the fixed sizes: FP32 rows of n <= 16 at 512 threads
-// leave room for a second workgroup on the CU.
+// Waves per SIMD: FP32 rows of n <= 16 on two lanes at 512 threads leave room for
+// a second workgroup on the CU, as the fixed sizes do; the instances of one lane
+// per row are held to three (FP32) or two (FP64) 256-thread workgroups per CU.
 template <typename T, int NT, int SET>
 constexpr int any_waves_per_eu() {
+  if (SET == kAnyRows) return sizeof(T) == 4 ? 3 : 2;
   return (sizeof(T) == 4 && NT == 512 && SET == kAnyNarrow) ? 4 : 1;
 }
 

@@ -24,11 +24,8 @@ const void *reg_ptr_n(int n) {
     case 12: return reg_ptr<T, 12, NT>();
     case 14: return reg_ptr<T, 14, NT>();
     case 28: return reg_ptr<T, 28, NT>();
-    case 0:  // mixed sizes (batches), every specialised size: 512 threads only
-      if constexpr (NT == 512) return reg_ptr<T, 0, NT>();
-      return nullptr;
-    case -1:  // mixed sizes up to 14 (batches whose n = 28 rows run apart): 512 only
-      if constexpr (NT == 512) return reg_ptr<T, -1, NT>();
+    case -1:  // mixed sizes up to 14 (FP64 batches): 512 threads only
+      if constexpr (NT == 512 && sizeof(T) == 8) return reg_ptr<T, -1, NT>();
       return nullptr;
     default: return nullptr;
   }
@@ -60,6 +57,7 @@ bool any_supported(uint32_t n, int nt, int set) {
   switch (set) {
     case kAnyTiny: return n <= 8 && nt == 64;
     case kAnyNarrow: return n <= 16 && (nt == 256 || nt == 512);
+    case kAnyRows: return n <= 16 && nt == 256;
     case kAnyWide: return n > 16 && n <= 32 && (nt == 256 || nt == 512);
     case kAnyAll: return n <= 32 && nt == 512;
     default: return false;

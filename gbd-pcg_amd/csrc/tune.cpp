@@ -249,9 +249,11 @@ extern "C" int gbdpcg_batch_autotune(gbdpcg_batch **out, int dtype, const gbdpcg
   uint32_t maxN = 0;
   for (uint32_t i = 0; i < count; ++i) maxN = std::max(maxN, systems[i].N);
   const uint32_t caps[] = {0, 2, 3, 4, 6, 8, 12, 16, 24, 32, 48, 64};
-  // what the untuned plan would use
-  const uint32_t def_nt = (cfg->threads == 256 || (cfg->threads == 0 && cfg->block[0] == 256)) ? 256u : 512u;
-  const std::vector<uint32_t> nts = {def_nt, def_nt == 512 ? 256u : 512u};
+  // the threads asked for first (0: the untuned plan's own choice), then 512 and 256
+  const uint32_t def_nt = (cfg->threads == 0 && cfg->block[0] == 256) ? 256u : cfg->threads;
+  std::vector<uint32_t> nts = {def_nt};
+  for (uint32_t nt : {512u, 256u})
+    if (nt != def_nt) nts.push_back(nt);
 
   LambdaSnapshot snap;
   int rc = snap.save(dtype, systems, count, st);
@@ -268,7 +270,7 @@ extern "C" int gbdpcg_batch_autotune(gbdpcg_batch **out, int dtype, const gbdpcg
 
   gbdpcg_batch *best = nullptr;
   double best_us = 1e300, default_us = -1.0;
-  uint32_t best_cap = 0, best_nt = 512, best_kernel = cfg->kernel, best_split = cfg->batch_split;
+  uint32_t best_cap = 0, best_nt = def_nt, best_kernel = cfg->kernel, best_split = cfg->batch_split;
   std::vector<std::vector<uint32_t>> seen;  // per-system workgroup vectors already timed
   std::vector<int> seen_nt, seen_k, seen_l;  // ... and the threads per workgroup, kernel and launches they ran with
   for (uint32_t kid : kernels)

@@ -58,3 +58,19 @@ def test_batches_of_any_size(gpu, dtype, recurrence, top):
     b = gbdpcg.Batch(systems, exit_mode=gbdpcg.EXIT_REL_RESID, recurrence=recurrence)
     b.run()
     check(systems, host, b.results(), dtype, recurrence, adjoint=True)
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("recurrence", [0, 1])
+def test_batches_of_several_rounds(gpu, dtype, recurrence):
+    """More systems than CUs: plans on small workgroups of one lane
+    per row, horizons on both sides of what one of those holds (256 // n knots)."""
+    import gbdpcg
+    tol = 1e-5 if dtype == np.float32 else 1e-9
+    sizes = [n for n in SIZES if n <= 16 and n > 3]
+    specs = [(n, 256 // n + d, tol) for _ in range(8) for n in sizes for d in (-2, -1, 0, 1, 2)]
+    systems, host = make_batch(specs, dtype, seed0=15000)
+    b = gbdpcg.Batch(systems, exit_mode=gbdpcg.EXIT_REL_RESID, recurrence=recurrence)
+    assert b.info()["wgs_per_cu"] == (3 if dtype == np.float32 else 2)
+    b.run()
+    check(systems, host, b.results(), dtype, recurrence)
