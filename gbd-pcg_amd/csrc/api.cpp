@@ -135,6 +135,7 @@ struct Layout {
   int any = kAnyNone;  // ... for any stateSize (which instance)
   bool fused = true;   // its recurrence (the LDS kernel takes it from the flags)
   int nt = 256;        // threads per workgroup
+  int block = 0;       // ... of which launched (0: all)
   RegVariant variant() const { return RegVariant{fused, bc, pair, any}; }
 };
 
@@ -300,8 +301,10 @@ static int plan_single(int dtype, uint32_t n, uint32_t N, bool fused, uint32_t w
   return GBDPCG_OK;
 }
 
-// The instance for any stateSize that takes n at nt threads.
-static int any_set(uint32_t n, int nt) { return nt == 64 ? kAnyTiny : n <= 16 ? kAnyNarrow : kAnyWide; }
+// The instance for any stateSize that runs single solves of n at nt threads.
+static int any_set(uint32_t n, int nt) {
+  return nt == 64 ? kAnyTiny : nt == 512 ? kAnyAll : n <= 16 ? kAnyNarrow : kAnyWide;
+}
 
 // Checks that a register layout of G workgroups (c: kernel, threads, G, stride 0 =
 // one XCD when they fit there) can run co-resident and completes it.
@@ -319,6 +322,12 @@ static int finish_reg_layout(int dtype, uint32_t n, uint32_t N, Layout *c) {
   const uint32_t per_xcd = (uint32_t)(di.cus / kXcds) * (uint32_t)occ;
   if (occ <= 0 || c->G > (uint32_t)di.cus * (uint32_t)occ || (c->stride == (uint32_t)kXcds && c->G > per_xcd))
     return GBDPCG_ERR_UNSUPPORTED;
+  // a lone workgroup needs the waves of its rows only: at n = 20, N = 12 FP32 four
+  // of eight
+  if (c->G == 1 && c->any && any_alone(c->any)) {
+    const uint32_t lanes = n * N * (uint32_t)any_lpr(c->any, (int)tsize(dtype));
+    c->block = (int)std::min<uint32_t>((uint32_t)c->nt, ceil_div(lanes, 64) * 64);
+  }
   if (!c->stride) c->stride = c->G <= per_xcd ? (uint32_t)kXcds : 1u;
   c->grid = c->G * c->stride;
   return GBDPCG_OK;
@@ -379,25 +388,25 @@ static int plan_single_reg(int dtype, uint32_t n, uint32_t N, uint32_t want_G, u
 // One workgroup for the whole system, the smallest that holds it: no exchange at
 // all, which is more than the smaller matvecs of several workgroups save at every
 // size that fits (microseconds per iteration, one workgroup against the best of
-// several, FP32: n = 14 N = 16 fused 0.96 / 1.36 and reference form 1.33 / 2.28,
-// n = 32 N = 8 1.28 / 1.90 and 1.60 / 2.69, n = 2 N = 30 on one wave 0.42 / 1.13
-// and 0.67 / 1.99; FP64 n = 28 N = 9 2.50 / 3.40 and 2.84 / 4.48).
+// several, fused and reference form; FP32: n = 14 N = 36 1.05 / 1.47 and 1.27 /
+// 2.35, n = 12 N = 42 0.89 / 1.34 and 1.14 / 2.20, n = 32 N = 16 1.51 / 1.89 and
+// 1.75 / 2.67, n = 2 N = 30 on one wave 0.19 / 1.13 and 0.23 / 1.99; FP64: n = 6
+// N = 40 0.90 / 1.75 and 1.21 / 2.92, n = 32 N = 8 2.07 / 3.91 reference form).
 // GBDPCG_ERR_UNSUPPORTED when no workgroup holds it.
 static int plan_one_workgroup(int dtype, uint32_t n, uint32_t N, bool fused, bool pair, Layout *L) {
   if (n > 32 || (fused && N < 2)) return GBDPCG_ERR_UNSUPPORTED;
+  const bool both = pair && fused && n <= 14 && reg_supported((int)n) && N >= 4;
   for (int nt : {64, 256, 512}) {
-    const bool fixed = reg_supported((int)n) && N >= 4 && nt != 64 && (fused || nt == 256) &&
-                       !(dtype == GBDPCG_F64 && n > 14 && nt > 256);
     Layout c;
-    // FP64 rows of n = 12 and 14 broadcast by DPP: 1.13 us per fused iteration at
-    // N = 14 where two lanes per row at 512 threads take 1.56 (reference form
-    // 1.41 against 2.13)
-    c.bc = fixed && nt == 256 && dtype == GBDPCG_F64 && reg_supported((int)n, true);
-    c.pair = pair && fused && n <= 14 && fixed;
-    c.any = fixed ? kAnyNone : any_set(n, nt);
+    c.pair = both;
+    // FP64 rows of n = 12 and 14 broadcast by DPP up to N = 14: 1.14 us per fused
+    // iteration at N = 14, 1.31 on kAnyRows (reference form 1.46, 1.53)
+    c.bc = nt == 256 && dtype == GBDPCG_F64 && N >= 4 && reg_supported((int)n, true) &&
+           N <= reg_max_knots(dtype, n, nt, RegVariant{fused, true});
+    c.any = both || c.bc ? kAnyNone : nt == 256 ? kAnyRows : any_set(n, nt);
     c.fused = fused;
     c.nt = nt;
-    if (c.any && !any_supported(n, nt, c.any)) continue;
+    if (c.any ? !any_supported(n, nt, c.any) : nt == 64) continue;
     if (N > reg_max_knots(dtype, n, nt, c.variant(), true)) continue;
     c.G = 1;
     c.stride = 0;
@@ -418,9 +427,9 @@ static std::string single_key(int dev, int dtype, uint32_t n, uint32_t N, bool f
 }
 
 // Kinds of layout, as the tuner's choices name them (TuneChoice.a).
-enum : uint32_t { kKindLds = 0, kKindReg = 1, kKindRowcast = 2, kKindAny = 3 };
+enum : uint32_t { kKindLds = 0, kKindReg = 1, kKindRowcast = 2, kKindAny = 3, kKindRows = 4 };
 static uint32_t kind_of(const Layout &L) {
-  return !L.reg ? kKindLds : L.bc ? kKindRowcast : L.any ? kKindAny : kKindReg;
+  return !L.reg ? kKindLds : L.bc ? kKindRowcast : L.any == kAnyRows ? kKindRows : L.any ? kKindAny : kKindReg;
 }
 
 // Rebuilds a layout from its (kind, threads, workgroups, stride); checks that it
@@ -430,14 +439,14 @@ static int layout_from(int dtype, uint32_t n, uint32_t N, uint32_t kind, int nt,
   DeviceInfo di;
   int rc = device_info(cur_dev(), &di);
   if (rc < 0) return rc;
-  if (kind > kKindAny || G == 0 || G > N || (stride != 1 && stride != (uint32_t)kXcds)) return GBDPCG_ERR_UNSUPPORTED;
+  if (kind > kKindRows || G == 0 || G > N || (stride != 1 && stride != (uint32_t)kXcds)) return GBDPCG_ERR_UNSUPPORTED;
   Layout t;
   t.G = G;
   t.stride = stride;
   t.grid = G * stride;
   t.reg = kind != kKindLds;
   t.bc = kind == kKindRowcast;
-  t.any = kind == kKindAny ? any_set(n, nt) : kAnyNone;
+  t.any = kind == kKindRows ? kAnyRows : kind == kKindAny ? any_set(n, nt) : kAnyNone;
   t.pair = t.reg && !t.any && fused && pair && n <= 14;
   t.fused = fused;
   t.nt = t.reg ? nt : kThreads;
@@ -691,7 +700,7 @@ static int solve_locked(Workspace *ws, int dtype, uint32_t n, uint32_t N, const 
               exchange_flags(cfg);
   if (L.reg) {
     HIPCHK(reg_launch(dtype, (int)n, L.nt, one, nullptr, nullptr, 0, L.stride, L.grid, L.lds, stream,
-                      L.variant()));
+                      L.variant(), L.block));
   } else {
     HIPCHK(pcg_launch(dtype, one, nullptr, nullptr, 0, L.stride, L.grid, L.lds, stream));
   }
@@ -838,7 +847,7 @@ int solve_on_scratch(int dtype, uint32_t n, uint32_t N, const void *S, const voi
               exchange_flags(cfg);
   if (L.reg) {
     HIPCHK(reg_launch(dtype, (int)n, L.nt, one, nullptr, nullptr, 0, L.stride, L.grid, L.lds, stream,
-                      L.variant()));
+                      L.variant(), L.block));
   } else {
     HIPCHK(pcg_launch(dtype, one, nullptr, nullptr, 0, L.stride, L.grid, L.lds, stream));
   }
@@ -1163,7 +1172,9 @@ int gbdpcg_tune_single(int dtype, uint32_t n, uint32_t N, const void *d_S, const
   }
 
   const uint32_t Ks[] = {1, 2, 3, 4, 5, 6, 7, 8, 10, 12, 14, 16, 20, 24, 28, 32, 40, 48, 64};
-  for (const uint32_t kind : {(uint32_t)kKindRowcast, (uint32_t)kKindReg, (uint32_t)kKindAny, (uint32_t)kKindLds}) {
+  for (const uint32_t kind : {(uint32_t)kKindRowcast, (uint32_t)kKindReg, (uint32_t)kKindAny, (uint32_t)kKindRows,
+                              (uint32_t)kKindLds}) {
+    const bool any = kind == kKindAny || kind == kKindRows;
     const uint32_t kid = kind == kKindRowcast ? GBDPCG_KERNEL_ROWCAST
                          : kind == kKindLds   ? GBDPCG_KERNEL_LDS
                                               : GBDPCG_KERNEL_REGISTER;
@@ -1171,14 +1182,14 @@ int gbdpcg_tune_single(int dtype, uint32_t n, uint32_t N, const void *d_S, const
     if (kind == kKindLds && cfg->threads) continue;  // a thread request names a register kernel
     // the instances for any size: automatic solves of the sizes without instances
     // of their own, and systems of one workgroup
-    if (kind == kKindAny && (cfg->kernel != GBDPCG_KERNEL_AUTO || unfit)) continue;
+    if (any && (cfg->kernel != GBDPCG_KERNEL_AUTO || unfit)) continue;
     for (int nt : {256, 512, 64}) {
       if (kind == kKindLds && nt != kThreads) continue;
       if (nt == 64 && kind != kKindRowcast && kind != kKindAny) continue;  // one-wave workgroups
       for (uint32_t K : Ks) {
         const uint32_t G = ceil_div(N, K);
         if (G > (uint32_t)kMaxWgsPerSystem || (fused && N / G < 2)) continue;
-        if (kind == kKindAny && G > 1 && reg_supported((int)n) && N >= 4) continue;
+        if (any && G > 1 && reg_supported((int)n) && N >= 4) continue;
         for (uint32_t stride : {(uint32_t)kXcds, 1u}) {
           Layout L;
           if (layout_from(dtype, n, N, kind, nt, G, stride, &L, fused) == GBDPCG_OK) add(L);
@@ -1252,7 +1263,7 @@ int gbdpcg_tune_single(int dtype, uint32_t n, uint32_t N, const void *d_S, const
       if ((e = hipMemsetAsync(lam, 0, (size_t)n * N * ts, st)) != hipSuccess) return fail("hipMemsetAsync", e);
       if ((e = hipEventRecord(ea, st)) != hipSuccess) return fail("hipEventRecord", e);
       e = L.reg ? reg_launch(dtype, (int)n, L.nt, one, nullptr, nullptr, 0, L.stride, L.grid, L.lds, st,
-                             L.variant())
+                             L.variant(), L.block)
                 : pcg_launch(dtype, one, nullptr, nullptr, 0, L.stride, L.grid, L.lds, st);
       if (e != hipSuccess) return fail("solve launch", e);
       if ((e = hipEventRecord(eb, st)) != hipSuccess) return fail("hipEventRecord", e);

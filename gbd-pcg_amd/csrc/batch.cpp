@@ -487,11 +487,8 @@ int gbdpcg_batch_create(gbdpcg_batch **out, int dtype, const gbdpcg_system_desc 
     // What the LDS-resident kernel takes (its plan decides what is refused and
     // which recurrence a system runs) goes to the register kernel for any
     // stateSize when that holds every system of the launch with the recurrence
-    // asked for: rows in registers, several times the LDS kernel's rate.  FP32
-    // on one lane per row, FP64 of n <= 16 on two (40 systems of n 3 and 13, N 5..40,
-    // 278 against 297 us with the instance that also holds larger sizes).
-    if (!launches[li].reg)
-      instead(narrow && dtype == GBDPCG_F64 ? kAnyNarrow : kAnyAll, 512, [](const BatchLaunch &) { return true; });
+    // asked for: rows in registers, several times the LDS kernel's rate.
+    if (!launches[li].reg) instead(kAnyAll, 512, [](const BatchLaunch &) { return true; });
     if (!launches[li].reg || !narrow) continue;
     // Systems of one workgroup each have no exchange: worth a change of layout
     // (100 systems of n = 12, N 10..40, FP32: 69 against 99 us on several).

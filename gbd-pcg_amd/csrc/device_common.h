@@ -183,6 +183,17 @@ __device__ __forceinline__ double read_lane63(double v) {
   return __longlong_as_double((long long)(((uint64_t)hi << 32) | lo));
 }
 
+// Value of lane l (a constant), uniform.
+__device__ __forceinline__ float read_lane(float v, int l) {
+  return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), l));
+}
+__device__ __forceinline__ double read_lane(double v, int l) {
+  const uint64_t b = (uint64_t)__double_as_longlong(v);
+  const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)b, l);
+  const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(b >> 32), l);
+  return __longlong_as_double((long long)(((uint64_t)hi << 32) | lo));
+}
+
 // Sum over the 64 lanes of a wave (all lanes active): inclusive scan inside each
 // row of 16 lanes, then the row totals are folded into lane 63, which is
 // broadcast.  A fixed tree: identical inputs give identical bits in every wave.

@@ -76,14 +76,17 @@ __host__ __device__ constexpr uint32_t reg_chunk(uint32_t n, uint32_t lpr) {
 enum : int {
   kAnyNone = 0,
   kAnyTiny = 1,    // n <= 8, one lane per row, 64 threads: systems of one wave
-  kAnyNarrow = 2,  // n <= 16, two lanes per row
-  kAnyWide = 3,    // 16 < n <= 32, two lanes per row: single solves
-  kAnyAll = 4,     // n <= 32, one (FP32) or two (FP64) lanes per row: batches
-  kAnyRows = 5,    // n <= 16, one lane per row, 256 threads: batches of several rounds
+  kAnyNarrow = 2,  // n <= 16, two lanes per row, 256 threads: single solves
+  kAnyWide = 3,    // 16 < n <= 32, two lanes per row, 256 threads: single solves
+  kAnyAll = 4,     // n <= 32, one (FP32) or two (FP64) lanes per row, 512 threads
+  kAnyRows = 5,    // n <= 16, one lane per row, 256 threads
 };
 __host__ __device__ constexpr int any_lpr(int set, int tsize) {
-  return set == kAnyTiny || set == kAnyRows || (set == kAnyAll && tsize == 4) ? 1 : 2;
+  return set == kAnyNarrow || set == kAnyWide || (set == kAnyAll && tsize == 8) ? 2 : 1;
 }
+// Whether an instance runs systems of one workgroup without exchange code, ghost
+// rows or their lanes (kAnyTiny runs nothing else).
+__host__ __device__ constexpr bool any_alone(int set) { return set != kAnyNarrow && set != kAnyWide; }
 
 // Words (64-bit) of one exchange record: kRecScalars scalar slots (3 per wave of
 // the publishing workgroup, up to 8 waves) + two edge blocks, each a left edge
@@ -185,7 +188,7 @@ hipError_t reg_prepare(int dtype, int n, int nt, size_t lds, RegVariant v = {});
 hipError_t reg_occupancy(int dtype, int n, int nt, size_t lds, int *wgs_per_cu, RegVariant v = {});
 hipError_t reg_launch(int dtype, int n, int nt, const KSys &one, const KSys *systems, const uint32_t *items,
                       uint32_t rounds, uint32_t stride, uint32_t grid, size_t lds, hipStream_t stream,
-                      RegVariant v = {});
+                      RegVariant v = {}, int block = 0);
 const void *rowcast_kernel_ptr(int dtype, int n, int nt, bool fused);
 const void *pair_kernel_ptr_f32(int n, int nt, bool bc);
 const void *pair_kernel_ptr_f64(int n, int nt, bool bc);

@@ -1,6 +1,5 @@
 // Register-resident PCG kernels for any stateSize up to 32, double reference-recurrence
-// instances (the kernel is in pcg_reg_impl.h): 64 threads (systems of one wave),
-// 256 and 512 (single solves and batches).
+// instances (the kernel is in pcg_reg_impl.h).
 #include "pcg_reg_impl.h"
 
 namespace gbdpcg {
@@ -14,19 +13,12 @@ const void *ap() {
 
 const void *any_ref_kernel_ptr_f64(int nt, int set) {
   if (nt == 64) return set == kAnyTiny ? ap<64, kAnyTiny>() : nullptr;
-  if (nt == 256) {
-    switch (set) {
-      case kAnyNarrow: return ap<256, kAnyNarrow>();
-      case kAnyWide: return ap<256, kAnyWide>();
-      case kAnyRows: return ap<256, kAnyRows>();
-      default: return nullptr;
-    }
-  }
-  if (nt != 512) return nullptr;
+  if (nt == 512) return set == kAnyAll ? ap<512, kAnyAll>() : nullptr;
+  if (nt != 256) return nullptr;
   switch (set) {
-    case kAnyNarrow: return ap<512, kAnyNarrow>();
-    case kAnyWide: return ap<512, kAnyWide>();
-    case kAnyAll: return ap<512, kAnyAll>();
+    case kAnyNarrow: return ap<256, kAnyNarrow>();
+    case kAnyWide: return ap<256, kAnyWide>();
+    case kAnyRows: return ap<256, kAnyRows>();
     default: return nullptr;
   }
 }

@@ -78,7 +78,8 @@ struct StateSize<NS, true> {
 // LP > 0: any stateSize n <= NS with padded_n(n) == NS (a multiple of 4), LP
 // lanes per row.  Vectors and chunks have the compile-time stride NS, so the
 // matvecs are those of a fixed size; lanes, records and HBM offsets follow n.
-template <typename T, int NS, int NT, bool BC = false, int LP = 0>
+// ALONE: the system's only rank, with no ghost rows and no exchange.
+template <typename T, int NS, int NT, bool BC = false, int LP = 0, bool ALONE = false>
 struct RegItem : StateSize<NS, (LP > 0)> {
   static constexpr bool RT = LP > 0;
   using StateSize<NS, RT>::n;
@@ -103,6 +104,7 @@ struct RegItem : StateSize<NS, (LP > 0)> {
   int gpos;
   // LDS
   T *rv, *uv, *wv, *xv, *lv, *wsum, *tot;
+  T only[3];  // ALONE on one wave: its sums
   int *ctl;
 
   __device__ __forceinline__ uint64_t *rec(int type, int g) const {
@@ -148,7 +150,7 @@ struct RegItem : StateSize<NS, (LP > 0)> {
   }
 
   __device__ __forceinline__ void publish_edge(T val, int edge, int voff = 0) const {
-    if (G == 1) return;
+    if (ALONE || G == 1) return;
     const uint32_t epoch = base + seq;
     uint64_t *r = rec((int)(seq & 1u), rank);
     if (xcd)
@@ -163,14 +165,22 @@ struct RegItem : StateSize<NS, (LP > 0)> {
   // second and third scalars are replaced by x and x^2, x = 1 + this XCD's id,
   // so that after the gather every rank can tell (identically) whether all ranks
   // share one XCD: G * sum(x^2) == sum(x)^2 exactly when all x are equal.
-  __device__ __forceinline__ void reduce_publish(T s0, T s1, T s2, bool placement = false) const {
+  // ALONE: the waves' sums only, which only_totals adds up.
+  __device__ __forceinline__ void reduce_publish(T s0, T s1, T s2, bool placement = false) {
     wave_sum3(s0, s1, s2);
+    if constexpr (ALONE && NWAVES == 1) {
+      only[0] = s0;
+      only[1] = s1;
+      only[2] = s2;
+      return;
+    }
     const int w = threadIdx.x >> 6;
     if ((threadIdx.x & 63) == 0) {
       wsum[w * 3 + 0] = s0;
       wsum[w * 3 + 1] = s1;
       wsum[w * 3 + 2] = s2;
     }
+    if constexpr (ALONE) return;
     __syncthreads();
     // lanes 0..2 of wave 0: scalar l summed over the waves in order, published
     const int l = threadIdx.x;
@@ -188,6 +198,29 @@ struct RegItem : StateSize<NS, (LP > 0)> {
     uint64_t *r = rec((int)(seq & 1u), rank);
 #pragma unroll
     for (int qq = 0; qq < WPV; ++qq) xstore_sel(r + l * WPV + qq, payload_word(tv, qq), epoch, xcd);
+  }
+
+  // ALONE: every wave adds up the waves' sums itself, in waves_total's order: one
+  // LDS round trip and one barrier (through wave 0 and tot, a second of each).
+  // Waves that were not launched left theirs zero.
+  // The next reduction writes the same sums: settle() stands between the two
+  // where the solve has no barrier of its own.
+  __device__ __forceinline__ void settle() const {
+    if constexpr (ALONE) __syncthreads();
+  }
+  __device__ __forceinline__ void only_totals(T &t0, T &t1, T &t2) const {
+    __syncthreads();
+    if constexpr (NWAVES == 1) {
+      t0 = only[0];
+      t1 = only[1];
+      t2 = only[2];
+    } else {
+      const int l = (int)threadIdx.x & 3;
+      const T v = waves_total<NWAVES, 3>(wsum, l < 3 ? l : 0);
+      t0 = read_lane(v, 0);
+      t1 = read_lane(v, 1);
+      t2 = read_lane(v, 2);
+    }
   }
 
   static __device__ __forceinline__ T word_value(const uint32_t *w, int v) {
@@ -298,6 +331,10 @@ struct RegItem : StateSize<NS, (LP > 0)> {
   // which t0..t2 hold the totals in every thread; returns false (uniformly) if
   // a wait hit its bound.
   __device__ __forceinline__ bool gather(T *vec, int edge, T &t0, T &t1, T &t2) {
+    if constexpr (ALONE) {
+      only_totals(t0, t1, t2);
+      return true;
+    }
     if (G == 1) {
       __syncthreads();
       t0 = uniform(tot[0]);
@@ -361,8 +398,7 @@ struct RegItem : StateSize<NS, (LP > 0)> {
   // three for B; each scalar reduced exactly as reduce_publish reduces it),
   // wsum holding 6 per wave.  Lanes 0..5 publish.  placement as in
   // reduce_publish, for scalars 1 and 2.
-  __device__ __forceinline__ void reduce_publish6(T s0, T s1, T s2, T s3, T s4, T s5,
-                                                  bool placement = false) const {
+  __device__ __forceinline__ void reduce_publish6(T s0, T s1, T s2, T s3, T s4, T s5, bool placement = false) {
     wave_sum3(s0, s1, s2);
     wave_sum3(s3, s4, s5);
     const int w = threadIdx.x >> 6;
@@ -805,9 +841,10 @@ __device__ __forceinline__ bool finite_t(double v) { return __builtin_isfinite(v
 
 // One matvec row pass: this lane's row of a resident block row times the vector
 // window of knots m-1..m+1 (local knots m..m+2) of `vec`; 0 on inactive lanes.
-template <typename T, int NS, int NT, bool BC, int LP, int CW>
-__device__ __forceinline__ T row_mv(const RegItem<T, NS, NT, BC, LP> &it, const T (&mat)[CW], const T *vec, bool act) {
-  using R = RegItem<T, NS, NT, BC, LP>;
+template <typename T, int NS, int NT, bool BC, int LP, bool ALONE, int CW>
+__device__ __forceinline__ T row_mv(const RegItem<T, NS, NT, BC, LP, ALONE> &it, const T (&mat)[CW], const T *vec,
+                                    bool act) {
+  using R = RegItem<T, NS, NT, BC, LP, ALONE>;
   if constexpr (BC) {
     // every lane of the 16-lane row takes part in the broadcasts; lanes past the
     // window read (and discard) the last knot's entries
@@ -938,19 +975,23 @@ __device__ __forceinline__ void write_gS(T *gS, const T *gg, const T *lam, int a
 // own set-up reads together).
 // BF: the matrix chunks loaded branch-free (load_chunk), for the fixed-size
 // instances; the runtime-n instances keep the guarded loads.
-// LP: lanes per row of the runtime-stateSize items (RegItem), 0 for fixed sizes.
-template <typename T, int NS, int NT, bool FUSED, bool BC = false, bool PRE = true, bool BF = PRE, int LP = 0>
+// LP: lanes per row of the runtime-stateSize items, ALONE: a system's only rank
+// (RegItem).
+template <typename T, int NS, int NT, bool FUSED, bool BC = false, bool PRE = true, bool BF = PRE, int LP = 0,
+          bool ALONE = false>
 __device__ __forceinline__ void reg_item(const KSys &d, uint32_t rank, T *lds) {
-  using R = RegItem<T, NS, NT, BC, LP>;
+  using R = RegItem<T, NS, NT, BC, LP, ALONE>;
   constexpr int nP = R::nP, CW = R::CW;
   R it;
   it.set_n((int)d.n);
   const int n = it.n;
+  // a single solve's only workgroup is launched with the waves its rows need
+  const int stride = ALONE ? (int)blockDim.x : NT;
   it.N = (int)d.N;
-  it.G = (int)d.G;
-  it.rank = (int)rank;
-  it.a = (int)knot_begin(rank, d.G, d.N);
-  it.b = (int)knot_begin(rank + 1, d.G, d.N);
+  it.G = ALONE ? 1 : (int)d.G;
+  it.rank = ALONE ? 0 : (int)rank;
+  it.a = ALONE ? 0 : (int)knot_begin(rank, d.G, d.N);
+  it.b = ALONE ? it.N : (int)knot_begin(rank + 1, d.G, d.N);
   it.K = it.b - it.a;
   const int K = it.K;
   it.VL = (K + 4) * nP + (BC ? 16 : R::LPR * CW);
@@ -968,17 +1009,17 @@ __device__ __forceinline__ void reg_item(const KSys &d, uint32_t rank, T *lds) {
     it.m = t >> 4;
     it.row = t & 15;
   } else {
-    const int kq = it.q / n;
-    it.row = it.q - kq * n;
-    // one rank has no neighbours: no lanes for ghost rows, so it holds two knots more
-    it.m = kq + (it.G == 1 ? 1 : 0);
+    it.m = it.q / n;
+    it.row = it.q - it.m * n;
+    // no neighbours: no lanes for ghost rows, so it holds two knots more
+    if (ALONE || (!R::RT && it.G == 1)) ++it.m;
   }
   it.kg = it.a - 1 + it.m;
   it.act_u = it.m < K + 2 && (!BC || it.row < n);
   it.act_w = it.m >= 1 && it.m <= K && (!BC || it.row < n);
   it.owner = it.act_w && it.c == 0;
-  it.ghost = it.c == R::LPR - 1 && it.q < 4 * n && it.G > 1;
-  it.set_edge_slots();
+  it.ghost = it.c == R::LPR - 1 && it.q < 4 * n && !ALONE && (R::RT || it.G > 1);
+  if (!ALONE) it.set_edge_slots();
   {
     const int gk = it.q / n, gr = it.q - (it.q / n) * n;  // ghost element q: knot slot 0..3
     const int gj = gk < 2 ? gk : K + gk;                  // local knots 0, 1, K+2, K+3
@@ -998,7 +1039,7 @@ __device__ __forceinline__ void reg_item(const KSys &d, uint32_t rank, T *lds) {
   const int m = it.m, row = it.row, c = it.c, kg = it.kg;
   const int own_pos = (m + 1) * nP + row;  // local knot of own row kl = m - 1 is m + 1
 
-  if (t == 0) {
+  if (!ALONE && t == 0) {
     const uint32_t ea = (uint32_t)(xload(it.rec(0, it.rank)) >> 32);
     const uint32_t eb = (uint32_t)(xload(it.rec(1, it.rank)) >> 32);
     uint32_t base = (ea > eb ? ea : eb) + 1u;
@@ -1006,13 +1047,13 @@ __device__ __forceinline__ void reg_item(const KSys &d, uint32_t rank, T *lds) {
     it.ctl[0] = 0;
     it.ctl[1] = (int)base;
   }
-  for (int i = opaque_tid(); i < total; i += NT) lds[i] = (T)0;
+  for (int i = opaque_tid(); i < total; i += stride) lds[i] = (T)0;
 
   const bool fwd = (d.flags & KF_FWD) != 0;
   const bool adj = (d.flags & KF_ADJ) != 0;
   // every HBM read of the set-up in one round trip (PRE): the initial guess
-  // window (own + one ghost knot each side; (K + 2) n <= NT values, one per
-  // thread below NT, the rest after the barrier) and the first right-hand side,
+  // window (own + one ghost knot each side; one per thread, the rest after the
+  // barrier) and the first right-hand side,
   // issued with the matrix chunks
   const T *lam0 = static_cast<const T *>(d.lambda);
   const int wl = (K + 2) * n;
@@ -1052,12 +1093,12 @@ __device__ __forceinline__ void reg_item(const KSys &d, uint32_t rank, T *lds) {
     load_chunk<T, NS, CW, kMode>(mM, static_cast<const T *>(d.Pinv), kg, row, c, it.N, it.act_u, n);
   }
   __syncthreads();
-  it.base = (uint32_t)it.ctl[1];
+  it.base = ALONE ? 0u : (uint32_t)it.ctl[1];
   it.seq = 0;
   {
     T *dst = fwd ? it.xv : it.lv;
     if (lam_pos >= 0) dst[lam_pos] = lam_pre;
-    for (int i = opaque_tid() + (PRE ? NT : 0); i < wl; i += NT) {
+    for (int i = opaque_tid() + (PRE ? stride : 0); i < wl; i += stride) {
       const int jj = i / n, e = i - jj * n;
       const int k = it.a - 1 + jj;
       if (k >= 0 && k < it.N) dst[(jj + 1) * nP + e] = gptr(lam0)[(size_t)k * n + e];
@@ -1073,9 +1114,9 @@ __device__ __forceinline__ void reg_item(const KSys &d, uint32_t rank, T *lds) {
       // adjoint: lambda (own + ghosts) was left in xv by the forward pass, or
       // loaded into lv above; keep it in lv and restart from x = 0
       if (fwd) {
-        for (int i = opaque_tid(); i < it.VL; i += NT) it.lv[i] = it.xv[i];
+        for (int i = opaque_tid(); i < it.VL; i += stride) it.lv[i] = it.xv[i];
       }
-      for (int i = opaque_tid(); i < it.VL; i += NT) it.xv[i] = (T)0;
+      for (int i = opaque_tid(); i < it.VL; i += stride) it.xv[i] = (T)0;
       __syncthreads();
     }
     // with PRE the first pass's right-hand side was read with the set-up
@@ -1104,7 +1145,8 @@ __device__ __forceinline__ void reg_item(const KSys &d, uint32_t rank, T *lds) {
     // the sums are of small integers, exact in T; compare in double
     // (uniform by construction; readfirstlane lets the compiler branch on it in
     // scalar code)
-    it.xcd = __builtin_amdgcn_readfirstlane(
+    if constexpr (!ALONE)
+      it.xcd = __builtin_amdgcn_readfirstlane(
                  (int)(it.xcd_ok && it.G > 1 && (double)sx * (double)sx == (double)it.G * (double)sxx)) != 0;
     // exit threshold: |r'z| < tol (reference) or r'r <= tol^2 rhs'rhs
     const double thr = it.rel ? it.tol * it.tol * (double)gg : it.tol;
@@ -1115,6 +1157,7 @@ __device__ __forceinline__ void reg_item(const KSys &d, uint32_t rank, T *lds) {
       T z_i, p_i, eta, rr;
       {
         z_i = row_mv(it, mM, it.rv, it.act_u);
+        it.settle();
         p_i = z_i;
         if (it.act_u && c == 0) it.uv[(m + 1) * nP + row] = p_i;  // uv holds p
         const T rz = it.owner ? r_i * z_i : (T)0;
@@ -1141,6 +1184,7 @@ __device__ __forceinline__ void reg_item(const KSys &d, uint32_t rank, T *lds) {
           out.iters = 0;
           goto finish;
         }
+        it.settle();
       }
       {
         uint32_t iter = 0;
@@ -1327,6 +1371,7 @@ __device__ __forceinline__ void reg_item(const KSys &d, uint32_t rank, T *lds) {
     }
     if (adj) {
       if (it.owner) it.xv[own_pos] = x_i;
+      it.settle();
       it.publish_edge(x_i, 1);
       it.reduce_publish((T)0, (T)0, (T)0);
       T z0, z1, z2;
@@ -1343,7 +1388,7 @@ __device__ __forceinline__ void reg_item(const KSys &d, uint32_t rank, T *lds) {
       // second workgroup per CU)
       const int bs = 3 * n * n;
       T *gS = static_cast<T *>(d.gS);
-      for (int e = opaque_tid(); e < K * bs; e += NT) {
+      for (int e = opaque_tid(); e < K * bs; e += stride) {
         const int kl = e / bs;
         const int wq = e - kl * bs;
         const int col = wq / n;
@@ -1935,35 +1980,47 @@ pcg_pair_kernel(KSys one, const KSys *__restrict__ systems,
 // reference form, 168 us (1,081).  SET names the classes one kernel
 // holds and with them its registers: the tiny and narrow ones serve systems of
 // n <= 8 and n <= 16, the wide one larger ones, kAnyAll batches of mixed sizes.
-template <typename T, int NT, bool FUSED, int SET>
-__device__ __forceinline__ void any_dispatch(const KSys &d, uint32_t rank, T *lds) {
+template <typename T, int NT, bool FUSED, int SET, bool ALONE>
+__device__ __forceinline__ void any_class(const KSys &d, uint32_t rank, T *lds) {
   constexpr int LP = any_lpr(SET, (int)sizeof(T));
   constexpr bool kLow = SET != kAnyWide, kMid = SET == kAnyNarrow || SET == kAnyAll || SET == kAnyRows,
                  kHigh = SET == kAnyWide || SET == kAnyAll;
   switch (padded_n(d.n)) {
-    case 4: if constexpr (kLow) reg_item<T, 4, NT, FUSED, false, true, true, LP>(d, rank, lds); break;
-    case 8: if constexpr (kLow) reg_item<T, 8, NT, FUSED, false, true, true, LP>(d, rank, lds); break;
-    case 12: if constexpr (kMid) reg_item<T, 12, NT, FUSED, false, true, true, LP>(d, rank, lds); break;
-    case 16: if constexpr (kMid) reg_item<T, 16, NT, FUSED, false, true, true, LP>(d, rank, lds); break;
-    case 20: if constexpr (kHigh) reg_item<T, 20, NT, FUSED, false, true, true, LP>(d, rank, lds); break;
-    case 24: if constexpr (kHigh) reg_item<T, 24, NT, FUSED, false, true, true, LP>(d, rank, lds); break;
-    case 28: if constexpr (kHigh) reg_item<T, 28, NT, FUSED, false, true, true, LP>(d, rank, lds); break;
-    case 32: if constexpr (kHigh) reg_item<T, 32, NT, FUSED, false, true, true, LP>(d, rank, lds); break;
+    case 4: if constexpr (kLow) reg_item<T, 4, NT, FUSED, false, true, true, LP, ALONE>(d, rank, lds); break;
+    case 8: if constexpr (kLow) reg_item<T, 8, NT, FUSED, false, true, true, LP, ALONE>(d, rank, lds); break;
+    case 12: if constexpr (kMid) reg_item<T, 12, NT, FUSED, false, true, true, LP, ALONE>(d, rank, lds); break;
+    case 16: if constexpr (kMid) reg_item<T, 16, NT, FUSED, false, true, true, LP, ALONE>(d, rank, lds); break;
+    case 20: if constexpr (kHigh) reg_item<T, 20, NT, FUSED, false, true, true, LP, ALONE>(d, rank, lds); break;
+    case 24: if constexpr (kHigh) reg_item<T, 24, NT, FUSED, false, true, true, LP, ALONE>(d, rank, lds); break;
+    case 28: if constexpr (kHigh) reg_item<T, 28, NT, FUSED, false, true, true, LP, ALONE>(d, rank, lds); break;
+    case 32: if constexpr (kHigh) reg_item<T, 32, NT, FUSED, false, true, true, LP, ALONE>(d, rank, lds); break;
     default: break;  // the planner only admits the sizes above
   }
 }
 
-// Waves per SIMD: FP32 rows of n <= 16 on two lanes at 512 threads leave room for
-// a second workgroup on the CU, as the fixed sizes do; the instances of one lane
-// per row are held to three (FP32) or two (FP64) 256-thread workgroups per CU.
-template <typename T, int NT, int SET>
+// Instances that hold systems of one workgroup, of several, or both (internal.h).
+template <typename T, int NT, bool FUSED, int SET>
+__device__ __forceinline__ void any_dispatch(const KSys &d, uint32_t rank, T *lds) {
+  if constexpr (!any_alone(SET)) {
+    any_class<T, NT, FUSED, SET, false>(d, rank, lds);
+  } else if constexpr (SET == kAnyTiny) {
+    any_class<T, NT, FUSED, SET, true>(d, rank, lds);
+  } else if (d.G == 1) {
+    any_class<T, NT, FUSED, SET, true>(d, rank, lds);
+  } else {
+    any_class<T, NT, FUSED, SET, false>(d, rank, lds);
+  }
+}
+
+// Waves per SIMD: kAnyRows is held to three (FP32) or two (FP64) workgroups of 256
+// threads per CU.
+template <typename T, int SET>
 constexpr int any_waves_per_eu() {
-  if (SET == kAnyRows) return sizeof(T) == 4 ? 3 : 2;
-  return (sizeof(T) == 4 && NT == 512 && SET == kAnyNarrow) ? 4 : 1;
+  return SET == kAnyRows ? (sizeof(T) == 4 ? 3 : 2) : 1;
 }
 
 template <typename T, int NT, bool FUSED, int SET>
-__global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(any_waves_per_eu<T, NT, SET>())))
+__global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(any_waves_per_eu<T, SET>())))
 pcg_any_kernel(KSys one, const KSys *__restrict__ systems, const uint32_t *__restrict__ items, uint32_t rounds,
                uint32_t stride) {
   extern __shared__ __attribute__((aligned(16))) unsigned char lds_raw[];

@@ -56,10 +56,10 @@ bool reg_supported(int n, bool bc) {
 bool any_supported(uint32_t n, int nt, int set) {
   switch (set) {
     case kAnyTiny: return n <= 8 && nt == 64;
-    case kAnyNarrow: return n <= 16 && (nt == 256 || nt == 512);
-    case kAnyRows: return n <= 16 && nt == 256;
-    case kAnyWide: return n > 16 && n <= 32 && (nt == 256 || nt == 512);
+    case kAnyNarrow: return n <= 16 && nt == 256;
+    case kAnyWide: return n > 16 && n <= 32 && nt == 256;
     case kAnyAll: return n <= 32 && nt == 512;
+    case kAnyRows: return n <= 16 && nt == 256;
     default: return false;
   }
 }
@@ -88,11 +88,12 @@ size_t reg_lds_bytes(int dtype, uint32_t n, uint32_t K, int nt, RegVariant v) {
 // Largest knots per workgroup the lane layout allows: lanes_per_row lanes per
 // row of the owned knots plus one ghost knot each side, and 4n ghost lanes (row
 // broadcast: 16 lanes per knot).  A system's only workgroup (alone) has no ghost
-// rows; the row-broadcast and paired items keep theirs.
+// rows on the instances that say so.
 uint32_t reg_max_knots(int dtype, uint32_t n, int nt, RegVariant v, bool alone) {
   if (v.bc) return n <= 16 && (uint32_t)nt >= 4 * n ? (uint32_t)nt / 16 - 2 : 0;
   const uint32_t rows = (uint32_t)nt / lanes_per_row(dtype, n, nt, v);
-  if (alone && !v.pair) return rows / n;
+  if (alone && any_alone(v.any) && v.any) return rows / n;
+  if (v.any == kAnyTiny) return 0;
   if (rows < 4 * n) return 0;
   return rows / n - 2;
 }
@@ -111,7 +112,7 @@ hipError_t reg_occupancy(int dtype, int n, int nt, size_t lds, int *wgs_per_cu, 
 
 hipError_t reg_launch(int dtype, int n, int nt, const KSys &one, const KSys *systems, const uint32_t *items,
                       uint32_t rounds, uint32_t stride, uint32_t grid, size_t lds, hipStream_t stream,
-                      RegVariant v) {
+                      RegVariant v, int block) {
   const void *k = reg_kernel(dtype, n, nt, v);
   if (!k) return hipErrorInvalidValue;
   KSys a0 = one;
@@ -119,7 +120,7 @@ hipError_t reg_launch(int dtype, int n, int nt, const KSys &one, const KSys *sys
   const uint32_t *a2 = items;
   uint32_t a3 = rounds, a4 = stride;
   void *args[] = {&a0, &a1, &a2, &a3, &a4};
-  return hipLaunchKernel(k, dim3(grid), dim3(nt), args, lds, stream);
+  return hipLaunchKernel(k, dim3(grid), dim3(block ? block : nt), args, lds, stream);
 }
 
 }  // namespace gbdpcg
