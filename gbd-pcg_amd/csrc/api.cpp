@@ -325,7 +325,9 @@ static int finish_reg_layout(int dtype, uint32_t n, uint32_t N, Layout *c) {
   // a lone workgroup needs the waves of its rows only: at n = 20, N = 12 FP32 four
   // of eight
   if (c->G == 1 && c->any && any_alone(c->any)) {
-    const uint32_t lanes = n * N * (uint32_t)any_lpr(c->any, (int)tsize(dtype));
+    const uint32_t lpr = (uint32_t)any_lpr(c->any, (int)tsize(dtype)), nt = (uint32_t)c->nt;
+    const uint32_t lanes = any_two_rows(c->any, (int)tsize(dtype)) ? two_rows_lanes(n, N, nt) * N
+                                                                   : alone_lanes(n, N, lpr, nt, (uint32_t)tsize(dtype)) * N * lpr;
     c->block = (int)std::min<uint32_t>((uint32_t)c->nt, ceil_div(lanes, 64) * 64);
   }
   if (!c->stride) c->stride = c->G <= per_xcd ? (uint32_t)kXcds : 1u;
@@ -393,21 +395,29 @@ static int plan_single_reg(int dtype, uint32_t n, uint32_t N, uint32_t want_G, u
 // 1.75 / 2.67, n = 2 N = 30 on one wave 0.19 / 1.13 and 0.23 / 1.99; FP64: n = 6
 // N = 40 0.90 / 1.75 and 1.21 / 2.92, n = 32 N = 8 2.07 / 3.91 reference form).
 // GBDPCG_ERR_UNSUPPORTED when no workgroup holds it.
-static int plan_one_workgroup(int dtype, uint32_t n, uint32_t N, bool fused, bool pair, Layout *L) {
+// as_pair: a solve whose sums are to be those of the paired forward + adjoint solve
+// of the same system (adjoint-only in FP64): that solve's layout.
+static int plan_one_workgroup(int dtype, uint32_t n, uint32_t N, bool fused, bool pair, bool as_pair, Layout *L) {
   if (n > 32 || (fused && N < 2)) return GBDPCG_ERR_UNSUPPORTED;
-  const bool both = pair && fused && n <= 14 && reg_supported((int)n) && N >= 4;
-  for (int nt : {64, 256, 512}) {
+  const bool both = (pair || as_pair) && fused && n <= 14 && reg_supported((int)n) && N >= 4;
+  for (const int set : {(int)kAnyTiny, (int)kAnyRows, (int)kAnyAll, (int)kAnyLong}) {
+    const int nt = set == kAnyTiny ? 64 : set == kAnyRows ? 256 : 512;
     Layout c;
-    c.pair = both;
+    c.pair = both && pair;
     // FP64 rows of n = 12 and 14 broadcast by DPP up to N = 14: 1.14 us per fused
     // iteration at N = 14, 1.31 on kAnyRows (reference form 1.46, 1.53)
     c.bc = nt == 256 && dtype == GBDPCG_F64 && N >= 4 && reg_supported((int)n, true) &&
            N <= reg_max_knots(dtype, n, nt, RegVariant{fused, true});
-    c.any = both || c.bc ? kAnyNone : nt == 256 ? kAnyRows : any_set(n, nt);
+    c.any = both || c.bc ? kAnyNone : set;
     c.fused = fused;
     c.nt = nt;
     if (c.any ? !any_supported(n, nt, c.any) : nt == 64) continue;
-    if (N > reg_max_knots(dtype, n, nt, c.variant(), true)) continue;
+    RegVariant v = c.variant();
+    v.pair = both;
+    if (N > reg_max_knots(dtype, n, nt, v, true)) continue;
+    // FP64 rows that must be packed (alone_lanes) gain nothing in the fused form:
+    // n = 14 N = 36 2.14 us per iteration, 2.04 on several ranks
+    if (set == kAnyLong && dtype == GBDPCG_F64 && fused && n > 12 && n < 16 && 16 * N > (uint32_t)nt) continue;
     c.G = 1;
     c.stride = 0;
     const int rc = finish_reg_layout(dtype, n, N, &c);
@@ -427,9 +437,11 @@ static std::string single_key(int dev, int dtype, uint32_t n, uint32_t N, bool f
 }
 
 // Kinds of layout, as the tuner's choices name them (TuneChoice.a).
-enum : uint32_t { kKindLds = 0, kKindReg = 1, kKindRowcast = 2, kKindAny = 3, kKindRows = 4 };
+enum : uint32_t { kKindLds = 0, kKindReg = 1, kKindRowcast = 2, kKindAny = 3, kKindRows = 4, kKindLong = 5 };
 static uint32_t kind_of(const Layout &L) {
-  return !L.reg ? kKindLds : L.bc ? kKindRowcast : L.any == kAnyRows ? kKindRows : L.any ? kKindAny : kKindReg;
+  if (!L.reg) return kKindLds;
+  if (L.any) return L.any == kAnyRows ? kKindRows : L.any == kAnyLong ? kKindLong : kKindAny;
+  return L.bc ? kKindRowcast : kKindReg;
 }
 
 // Rebuilds a layout from its (kind, threads, workgroups, stride); checks that it
@@ -439,19 +451,19 @@ static int layout_from(int dtype, uint32_t n, uint32_t N, uint32_t kind, int nt,
   DeviceInfo di;
   int rc = device_info(cur_dev(), &di);
   if (rc < 0) return rc;
-  if (kind > kKindRows || G == 0 || G > N || (stride != 1 && stride != (uint32_t)kXcds)) return GBDPCG_ERR_UNSUPPORTED;
+  if (kind > kKindLong || G == 0 || G > N || (stride != 1 && stride != (uint32_t)kXcds)) return GBDPCG_ERR_UNSUPPORTED;
   Layout t;
   t.G = G;
   t.stride = stride;
   t.grid = G * stride;
   t.reg = kind != kKindLds;
   t.bc = kind == kKindRowcast;
-  t.any = kind == kKindRows ? kAnyRows : kind == kKindAny ? any_set(n, nt) : kAnyNone;
+  t.any = kind == kKindRows ? kAnyRows : kind == kKindLong ? kAnyLong : kind == kKindAny ? any_set(n, nt) : kAnyNone;
   t.pair = t.reg && !t.any && fused && pair && n <= 14;
   t.fused = fused;
   t.nt = t.reg ? nt : kThreads;
   if (t.any) {
-    if (!any_supported(n, nt, t.any) || (nt == 64 && G != 1) || (fused && N < 2) || (G > 1 && N / G < 2) ||
+    if (!any_supported(n, nt, t.any) || ((nt == 64 || t.any == kAnyLong) && G != 1) || (fused && N < 2) || (G > 1 && N / G < 2) ||
         ceil_div(N, G) > reg_max_knots(dtype, n, nt, t.variant(), G == 1))
       return GBDPCG_ERR_UNSUPPORTED;
     rc = finish_reg_layout(dtype, n, N, &t);
@@ -480,7 +492,7 @@ static int layout_from(int dtype, uint32_t n, uint32_t N, uint32_t kind, int nt,
 }
 
 static int untuned_layout(int dtype, uint32_t n, uint32_t N, bool fused, const gbdpcg_config *cfg, Layout *L,
-                          bool pair) {
+                          bool pair, bool as_pair) {
   const bool open = cfg->grid[0] == 0 && cfg->knots_per_wg == 0;
   // automatic: one workgroup when it holds the system; then the row-broadcast
   // layout first for FP64 (measured faster there), the column-chunk register
@@ -495,7 +507,8 @@ static int untuned_layout(int dtype, uint32_t n, uint32_t N, bool fused, const g
     if (rc < 0) return rc;
   }
   int rc = GBDPCG_ERR_UNSUPPORTED;
-  if (cfg->kernel == GBDPCG_KERNEL_AUTO && open && req_nt == 0) rc = plan_one_workgroup(dtype, n, N, fused, pair, L);
+  if (cfg->kernel == GBDPCG_KERNEL_AUTO && open && req_nt == 0)
+    rc = plan_one_workgroup(dtype, n, N, fused, pair, as_pair, L);
   if (rc == GBDPCG_ERR_UNSUPPORTED &&
       ((cfg->kernel == GBDPCG_KERNEL_AUTO && dtype == GBDPCG_F64) || cfg->kernel == GBDPCG_KERNEL_ROWCAST))
     rc = plan_single_reg(dtype, n, N, cfg->grid[0], cfg->knots_per_wg, L, req_nt, fused, true, pair);
@@ -516,14 +529,14 @@ static int untuned_layout(int dtype, uint32_t n, uint32_t N, bool fused, const g
 }
 
 static int choose_layout(int dev, int dtype, uint32_t n, uint32_t N, bool fused, const gbdpcg_config *cfg,
-                         Layout *L, bool pair = false) {
+                         Layout *L, bool pair = false, bool as_pair = false) {
   if (cfg->grid[0] == 0 && cfg->knots_per_wg == 0 && cfg->kernel == GBDPCG_KERNEL_AUTO && cfg->threads == 0) {
     TuneChoice c;
     if (tune_lookup(single_key(dev, dtype, n, N, fused, cfg->exit_mode), &c) &&
         layout_from(dtype, n, N, c.a, (int)c.b, c.c, c.d, L, fused, pair) == GBDPCG_OK)
       return GBDPCG_OK;
   }
-  return untuned_layout(dtype, n, N, fused, cfg, L, pair);
+  return untuned_layout(dtype, n, N, fused, cfg, L, pair, as_pair);
 }
 
 // Whether the LDS-resident kernel cannot give every workgroup the 2 knots the
@@ -541,11 +554,11 @@ static bool lds_fused_unfit(int dtype, uint32_t n, uint32_t N) {
 // queries and the occupancy check (microseconds on every call otherwise).  The
 // caller holds ws->mu.
 static int cached_layout(Workspace *ws, int dtype, uint32_t n, uint32_t N, bool fused, const gbdpcg_config *cfg,
-                         Layout *L, bool pair) {
+                         Layout *L, bool pair, bool as_pair) {
   const uint64_t k0 = (uint64_t)n | ((uint64_t)N << 32);
   const uint64_t k1 = (uint64_t)cfg->grid[0] | ((uint64_t)cfg->knots_per_wg << 32);
   const uint64_t k2 = (uint64_t)(dtype & 3) | ((uint64_t)fused << 2) | ((uint64_t)pair << 3) |
-                      ((uint64_t)(cfg->exit_mode & 3) << 4) | ((uint64_t)(cfg->kernel & 15) << 8) |
+                      ((uint64_t)(cfg->exit_mode & 3) << 4) | ((uint64_t)as_pair << 6) | ((uint64_t)(cfg->kernel & 15) << 8) |
                       ((uint64_t)cfg->threads << 16);
   const uint64_t gen = tune_generation();
   for (const LayoutMemo &m : ws->layouts)
@@ -553,7 +566,7 @@ static int cached_layout(Workspace *ws, int dtype, uint32_t n, uint32_t N, bool 
       *L = m.L;
       return GBDPCG_OK;
     }
-  const int rc = choose_layout(ws->device, dtype, n, N, fused, cfg, L, pair);
+  const int rc = choose_layout(ws->device, dtype, n, N, fused, cfg, L, pair, as_pair);
   if (rc < 0) return rc;
   for (LayoutMemo &m : ws->layouts)
     if (m.k0 == k0 && m.k1 == k1 && m.k2 == k2) {
@@ -657,13 +670,15 @@ static int solve_locked(Workspace *ws, int dtype, uint32_t n, uint32_t N, const 
   if (fused && N < 2) fused = false;  // one knot: the reference recurrence
   // forward + adjoint on a register kernel (n <= 14): both solves in one loop
   bool pair = fused && (flags & KF_FWD) && (flags & KF_ADJ) && n <= 14;
+  // adjoint alone in FP64: the sums, to the last bits, of the paired solve
+  const bool as_pair = dtype == GBDPCG_F64 && (flags & (KF_FWD | KF_ADJ)) == KF_ADJ;
   Layout L;
-  int rc = cached_layout(ws, dtype, n, N, fused, cfg, &L, pair);
+  int rc = cached_layout(ws, dtype, n, N, fused, cfg, &L, pair, as_pair);
   if (rc == GBDPCG_ERR_TOO_LARGE && fused && lds_fused_unfit(dtype, n, N)) {
     // no layout with 2 knots per workgroup: the reference recurrence, which
     // takes one knot per workgroup (batch plans decide the same per system)
     fused = pair = false;
-    rc = cached_layout(ws, dtype, n, N, false, cfg, &L, false);
+    rc = cached_layout(ws, dtype, n, N, false, cfg, &L, false, as_pair);
   }
   if (rc < 0) return rc;
 
@@ -1137,7 +1152,7 @@ int gbdpcg_tune_single(int dtype, uint32_t n, uint32_t N, const void *d_S, const
     gbdpcg_config c = *cfg;  // the layout an untuned solve would take
     c.grid[0] = 0;
     c.knots_per_wg = c.threads = 0;
-    rc = untuned_layout(dtype, n, N, fused, &c, &def, false);
+    rc = untuned_layout(dtype, n, N, fused, &c, &def, false, false);
     if (rc == GBDPCG_ERR_TOO_LARGE && fused && lds_fused_unfit(dtype, n, N)) {
       // solves of this config run the reference iteration (solve_locked): tune
       // those layouts, cached under that recurrence's key, which they look up
@@ -1173,8 +1188,8 @@ int gbdpcg_tune_single(int dtype, uint32_t n, uint32_t N, const void *d_S, const
 
   const uint32_t Ks[] = {1, 2, 3, 4, 5, 6, 7, 8, 10, 12, 14, 16, 20, 24, 28, 32, 40, 48, 64};
   for (const uint32_t kind : {(uint32_t)kKindRowcast, (uint32_t)kKindReg, (uint32_t)kKindAny, (uint32_t)kKindRows,
-                              (uint32_t)kKindLds}) {
-    const bool any = kind == kKindAny || kind == kKindRows;
+                              (uint32_t)kKindLong, (uint32_t)kKindLds}) {
+    const bool any = kind == kKindAny || kind == kKindRows || kind == kKindLong;
     const uint32_t kid = kind == kKindRowcast ? GBDPCG_KERNEL_ROWCAST
                          : kind == kKindLds   ? GBDPCG_KERNEL_LDS
                                               : GBDPCG_KERNEL_REGISTER;

@@ -80,13 +80,30 @@ enum : int {
   kAnyWide = 3,    // 16 < n <= 32, two lanes per row, 256 threads: single solves
   kAnyAll = 4,     // n <= 32, one (FP32) or two (FP64) lanes per row, 512 threads
   kAnyRows = 5,    // n <= 16, one lane per row, 256 threads
+  kAnyLong = 6,    // n <= 16, 512 threads, two rows (FP32) or one (FP64) per lane: systems of one workgroup
 };
 __host__ __device__ constexpr int any_lpr(int set, int tsize) {
   return set == kAnyNarrow || set == kAnyWide || (set == kAnyAll && tsize == 8) ? 2 : 1;
 }
 // Whether an instance runs systems of one workgroup without exchange code, ghost
-// rows or their lanes (kAnyTiny runs nothing else).
+// rows or their lanes (kAnyTiny and kAnyLong run nothing else).
 __host__ __device__ constexpr bool any_alone(int set) { return set != kAnyNarrow && set != kAnyWide; }
+
+__host__ __device__ constexpr bool any_two_rows(int set, int tsize) { return set == kAnyLong && tsize == 4; }
+
+// Lanes (of one row each) between the knots of a system's only workgroup: 16 (two
+// rows per lane: 8) for n = 13..15 where that fits, so that the lanes which an LDS
+// read serves together want the same window.  FP64 n = 14 N = 32: 1.70 us per fused
+// iteration, 2.07 with the rows packed (reference form 2.01, 2.40); up to N = 12
+// the rows packed take fewer waves (N = 9: 1.12 against 1.16).  FP32 on one lane
+// per row is faster packed (N = 32: 1.01 against 1.05), on two rows per lane not
+// (n = 14 N = 64: 1.25 against 1.21).
+__host__ __device__ constexpr uint32_t alone_lanes(uint32_t n, uint32_t N, uint32_t lpr, uint32_t nt, uint32_t tsize) {
+  return tsize == 8 && n > 12 && n < 16 && N > 12 && 16 * N * lpr <= nt ? 16u : n;
+}
+__host__ __device__ constexpr uint32_t two_rows_lanes(uint32_t n, uint32_t N, uint32_t nt) {
+  return n > 12 && n < 16 && 8 * N <= nt ? 8u : (n + 1) / 2;
+}
 
 // Words (64-bit) of one exchange record: kRecScalars scalar slots (3 per wave of
 // the publishing workgroup, up to 8 waves) + two edge blocks, each a left edge

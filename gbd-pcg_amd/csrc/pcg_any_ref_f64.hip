@@ -13,7 +13,7 @@ const void *ap() {
 
 const void *any_ref_kernel_ptr_f64(int nt, int set) {
   if (nt == 64) return set == kAnyTiny ? ap<64, kAnyTiny>() : nullptr;
-  if (nt == 512) return set == kAnyAll ? ap<512, kAnyAll>() : nullptr;
+  if (nt == 512) return set == kAnyAll ? ap<512, kAnyAll>() : set == kAnyLong ? ap<512, kAnyLong>() : nullptr;
   if (nt != 256) return nullptr;
   switch (set) {
     case kAnyNarrow: return ap<256, kAnyNarrow>();

@@ -1009,14 +1009,15 @@ __device__ __forceinline__ void reg_item(const KSys &d, uint32_t rank, T *lds) {
     it.m = t >> 4;
     it.row = t & 15;
   } else {
-    it.m = it.q / n;
-    it.row = it.q - it.m * n;
+    const int ln = ALONE ? (int)alone_lanes((uint32_t)n, d.N, R::LPR, NT, sizeof(T)) : n;
+    it.m = it.q / ln;
+    it.row = it.q - it.m * ln;
     // no neighbours: no lanes for ghost rows, so it holds two knots more
     if (ALONE || (!R::RT && it.G == 1)) ++it.m;
   }
   it.kg = it.a - 1 + it.m;
-  it.act_u = it.m < K + 2 && (!BC || it.row < n);
-  it.act_w = it.m >= 1 && it.m <= K && (!BC || it.row < n);
+  it.act_u = it.m < K + 2 && (!(BC || ALONE) || it.row < n);
+  it.act_w = it.m >= 1 && it.m <= K && (!(BC || ALONE) || it.row < n);
   it.owner = it.act_w && it.c == 0;
   it.ghost = it.c == R::LPR - 1 && it.q < 4 * n && !ALONE && (R::RT || it.G > 1);
   if (!ALONE) it.set_edge_slots();
@@ -1421,6 +1422,270 @@ __device__ __forceinline__ void reg_item(const KSys &d, uint32_t rank, T *lds) {
   }
   if (timed_out && t == 0 && d.err != nullptr)
     __hip_atomic_store(d.err, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+// Two rows per lane: FP32 systems of one workgroup (stateSize n <= NS as in
+// RegItem) too large for a lane per row.  Lane (m, h) holds rows 2h and 2h + 1 of
+// knot m - 1, so a vector window read from LDS serves two rows: the iteration is
+// bound by those reads and the multiply-adds (two waves per SIMD), still without
+// an exchange.  Per iteration, fused / reference form, against several ranks:
+// n = 12 N = 64 1.09 / 1.27 us (1.36 / 2.23), n = 14 N = 64 1.21 / 1.41 (1.40 /
+// 2.32), n = 13 N = 50 1.22 / 1.39 (1.63 / 2.37), n = 8 N = 128 0.95 / 1.14 (1.50 /
+// 2.28).
+template <int NS, int NT>
+struct TwoRows {
+  static constexpr int nP = NS, CW = 3 * NS, NWAVES = NT / 64;
+  int n, N, m, row;        // row: the first of the lane's rows
+  bool act, second;        // the lane has rows; it has both (odd n: the last lane of a knot has one)
+  float *wsum;
+
+  // y = the lane's two rows times the window of knots m-1..m+1 of vec
+  __device__ __forceinline__ void mv(const float (&a)[CW], const float (&b)[CW], const float *vec, float &ya,
+                                     float &yb) const {
+    float a0 = 0, a1 = 0, a2 = 0, a3 = 0, b0 = 0, b1 = 0, b2 = 0, b3 = 0;
+    if (act) {
+      const float *x = vec + m * nP;
+#pragma unroll
+      for (int j = 0; j < CW; j += 4) {
+        const float4 xv = *reinterpret_cast<const float4 *>(x + j);
+        a0 = __builtin_fmaf(a[j + 0], xv.x, a0);
+        b0 = __builtin_fmaf(b[j + 0], xv.x, b0);
+        a1 = __builtin_fmaf(a[j + 1], xv.y, a1);
+        b1 = __builtin_fmaf(b[j + 1], xv.y, b1);
+        a2 = __builtin_fmaf(a[j + 2], xv.z, a2);
+        b2 = __builtin_fmaf(b[j + 2], xv.z, b2);
+        a3 = __builtin_fmaf(a[j + 3], xv.w, a3);
+        b3 = __builtin_fmaf(b[j + 3], xv.w, b3);
+      }
+    }
+    ya = (a0 + a1) + (a2 + a3);
+    yb = (b0 + b1) + (b2 + b3);
+  }
+
+  __device__ __forceinline__ void put(float *vec, float ya, float yb) const {
+    if (act) *reinterpret_cast<float2 *>(vec + (m + 1) * nP + row) = make_float2(ya, yb);
+  }
+
+  // Workgroup totals in every wave; the caller has a barrier between two calls.
+  __device__ __forceinline__ void totals(float &s0, float &s1, float &s2) const {
+    wave_sum3(s0, s1, s2);
+    const int w = threadIdx.x >> 6;
+    if ((threadIdx.x & 63) == 0) {
+      wsum[w * 3 + 0] = s0;
+      wsum[w * 3 + 1] = s1;
+      wsum[w * 3 + 2] = s2;
+    }
+    __syncthreads();
+    const int l = (int)threadIdx.x & 3;
+    const float v = waves_total<NWAVES, 3>(wsum, l < 3 ? l : 0);
+    s0 = read_lane(v, 0);
+    s1 = read_lane(v, 1);
+    s2 = read_lane(v, 2);
+  }
+};
+
+template <int NS, int NT, bool FUSED>
+__device__ __forceinline__ void two_rows_item(const KSys &d, float *lds) {
+  using R = TwoRows<NS, NT>;
+  constexpr int nP = R::nP, CW = R::CW;
+  R it;
+  const int n = (int)d.n, N = (int)d.N, stride = (int)blockDim.x;
+  it.n = n;
+  it.N = N;
+  const int VL = (N + 4) * nP + CW;
+  float *rv = lds, *uv = rv + VL, *xv = uv + VL, *lv = xv + VL;
+  it.wsum = lv + VL;
+  const int total = 4 * VL + 3 * R::NWAVES;
+  const int t = opaque_tid();
+  {
+    const int half = (int)two_rows_lanes((uint32_t)n, d.N, NT), k = t / half;
+    it.m = k + 1;
+    it.row = 2 * (t - k * half);
+    it.act = k < N && it.row < n;
+    it.second = it.act && it.row + 1 < n;
+  }
+  const int kg = it.m - 1, own = (it.m + 1) * nP + it.row;
+  const bool fwd = (d.flags & KF_FWD) != 0, adj = (d.flags & KF_ADJ) != 0, rel = (d.flags & KF_REL) != 0;
+  for (int i = opaque_tid(); i < total; i += stride) lds[i] = 0.f;
+
+  // one HBM round trip: right-hand side, guess and matrices together
+  const float *lam0 = static_cast<const float *>(d.lambda);
+  auto rhs_at = [&](const void *p, float &a, float &b) {
+    const float *v = static_cast<const float *>(p) + (size_t)kg * n + it.row;
+    a = it.act ? gptr(v)[0] : 0.f;
+    b = it.second ? gptr(v)[1] : 0.f;
+  };
+  float xa, xb, ba, bb;
+  rhs_at(lam0, xa, xb);
+  rhs_at(fwd ? d.gamma : d.glambda, ba, bb);
+  float sa[CW], sb[CW], pa[CW], pb[CW];
+  load_chunk<float, NS, CW, kLoadAny>(sa, static_cast<const float *>(d.S), kg, it.row, 0, N, it.act, n);
+  load_chunk<float, NS, CW, kLoadAny>(sb, static_cast<const float *>(d.S), kg, it.row + 1, 0, N, it.second, n);
+  load_chunk<float, NS, CW, kLoadAny>(pa, static_cast<const float *>(d.Pinv), kg, it.row, 0, N, it.act, n);
+  load_chunk<float, NS, CW, kLoadAny>(pb, static_cast<const float *>(d.Pinv), kg, it.row + 1, 0, N, it.second, n);
+  __syncthreads();
+  it.put(fwd ? xv : lv, xa, xb);
+  __syncthreads();
+
+  RegOut fo{0, GBDPCG_CONVERGED, 0.0, 0.0}, ao{0, GBDPCG_CONVERGED, 0.0, 0.0};
+  for (int pass = fwd ? 0 : 1; pass <= (adj ? 1 : 0); ++pass) {
+    RegOut out{0, GBDPCG_MAX_ITER, 0.0, 0.0};
+    if (pass == 1) {
+      // lambda stays in lv; the adjoint starts from x = 0
+      if (fwd) {
+        it.put(lv, xa, xb);
+        rhs_at(d.glambda, ba, bb);
+      }
+      xa = xb = 0.f;
+      it.put(xv, 0.f, 0.f);
+      __syncthreads();
+    }
+    float ra, rb;
+    it.mv(sa, sb, xv, ra, rb);
+    ra = ba - ra;
+    rb = bb - rb;
+    it.put(rv, ra, rb);
+    float gg = ba * ba + bb * bb, z0 = 0, z1 = 0;
+    it.totals(gg, z0, z1);
+    const double thr = rel ? d.tol * d.tol * (double)gg : d.tol;
+    // u = Pinv r (the reference form's z)
+    float ua, ub;
+    it.mv(pa, pb, rv, ua, ub);
+    it.put(uv, ua, ub);
+    __syncthreads();
+    float eta = ra * ua + rb * ub, delta = 0, rr = ra * ra + rb * rb, wa = 0, wb = 0;
+    if constexpr (FUSED) {
+      it.mv(sa, sb, uv, wa, wb);
+      delta = wa * ua + wb * ub;
+    }
+    it.totals(eta, delta, rr);
+    // p = u (reference form: held in uv as well); s = w
+    float qa = ua, qb = ub, va = wa, vb = wb;
+    float alpha = FUSED && delta != 0.f ? eta / delta : 0.f;
+    out.eta = (double)eta;
+    out.rr = (double)rr;
+    bool run = d.max_iter > 0;
+    if (!finite_t(eta) || !finite_t(rr)) {
+      out.status = GBDPCG_NONFINITE;
+      run = false;
+    } else if (eta == 0.f) {
+      out.status = rr == 0.f ? GBDPCG_CONVERGED : GBDPCG_BREAKDOWN;
+      run = false;
+    } else if (FUSED && (delta == 0.f || !finite_t(alpha))) {
+      out.status = GBDPCG_BREAKDOWN;
+      run = false;
+    }
+    uint32_t iter = 0;
+    __syncthreads();  // totals above before those of the loop
+    while (run) {
+      if constexpr (FUSED) {
+        xa = fmaT(alpha, qa, xa);
+        xb = fmaT(alpha, qb, xb);
+        ra = fmaT(-alpha, va, ra);
+        rb = fmaT(-alpha, vb, rb);
+        it.put(rv, ra, rb);
+        __syncthreads();
+        it.mv(pa, pb, rv, ua, ub);
+        it.put(uv, ua, ub);
+        __syncthreads();
+        it.mv(sa, sb, uv, wa, wb);
+        float eta_new = ra * ua + rb * ub, delta_new = wa * ua + wb * ub;
+        rr = ra * ra + rb * rb;
+        it.totals(eta_new, delta_new, rr);
+        ++iter;
+        out.eta = (double)eta_new;
+        out.rr = (double)rr;
+        const bool conv = rel ? ((double)rr <= thr) : (__builtin_fabs((double)eta_new) < thr);
+        const bool nonfin = !finite_t(eta_new);
+        const float beta = qdiv(eta_new, eta);
+        const float den = delta_new - beta * qdiv(eta_new, alpha);
+        const bool brk = den == 0.f || !finite_t(den);
+        const float alpha_new = qdiv(eta_new, den);
+        if (conv || nonfin || brk) {
+          out.status = conv ? GBDPCG_CONVERGED : nonfin ? GBDPCG_NONFINITE : GBDPCG_BREAKDOWN;
+          break;
+        }
+        alpha = alpha_new;
+        eta = eta_new;
+        qa = fmaT(beta, qa, ua);
+        qb = fmaT(beta, qb, ub);
+        va = fmaT(beta, va, wa);
+        vb = fmaT(beta, vb, wb);
+      } else {
+        it.mv(sa, sb, uv, va, vb);
+        float pv = qa * va + qb * vb, y1 = 0, y2 = 0;
+        it.totals(pv, y1, y2);
+        if (pv == 0.f || !finite_t(pv)) {
+          out.status = pv == 0.f ? GBDPCG_BREAKDOWN : GBDPCG_NONFINITE;
+          break;
+        }
+        alpha = qdiv(eta, pv);
+        xa = fmaT(alpha, qa, xa);
+        xb = fmaT(alpha, qb, xb);
+        ra = fmaT(-alpha, va, ra);
+        rb = fmaT(-alpha, vb, rb);
+        it.put(rv, ra, rb);
+        __syncthreads();
+        it.mv(pa, pb, rv, ua, ub);
+        float eta_new = ra * ua + rb * ub, y3 = 0;
+        rr = ra * ra + rb * rb;
+        it.totals(eta_new, y3, rr);
+        ++iter;
+        out.eta = (double)eta_new;
+        out.rr = (double)rr;
+        if (rel ? ((double)rr <= thr) : (__builtin_fabs((double)eta_new) < thr)) {
+          out.status = GBDPCG_CONVERGED;
+          break;
+        }
+        if (!finite_t(eta_new)) {
+          out.status = GBDPCG_NONFINITE;
+          break;
+        }
+        const float beta = qdiv(eta_new, eta);
+        eta = eta_new;
+        qa = fmaT(beta, qa, ua);
+        qb = fmaT(beta, qb, ub);
+        it.put(uv, qa, qb);
+        __syncthreads();
+      }
+      run = iter < d.max_iter;
+    }
+    out.iters = (int)iter;
+    if (pass == 0) fo = out; else ao = out;
+    float *dst = static_cast<float *>(pass == 0 ? d.lambda : d.ggamma) + (size_t)kg * n + it.row;
+    if (it.act) gptr(dst)[0] = xa;
+    if (it.second) gptr(dst)[1] = xb;
+    if (pass == 1) {
+      it.put(xv, xa, xb);
+      __syncthreads();
+      // g_S block rows, as in reg_item
+      const int bs = 3 * n * n;
+      float *gS = static_cast<float *>(d.gS);
+      for (int e = opaque_tid(); e < N * bs; e += stride) {
+        const int k = e / bs, wq = e - k * bs, col = wq / n, r_ = wq - col * n, seg = col / n, cc = col - seg * n;
+        const int j = k - 1 + seg;
+        float val = 0;
+        if (j >= 0 && j < N) {
+          const int lk = (k + 2) * nP, lj = (j + 2) * nP;
+          val = -0.5f * (xv[lk + r_] * lv[lj + cc] + lv[lk + r_] * xv[lj + cc]);
+        }
+        gptr(gS)[e] = val;
+      }
+    }
+    __syncthreads();
+  }
+  if (threadIdx.x == 0 && d.result != nullptr) {
+    gbdpcg_result res;
+    res.iters = fo.iters;
+    res.status = fo.status;
+    res.adj_iters = ao.iters;
+    res.adj_status = ao.status;
+    res.eta = fo.eta;
+    res.rr = fo.rr;
+    res.adj_eta = ao.eta;
+    res.adj_rr = ao.rr;
+    *d.result = res;
+  }
 }
 
 // Forward and adjoint solves of one system iterated together (fused recurrence;
@@ -1983,7 +2248,7 @@ pcg_pair_kernel(KSys one, const KSys *__restrict__ systems,
 template <typename T, int NT, bool FUSED, int SET, bool ALONE>
 __device__ __forceinline__ void any_class(const KSys &d, uint32_t rank, T *lds) {
   constexpr int LP = any_lpr(SET, (int)sizeof(T));
-  constexpr bool kLow = SET != kAnyWide, kMid = SET == kAnyNarrow || SET == kAnyAll || SET == kAnyRows,
+  constexpr bool kLow = SET != kAnyWide, kMid = SET != kAnyTiny && SET != kAnyWide,
                  kHigh = SET == kAnyWide || SET == kAnyAll;
   switch (padded_n(d.n)) {
     case 4: if constexpr (kLow) reg_item<T, 4, NT, FUSED, false, true, true, LP, ALONE>(d, rank, lds); break;
@@ -2001,9 +2266,17 @@ __device__ __forceinline__ void any_class(const KSys &d, uint32_t rank, T *lds) 
 // Instances that hold systems of one workgroup, of several, or both (internal.h).
 template <typename T, int NT, bool FUSED, int SET>
 __device__ __forceinline__ void any_dispatch(const KSys &d, uint32_t rank, T *lds) {
-  if constexpr (!any_alone(SET)) {
+  if constexpr (SET == kAnyLong && sizeof(T) == 4) {
+    switch (padded_n(d.n)) {
+      case 4: two_rows_item<4, NT, FUSED>(d, lds); break;
+      case 8: two_rows_item<8, NT, FUSED>(d, lds); break;
+      case 12: two_rows_item<12, NT, FUSED>(d, lds); break;
+      case 16: two_rows_item<16, NT, FUSED>(d, lds); break;
+      default: break;
+    }
+  } else if constexpr (!any_alone(SET)) {
     any_class<T, NT, FUSED, SET, false>(d, rank, lds);
-  } else if constexpr (SET == kAnyTiny) {
+  } else if constexpr (SET == kAnyTiny || SET == kAnyLong) {
     any_class<T, NT, FUSED, SET, true>(d, rank, lds);
   } else if (d.G == 1) {
     any_class<T, NT, FUSED, SET, true>(d, rank, lds);

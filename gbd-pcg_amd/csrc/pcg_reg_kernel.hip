@@ -60,6 +60,7 @@ bool any_supported(uint32_t n, int nt, int set) {
     case kAnyWide: return n > 16 && n <= 32 && nt == 256;
     case kAnyAll: return n <= 32 && nt == 512;
     case kAnyRows: return n <= 16 && nt == 256;
+    case kAnyLong: return n <= 16 && nt == 512;
     default: return false;
   }
 }
@@ -92,8 +93,9 @@ size_t reg_lds_bytes(int dtype, uint32_t n, uint32_t K, int nt, RegVariant v) {
 uint32_t reg_max_knots(int dtype, uint32_t n, int nt, RegVariant v, bool alone) {
   if (v.bc) return n <= 16 && (uint32_t)nt >= 4 * n ? (uint32_t)nt / 16 - 2 : 0;
   const uint32_t rows = (uint32_t)nt / lanes_per_row(dtype, n, nt, v);
-  if (alone && any_alone(v.any) && v.any) return rows / n;
-  if (v.any == kAnyTiny) return 0;
+  if (v.any && alone && any_alone(v.any))
+    return any_two_rows(v.any, dtype == GBDPCG_F64 ? 8 : 4) ? (uint32_t)nt / ((n + 1) / 2) : rows / n;
+  if (v.any == kAnyTiny || v.any == kAnyLong) return 0;
   if (rows < 4 * n) return 0;
   return rows / n - 2;
 }

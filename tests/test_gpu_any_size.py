@@ -18,9 +18,10 @@ SIZES = [1, 2, 3, 4, 5, 8, 9, 12, 13, 14, 16, 17, 20, 21, 24, 25, 28, 29, 32]
 
 
 def horizons(n):
-    """What 64 lanes of one per row, and 256 and 512 lanes of two (256 and 512 of
-    one for n <= 2) hold of a system without neighbours, and one knot more."""
-    edges = [64 // n, 128 // n, 256 // n] + ([512 // n] if n <= 2 else [])
+    """What one workgroup of 64, 256 or 512 lanes holds of a system without
+    neighbours, one or two lanes per row or two rows per lane, and one knot more;
+    where rows get 16 lanes per knot (n = 13..15 from N = 13 to 32)."""
+    edges = [64 // n, 128 // n, 256 // n, 512 // n, 512 // ((n + 1) // 2)] + ([12, 32, 64] if 12 < n < 16 else [])
     return sorted({N for e in edges for N in (e, e + 1) if 2 <= N <= 300})
 
 
