@@ -632,6 +632,101 @@ __host__ __device__ constexpr ChunkTables<NS, CW> chunk_tables() {
   return t;
 }
 
+// Element at a uniform element offset from A plus a per-lane one (32-bit byte
+// offsets against a scalar base: one scalar addition and one load).
+template <typename V, typename T>
+__device__ __forceinline__ V load_at(const T *A, uint32_t uniform_off, uint32_t lane_off) {
+  const auto *col = reinterpret_cast<const __attribute__((address_space(1))) unsigned char *>(gptr(A + uniform_off));
+  return *reinterpret_cast<const __attribute__((address_space(1))) V *>(col + lane_off * (uint32_t)sizeof(T));
+}
+
+// Lane offsets of the three blocks of block row kg at `row` (a lane without the
+// block is sent to the diagonal block of its own or of the first knot, so that
+// every load is in bounds and none reads the padding) and whether each is absent.
+struct BlockRow {
+  uint32_t off[3];
+  bool absent[3];
+};
+__device__ __forceinline__ BlockRow block_row(int kg, int row, int N, bool active, int n) {
+  BlockRow b;
+  const uint32_t nn = (uint32_t)(n * n);
+  const bool ok = active && kg >= 0 && kg < N;
+  b.absent[0] = !(ok && kg > 0);
+  b.absent[1] = !ok;
+  b.absent[2] = !(ok && kg < N - 1);
+  b.off[1] = ok ? (uint32_t)kg * 3u * nn + nn + (uint32_t)row : nn;
+  b.off[0] = b.absent[0] ? b.off[1] : b.off[1] - nn;
+  b.off[2] = b.absent[2] ? b.off[1] : b.off[1] + nn;
+  return b;
+}
+
+// kLoadAny: chunk c1 (0 or 1) of the padded row, stateSize n <= NS known at run time
+// only (NS - n < 4).  Few instructions per element matter: the set-up is
+// straight-line code that runs once, at the rate at which it is fetched.  Set-up
+// (max_iter = 0) with one lane per row, against a select of offset and value per
+// element: FP32 n = 32 N = 16 8.9 us (16.9), n = 20 N = 20 7.2 (10.4), FP64 n = 13 N = 16
+// 7.3 (9.0).  The two chunks of a row differ by a lane offset that depends on the
+// pair of blocks they are in, of which a row has few (n = 24 N = 100 13.3, 14.6);
+// columns that may be padding are tested in scalar code.
+template <typename T, int NS, int CW>
+__device__ __forceinline__ void load_chunk_any(T (&dst)[CW], const T *__restrict__ A, int kg, int row, bool c1, int N,
+                                               bool active, int n) {
+  static_assert(3 * NS <= 2 * CW, "at most two chunks per row");
+  const BlockRow b = block_row(kg, row, N, active, n);
+#pragma unroll
+  for (int j = 0; j < CW; ++j) {
+    const int s0 = j / NS, k0 = j % NS;
+    if constexpr (CW >= 3 * NS) {  // one lane per row
+      T v = 0;
+      if (k0 < NS - 3 || k0 < n) v = load_at<T>(A, (uint32_t)(k0 * n), b.off[s0]);
+      dst[j] = b.absent[s0] ? (T)0 : v;
+    } else {
+      const int s1 = (CW + j) / NS, k1 = (CW + j) % NS;
+      const bool sure = k0 < NS - 3 && k1 < NS - 3 && s1 < 3;
+      if (sure) {
+        const int d = k1 - k0;  // the same for every column of the pair of blocks
+        const uint32_t lane = d >= 0 ? (c1 ? b.off[s1] + (uint32_t)(d * n) : b.off[s0])
+                                     : (c1 ? b.off[s1] : b.off[s0] + (uint32_t)(-d * n));
+        const T v = load_at<T>(A, (uint32_t)((d >= 0 ? k0 : k1) * n), lane);
+        dst[j] = (c1 ? b.absent[s1] : b.absent[s0]) ? (T)0 : v;
+      } else {
+        const bool v0 = k0 < n, v1 = s1 < 3 && k1 < n;  // uniform
+        T v = 0;
+        bool no = true;
+        if (v0 || v1) {
+          const int t1 = s1 < 3 ? s1 : 2;
+          const uint32_t lane = c1 ? (v1 ? b.off[t1] + (uint32_t)(k1 * n) : b.off[1])
+                                   : (v0 ? b.off[s0] + (uint32_t)(k0 * n) : b.off[1]);
+          v = load_at<T>(A, 0u, lane);
+          no = c1 ? (!v1 || b.absent[t1]) : (!v0 || b.absent[s0]);
+        }
+        dst[j] = no ? (T)0 : v;
+      }
+    }
+  }
+}
+
+// Rows `row` and `row` + 1 (when second) of block row kg, whole: adjacent in the
+// column-major blocks, so one 8-byte load serves both (4-byte aligned when n is
+// odd).  A lane with one row takes it from the upper half of the pair before it.
+// Set-up of n = 14 N = 64 11.4 us, of n = 8 N = 100 6.7 (row by row, with selects: 21.5
+// and 20.7).
+template <int NS>
+__device__ __forceinline__ void load_two_rows(float (&a)[3 * NS], float (&b)[3 * NS], const float *__restrict__ A,
+                                              int kg, int row, int N, bool active, bool second, int n) {
+  typedef float pair_t __attribute__((ext_vector_type(2), aligned(4)));
+  const bool last = active && !second;
+  const BlockRow r = block_row(kg, last ? row - 1 : row, N, active, n);
+#pragma unroll
+  for (int j = 0; j < 3 * NS; ++j) {
+    const int s = j / NS, k = j % NS;
+    pair_t v = {0.f, 0.f};
+    if (k < NS - 3 || k < n) v = load_at<pair_t>(A, (uint32_t)(k * n), r.off[s]);
+    a[j] = r.absent[s] ? 0.f : last ? v.y : v.x;
+    b[j] = (r.absent[s] || last) ? 0.f : v.y;
+  }
+}
+
 // Matrix chunk loads.  kLoadTables: branch-free, offsets from compile-time
 // tables (fewest instructions, but the table constants take VGPRs: FP32
 // 256-thread fixed-size instances, the single-solve layout); kLoadArith:
@@ -642,8 +737,7 @@ __host__ __device__ constexpr ChunkTables<NS, CW> chunk_tables() {
 // instances); kLoadRows: whole rows (one lane per row, CW = 3 nP), whose guards
 // are uniform over each block of n columns: one branch per block (the n = 28
 // one-lane-per-row instances).  kLoadAny: branch-free for a stateSize known at
-// run time only: the offsets are uniform per column and chunk, the masks combine
-// per-lane flags with uniform column tests.
+// run time only (load_chunk_any).
 template <typename T, int NS, int CW, int MODE = kLoadTables>
 __device__ __forceinline__ void load_chunk(T (&dst)[CW], const T *__restrict__ A, int kg, int row, int c, int N,
                                            bool active, int n_rt = 0) {
@@ -653,31 +747,7 @@ __device__ __forceinline__ void load_chunk(T (&dst)[CW], const T *__restrict__ A
   int cl = c, rl = row;
   asm volatile("" : "+v"(cl), "+v"(rl));
   if constexpr (MODE == kLoadAny) {
-    // one or two chunks per row: the block and the column within it of element j
-    // are constants of the chunk
-    static_assert(3 * nP <= 2 * CW, "at most two chunks per row");
-    const bool mid = active && kg >= 0 && kg < N;
-    const bool ok3[3] = {mid && kg > 0, mid, mid && kg < N - 1};
-    const uint32_t base = mid ? (uint32_t)kg * (uint32_t)(3 * n_rt * n_rt) + (uint32_t)rl : 0u;
-    const bool c1 = cl != 0;
-#pragma unroll
-    for (int j = 0; j < CW; ++j) {
-      const int s0 = j / nP, k0 = j % nP, s1 = (CW + j) / nP, k1 = (CW + j) % nP;
-      const bool v0 = s0 < 3 && k0 < n_rt, v1 = s1 < 3 && k1 < n_rt;  // uniform
-      const uint32_t o0 = v0 ? (uint32_t)((s0 * n_rt + k0) * n_rt) : 0u;
-      const uint32_t o1 = v1 ? (uint32_t)((s1 * n_rt + k1) * n_rt) : 0u;
-      bool ok;
-      uint32_t off;
-      if constexpr (CW >= 3 * nP) {  // one lane per row
-        ok = v0 && ok3[s0 < 3 ? s0 : 2];
-        off = o0;
-      } else {
-        ok = c1 ? (v1 && ok3[s1 < 3 ? s1 : 2]) : (v0 && ok3[s0 < 3 ? s0 : 2]);
-        off = c1 ? o1 : o0;
-      }
-      const T v = gptr(A)[ok ? base + off : 0u];
-      dst[j] = ok ? v : (T)0;
-    }
+    load_chunk_any<T, NS, CW>(dst, A, kg, rl, cl != 0, N, active, n_rt);
   } else if constexpr (MODE == kLoadRows) {
     static_assert(CW == 3 * nP, "whole-row loads");
     const bool rowok = active && kg >= 0 && kg < N;
@@ -762,16 +832,13 @@ __device__ __forceinline__ void load_row(T (&dst)[3 * NS], const T *__restrict__
     }
     return;
   }
-  // branch-free, as load_chunk
-  const bool rowok = active & (kg >= 0) & (kg < N);
-  const uint32_t base = rowok ? (uint32_t)kg * (uint32_t)(3 * n * n) + (uint32_t)rl : 0u;
-  const bool first = kg == 0, last = kg == N - 1;
+  // branch-free, as load_chunk_any
+  const BlockRow b = block_row(kg, rl, N, active, n);
 #pragma unroll
   for (int j = 0; j < 3 * n; ++j) {
-    const int seg = j / n;
-    const bool ok = rowok & !(first & (seg == 0)) & !(last & (seg == 2));
-    const T v = gptr(A)[ok ? base + (uint32_t)(j * n) : 0u];
-    dst[j] = ok ? v : (T)0;
+    const int s = j / n, k = j % n;
+    const T v = load_at<T>(A, (uint32_t)(k * n), b.off[s]);
+    dst[j] = b.absent[s] ? (T)0 : v;
   }
 }
 
@@ -1079,11 +1146,15 @@ __device__ __forceinline__ void reg_item(const KSys &d, uint32_t rank, T *lds) {
   // matrix chunks straight from HBM into registers
   T mM[CW], mS[CW];
   // branch-free loads for the fixed-size instances of n <= 14 (the single-solve
-  // layouts); the runtime-n and n = 28 instances keep the guarded form, whose
-  // fewer live masks leave their batches faster
+  // layouts), n = 28 on two lanes per row (set-up 9.2 us against 12.6 guarded, N = 64)
+  // and the instances for any size; the runtime-n and other n = 28 instances keep
+  // the guarded form, whose fewer live masks leave their batches faster
   constexpr bool kGuarded = !(BF && NS <= 14);
-  constexpr int kMode = R::RT ? kLoadAny : kGuarded ? (R::LPR == 1 && CW == 3 * nP ? kLoadRows : kLoadGuarded)
-                                 : (sizeof(T) == 4 && NT == 256) ? kLoadTables : kLoadArith;
+  constexpr int kMode = R::RT || (PRE && NS > 14 && R::LPR == 2)         ? kLoadAny
+                        : !kGuarded                                       ? (sizeof(T) == 4 && NT == 256) ? kLoadTables
+                                                                                                          : kLoadArith
+                        : R::LPR == 1 && CW == 3 * nP                     ? kLoadRows
+                                                                          : kLoadGuarded;
   // S first: loads complete in issue order, so the first product r = b - S x
   // (and the first exchange) can start while the Pinv chunks are in flight
   if constexpr (BC) {
@@ -1519,10 +1590,8 @@ __device__ __forceinline__ void two_rows_item(const KSys &d, float *lds) {
   rhs_at(lam0, xa, xb);
   rhs_at(fwd ? d.gamma : d.glambda, ba, bb);
   float sa[CW], sb[CW], pa[CW], pb[CW];
-  load_chunk<float, NS, CW, kLoadAny>(sa, static_cast<const float *>(d.S), kg, it.row, 0, N, it.act, n);
-  load_chunk<float, NS, CW, kLoadAny>(sb, static_cast<const float *>(d.S), kg, it.row + 1, 0, N, it.second, n);
-  load_chunk<float, NS, CW, kLoadAny>(pa, static_cast<const float *>(d.Pinv), kg, it.row, 0, N, it.act, n);
-  load_chunk<float, NS, CW, kLoadAny>(pb, static_cast<const float *>(d.Pinv), kg, it.row + 1, 0, N, it.second, n);
+  load_two_rows<NS>(sa, sb, static_cast<const float *>(d.S), kg, it.row, N, it.act, it.second, n);
+  load_two_rows<NS>(pa, pb, static_cast<const float *>(d.Pinv), kg, it.row, N, it.act, it.second, n);
   __syncthreads();
   it.put(fwd ? xv : lv, xa, xb);
   __syncthreads();

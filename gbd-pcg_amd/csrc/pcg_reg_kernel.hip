@@ -60,7 +60,7 @@ bool any_supported(uint32_t n, int nt, int set) {
     case kAnyWide: return n > 16 && n <= 32 && nt == 256;
     case kAnyAll: return n <= 32 && nt == 512;
     case kAnyRows: return n <= 16 && nt == 256;
-    case kAnyLong: return n <= 16 && nt == 512;
+    case kAnyLong: return n >= 2 && n <= 16 && nt == 512;
     default: return false;
   }
 }
