@@ -89,6 +89,11 @@ struct RegItem : StateSize<NS, (LP > 0)> {
   static constexpr int CW = BC ? 3 * NS : (int)reg_chunk(NS, LPR);           // columns per lane
   static constexpr int WPV = (int)(sizeof(T) / 4);
   static constexpr int NWAVES = NT / 64;
+  // Tiled rows (tile_dot): TL lanes share two rows, each with TW columns of every
+  // block of both; MW values per lane and matrix.
+  static constexpr bool TILED = !BC && !RT && NS == 28 && NT == 256;
+  static constexpr int TL = 2 * LPR, TW = TILED ? NS / TL : 1;
+  static constexpr int MW = TILED ? 6 * TW : CW;
 
   // geometry
   int N, G, rank, a, b, K, VL;
@@ -100,6 +105,7 @@ struct RegItem : StateSize<NS, (LP > 0)> {
   bool xcd_ok;  // the system allows XCD-local stores (KF_NOXCD clear)
   // lane roles
   int q, c, m, row, kg;
+  int i;  // tiled rows: number of the lane in its group
   bool act_u, act_w, owner, ghost;
   int gpos;
   // LDS
@@ -601,37 +607,6 @@ __device__ __forceinline__ T group_sum(T v) {
   return v;
 }
 
-// Loads this lane's chunk of row `row` of block row kg of a cbtd matrix
-// (padded row-major columns [c*CW, (c+1)*CW) of the n x 3nP block row).
-constexpr int kLoadTables = 0, kLoadArith = 1, kLoadGuarded = 2, kLoadRows = 3, kLoadAny = 4;
-
-// Per-chunk column tables of a block row (lane chunk c of CW padded columns):
-// the element offset of each column (0 for a padded column) and bit masks of
-// the valid columns, of those in the first block (S_{k,k-1}) and in the last
-// (S_{k,k+1}).
-template <int NS, int CW>
-struct ChunkTables {
-  uint32_t off[2][CW];
-  uint32_t valid[2], seg0[2], seg2[2];
-};
-template <int NS, int CW>
-__host__ __device__ constexpr ChunkTables<NS, CW> chunk_tables() {
-  constexpr int n = NS, nP = (int)padded_n(NS);
-  ChunkTables<NS, CW> t{};
-  for (int c = 0; c < 2; ++c) {
-    t.valid[c] = t.seg0[c] = t.seg2[c] = 0u;
-    for (int j = 0; j < CW; ++j) {
-      const int col = c * CW + j, seg = col / nP, cc = col - seg * nP;
-      const bool ok = seg < 3 && cc < n;
-      t.off[c][j] = ok ? (uint32_t)((seg * n + cc) * n) : 0u;
-      if (ok) t.valid[c] |= 1u << j;
-      if (ok && seg == 0) t.seg0[c] |= 1u << j;
-      if (ok && seg == 2) t.seg2[c] |= 1u << j;
-    }
-  }
-  return t;
-}
-
 // Element at a uniform element offset from A plus a per-lane one (32-bit byte
 // offsets against a scalar base: one scalar addition and one load).
 template <typename V, typename T>
@@ -660,8 +635,8 @@ __device__ __forceinline__ BlockRow block_row(int kg, int row, int N, bool activ
   return b;
 }
 
-// kLoadAny: chunk c1 (0 or 1) of the padded row, stateSize n <= NS known at run time
-// only (NS - n < 4).  Few instructions per element matter: the set-up is
+// Chunk c1 (0 or 1) of CW columns of a padded row (NS columns per block, stateSize
+// n <= NS, NS - n < 4, a constant or known at run time only).  Few instructions per element matter: the set-up is
 // straight-line code that runs once, at the rate at which it is fetched.  Set-up
 // (max_iter = 0) with one lane per row, against a select of offset and value per
 // element: FP32 n = 32 N = 16 8.9 us (16.9), n = 20 N = 20 7.2 (10.4), FP64 n = 13 N = 16
@@ -669,14 +644,21 @@ __device__ __forceinline__ BlockRow block_row(int kg, int row, int N, bool activ
 // pair of blocks they are in, of which a row has few (n = 24 N = 100 13.3, 14.6);
 // columns that may be padding are tested in scalar code.
 template <typename T, int NS, int CW>
-__device__ __forceinline__ void load_chunk_any(T (&dst)[CW], const T *__restrict__ A, int kg, int row, bool c1, int N,
+__device__ __forceinline__ void load_chunk(T (&dst)[CW], const T *__restrict__ A, int kg, int row, bool c1, int N,
                                                bool active, int n) {
   static_assert(3 * NS <= 2 * CW, "at most two chunks per row");
+  // opaque copy: keeps the lane offsets below from being hoisted out of the batched
+  // item loop (they would stay live, in registers, for the whole solve)
+  asm volatile("" : "+v"(row));
   const BlockRow b = block_row(kg, row, N, active, n);
 #pragma unroll
   for (int j = 0; j < CW; ++j) {
     const int s0 = j / NS, k0 = j % NS;
     if constexpr (CW >= 3 * NS) {  // one lane per row
+      if (s0 > 2) {
+        dst[j] = (T)0;
+        continue;
+      }
       T v = 0;
       if (k0 < NS - 3 || k0 < n) v = load_at<T>(A, (uint32_t)(k0 * n), b.off[s0]);
       dst[j] = b.absent[s0] ? (T)0 : v;
@@ -727,29 +709,17 @@ __device__ __forceinline__ void load_two_rows(float (&a)[3 * NS], float (&b)[3 *
   }
 }
 
-// Matrix chunk loads.  kLoadTables: branch-free, offsets from compile-time
-// tables (fewest instructions, but the table constants take VGPRs: FP32
-// 256-thread fixed-size instances, the single-solve layout); kLoadArith:
-// branch-free, offsets computed per element (other fixed sizes n <= 14);
-// kLoadGuarded: one guarded load per element (an exec-mask branch each, so the
-// loads issue slowly), kept where the branch-free forms' live masks cost more
-// than they save (the paired kernel's 128-VGPR allocation, the runtime-n
-// instances); kLoadRows: whole rows (one lane per row, CW = 3 nP), whose guards
-// are uniform over each block of n columns: one branch per block (the n = 28
-// one-lane-per-row instances).  kLoadAny: branch-free for a stateSize known at
-// run time only (load_chunk_any).
-template <typename T, int NS, int CW, int MODE = kLoadTables>
-__device__ __forceinline__ void load_chunk(T (&dst)[CW], const T *__restrict__ A, int kg, int row, int c, int N,
-                                           bool active, int n_rt = 0) {
+// The same in guarded loads, for the n = 28 instances of 512 threads, whose registers
+// leave no room for the masks and offsets above (their batches reload every item's
+// matrices: FP64 forward + adjoint of 32 systems of N = 512, no iterations, 405 us
+// against 426).  One lane per row: the guards are uniform over each block.
+template <typename T, int NS, int CW>
+__device__ __forceinline__ void load_guarded(T (&dst)[CW], const T *__restrict__ A, int kg, int row, int c, int N,
+                                             bool active) {
   constexpr int n = NS, nP = (int)padded_n(NS);
-  // opaque copies: keeps the per-lane offsets below from being hoisted out of the
-  // batched item loop (they would stay live, in registers, for the whole solve)
   int cl = c, rl = row;
   asm volatile("" : "+v"(cl), "+v"(rl));
-  if constexpr (MODE == kLoadAny) {
-    load_chunk_any<T, NS, CW>(dst, A, kg, rl, cl != 0, N, active, n_rt);
-  } else if constexpr (MODE == kLoadRows) {
-    static_assert(CW == 3 * nP, "whole-row loads");
+  if constexpr (CW == 3 * nP) {
     const bool rowok = active && kg >= 0 && kg < N;
 #pragma unroll
     for (int s3 = 0; s3 < 3; ++s3) {
@@ -762,7 +732,7 @@ __device__ __forceinline__ void load_chunk(T (&dst)[CW], const T *__restrict__ A
         for (int cc = 0; cc < nP; ++cc) dst[s3 * nP + cc] = (T)0;
       }
     }
-  } else if constexpr (MODE == kLoadGuarded) {
+  } else {
 #pragma unroll
     for (int j = 0; j < CW; ++j) {
       const int col = cl * CW + j;
@@ -772,44 +742,104 @@ __device__ __forceinline__ void load_chunk(T (&dst)[CW], const T *__restrict__ A
         v = gptr(A)[(size_t)kg * 3 * n * n + (size_t)(seg * n + cc) * n + rl];
       dst[j] = v;
     }
-  } else if constexpr (MODE == kLoadArith) {
-    // branch-free, offsets computed per element (no table registers)
-    const bool rowok = active & (kg >= 0) & (kg < N);
-    const uint32_t base = rowok ? (uint32_t)kg * (uint32_t)(3 * n * n) + (uint32_t)rl : 0u;
-    const bool first = kg == 0, last = kg == N - 1;
+  }
+}
+
+// A fixed size's chunk of either kind.
+template <typename T, int NS, int NT, int CW>
+__device__ __forceinline__ void load_fixed(T (&dst)[CW], const T *__restrict__ A, int kg, int row, int c, int N,
+                                           bool active) {
+  if constexpr (NS == 28 && NT == 512)
+    load_guarded<T, NS, CW>(dst, A, kg, row, c, N, active);
+  else
+    load_chunk<T, (int)padded_n(NS), CW>(dst, A, kg, row, c != 0, N, active, NS);
+}
+
+// Tiled rows.  A vector window read from LDS costs as many cycles as the bytes it
+// hands to the lanes, broadcast or not, and two matrix rows of a knot want the same
+// window: so the TL lanes that hold two rows (LPR each) do not take a row's columns
+// each, but TW columns of every block of both rows, and each reads half the window
+// that its own row would need.  Two partial sums per lane are then added up across
+// the lanes by DPP, one row to each half of the group.  Value (s TW + j) 2 + r of a
+// lane is row r, column j of its columns in block s.  For n = 28 at 256 threads (single
+// solves), per iteration: FP64 N = 100 3.45 -> 2.79 us, FP32 N = 64 1.73 -> 1.61; n = 6 to
+// 14 and the instances of 512 threads, which VALU issue bounds, gain nothing by it.
+
+// Columns j of this lane (number i of its group), block s, of rows r0 and r0 + 1 of
+// block row kg: adjacent in the column-major blocks, so one load serves both rows
+// (aligned to T only).  Branch-free as load_chunk: a scalar offset per column, a
+// lane offset per block.
+template <typename T, int NS, int TL, int TW>
+__device__ __forceinline__ void load_tile(T (&dst)[6 * TW], const T *__restrict__ A, int kg, int r0, int i, int N,
+                                          bool active) {
+  typedef T pair_t __attribute__((ext_vector_type(2), aligned(sizeof(T))));
+  constexpr int n = NS;
+  static_assert(n % TL == 0 && TW == n / TL, "tiles without padded columns");
+  int il = i;
+  asm volatile("" : "+v"(il));
+  const BlockRow b = block_row(kg, r0, N, active, n);
+  const uint32_t col0 = (uint32_t)(il * TW * n);
 #pragma unroll
-    for (int j = 0; j < CW; ++j) {
-      const int col = cl * CW + j;
-      const int seg = col / nP, cc = col - seg * nP;
-      const bool ok = rowok & (seg < 3) & (cc < n) & !(first & (seg == 0)) & !(last & (seg == 2));
-      const T v = gptr(A)[ok ? base + (uint32_t)((seg * n + cc) * n) : 0u];
-      dst[j] = ok ? v : (T)0;
+  for (int s = 0; s < 3; ++s) {
+#pragma unroll
+    for (int j = 0; j < TW; ++j) {
+      const pair_t v = load_at<pair_t>(A, (uint32_t)(j * n), b.off[s] + col0);
+      dst[(s * TW + j) * 2] = b.absent[s] ? (T)0 : v.x;
+      dst[(s * TW + j) * 2 + 1] = b.absent[s] ? (T)0 : v.y;
     }
+  }
+}
+
+// TW consecutive vector entries from LDS, in the widest reads their alignment
+// (a multiple of TW values from a 16-byte boundary) allows.
+template <typename T, int TW>
+__device__ __forceinline__ void read_window(const T *__restrict__ x, T (&o)[TW]) {
+  constexpr int V = (TW * (int)sizeof(T)) % 16 == 0 ? 16 / (int)sizeof(T) : (TW * (int)sizeof(T)) % 8 == 0 ? 8 / (int)sizeof(T) : 1;
+  typedef T vec_t __attribute__((ext_vector_type(V)));
+#pragma unroll
+  for (int j = 0; j < TW; j += V) {
+    const vec_t v = *reinterpret_cast<const vec_t *>(x + j);
+#pragma unroll
+    for (int k = 0; k < V; ++k) o[j + k] = v[k];
+  }
+}
+
+// A lane's partial sums of its two rows over its columns of the window at x (the
+// lane's first column; blocks nP apart): two accumulator chains per row.
+template <typename T, int TW, int nP>
+__device__ __forceinline__ void tile_dot(const T (&mat)[6 * TW], const T *__restrict__ x, T &ya, T &yb) {
+  T a0 = 0, a1 = 0, b0 = 0, b1 = 0;
+#pragma unroll
+  for (int s = 0; s < 3; ++s) {
+    T xs[TW];
+    read_window<T, TW>(x + s * nP, xs);
+#pragma unroll
+    for (int j = 0; j < TW; ++j) {
+      const int e = s * TW + j;
+      if (e % 2 == 0) {
+        a0 = fmaT(mat[2 * e], xs[j], a0);
+        b0 = fmaT(mat[2 * e + 1], xs[j], b0);
+      } else {
+        a1 = fmaT(mat[2 * e], xs[j], a1);
+        b1 = fmaT(mat[2 * e + 1], xs[j], b1);
+      }
+    }
+  }
+  ya = a0 + a1;
+  yb = b0 + b1;
+}
+
+// Adds a group's partial sums up: the lanes of its first half get row a's total, the
+// others row b's, the same bits in every lane of a row.
+template <int TL, typename T>
+__device__ __forceinline__ T tile_sum(T ya, T yb, int i) {
+  const bool upper = i >= TL / 2;
+  const T keep = upper ? yb : ya, send = upper ? ya : yb;
+  if constexpr (TL == 2) {
+    return keep + dpp<kDppQuadXor1>(send);
   } else {
-    // branch-free: every lane loads (an absent element from an in-bounds offset:
-    // row rl of column 0 of its block row, or offset 0 for a row outside the
-    // system) and a select zeroes what it must not hold, so the loads issue back
-    // to back instead of one exec-mask branch each.  Column offsets and the masks
-    // of valid / first-block / last-block columns come from compile-time tables of
-    // the (at most two) chunks; 32-bit offsets (3 n^2 N < 2^31 for every size the
-    // planner accepts).
-    static_assert(3 * nP <= 2 * CW && CW <= 32, "branch-free loads: two chunks of at most 32 columns");
-    constexpr ChunkTables<NS, CW> tab = chunk_tables<NS, CW>();
-    const bool rowok = active & (kg >= 0) & (kg < N);
-    // byte offsets in 32 bits: one VGPR offset per load against the uniform base
-    const uint32_t base = rowok ? ((uint32_t)kg * (uint32_t)(3 * n * n) + (uint32_t)rl) * (uint32_t)sizeof(T) : 0u;
-    const bool c1 = cl != 0;
-    uint32_t mask = c1 ? tab.valid[1] : tab.valid[0];
-    if (kg == 0) mask &= ~(c1 ? tab.seg0[1] : tab.seg0[0]);
-    if (kg == N - 1) mask &= ~(c1 ? tab.seg2[1] : tab.seg2[0]);
-    mask = rowok ? mask : 0u;
-    const auto *bytes = reinterpret_cast<const __attribute__((address_space(1))) unsigned char *>(gptr(A));
-#pragma unroll
-    for (int j = 0; j < CW; ++j) {
-      const uint32_t off = base + (c1 ? tab.off[1][j] : tab.off[0][j]) * (uint32_t)sizeof(T);
-      const T v = *reinterpret_cast<const __attribute__((address_space(1))) T *>(bytes + off);
-      dst[j] = ((mask >> j) & 1u) ? v : (T)0;
-    }
+    const T v = keep + dpp<kDppQuadXor2>(send);
+    return v + dpp<kDppQuadXor1>(v);
   }
 }
 
@@ -832,7 +862,7 @@ __device__ __forceinline__ void load_row(T (&dst)[3 * NS], const T *__restrict__
     }
     return;
   }
-  // branch-free, as load_chunk_any
+  // branch-free, as load_chunk
   const BlockRow b = block_row(kg, rl, N, active, n);
 #pragma unroll
   for (int j = 0; j < 3 * n; ++j) {
@@ -908,9 +938,10 @@ __device__ __forceinline__ bool finite_t(double v) { return __builtin_isfinite(v
 
 // One matvec row pass: this lane's row of a resident block row times the vector
 // window of knots m-1..m+1 (local knots m..m+2) of `vec`; 0 on inactive lanes.
+// chunk_mv: each lane holding columns of its own row; row_mv: as reg_item holds it.
 template <typename T, int NS, int NT, bool BC, int LP, bool ALONE, int CW>
-__device__ __forceinline__ T row_mv(const RegItem<T, NS, NT, BC, LP, ALONE> &it, const T (&mat)[CW], const T *vec,
-                                    bool act) {
+__device__ __forceinline__ T chunk_mv(const RegItem<T, NS, NT, BC, LP, ALONE> &it, const T (&mat)[CW], const T *vec,
+                                      bool act) {
   using R = RegItem<T, NS, NT, BC, LP, ALONE>;
   if constexpr (BC) {
     // every lane of the 16-lane row takes part in the broadcasts; lanes past the
@@ -922,6 +953,19 @@ __device__ __forceinline__ T row_mv(const RegItem<T, NS, NT, BC, LP, ALONE> &it,
   } else {
     T y = act ? chunk_dot<T, CW>(mat, vec + it.m * R::nP + it.c * CW) : (T)0;
     return group_sum<R::LPR>(y);
+  }
+}
+
+template <typename T, int NS, int NT, bool BC, int LP, bool ALONE, int MW>
+__device__ __forceinline__ T row_mv(const RegItem<T, NS, NT, BC, LP, ALONE> &it, const T (&mat)[MW], const T *vec,
+                                    bool act) {
+  using R = RegItem<T, NS, NT, BC, LP, ALONE>;
+  if constexpr (R::TILED) {
+    T ya = 0, yb = 0;
+    if (act) tile_dot<T, R::TW, R::nP>(mat, vec + it.m * R::nP + it.i * R::TW, ya, yb);
+    return tile_sum<R::TL>(ya, yb, it.i);
+  } else {
+    return chunk_mv(it, mat, vec, act);
   }
 }
 
@@ -960,8 +1004,8 @@ __device__ __forceinline__ void pinv_mv2(const RegItem<T, NS, NT, BC> &it, const
     ya = group_sum<R::LPR>(a);
     yb = group_sum<R::LPR>(b);
   } else {
-    ya = row_mv(it, mM, va, it.act_u);
-    yb = row_mv(it, mM, vb, it.act_u);
+    ya = chunk_mv(it, mM, va, it.act_u);
+    yb = chunk_mv(it, mM, vb, it.act_u);
   }
 }
 
@@ -977,7 +1021,7 @@ __device__ __forceinline__ T s_mv1(const RegItem<T, NS, NT, BC> &it, const T (&m
     if (it.act_w) a = chunk_dot_lds_d<R::CW, SL>(slds, tid - R::LPR * NS, v + it.m * R::nP + it.c * R::CW);
     return group_sum<R::LPR>(a);
   } else {
-    return row_mv(it, mS, v, it.act_w);
+    return chunk_mv(it, mS, v, it.act_w);
   }
 }
 
@@ -994,8 +1038,8 @@ __device__ __forceinline__ void s_mv2(const RegItem<T, NS, NT, BC> &it, const T 
     ya = group_sum<R::LPR>(a);
     yb = group_sum<R::LPR>(b);
   } else {
-    ya = row_mv(it, mS, va, it.act_w);
-    yb = row_mv(it, mS, vb, it.act_w);
+    ya = chunk_mv(it, mS, va, it.act_w);
+    yb = chunk_mv(it, mS, vb, it.act_w);
   }
 }
 
@@ -1072,6 +1116,7 @@ __device__ __forceinline__ void reg_item(const KSys &d, uint32_t rank, T *lds) {
   const int t = opaque_tid();
   it.q = t / R::LPR;
   it.c = t % R::LPR;
+  it.i = t & (R::TL - 1);
   if constexpr (BC) {
     it.m = t >> 4;
     it.row = t & 15;
@@ -1144,25 +1189,25 @@ __device__ __forceinline__ void reg_item(const KSys &d, uint32_t rank, T *lds) {
   }
 
   // matrix chunks straight from HBM into registers
-  T mM[CW], mS[CW];
-  // branch-free loads for the fixed-size instances of n <= 14 (the single-solve
-  // layouts), n = 28 on two lanes per row (set-up 9.2 us against 12.6 guarded, N = 64)
-  // and the instances for any size; the runtime-n and other n = 28 instances keep
-  // the guarded form, whose fewer live masks leave their batches faster
+  T mM[R::MW], mS[R::MW];
+  // row broadcast: branch-free loads on the single-solve instances; guarded ones
+  // leave fewer live masks, which the paired and runtime-n instances need more
   constexpr bool kGuarded = !(BF && NS <= 14);
-  constexpr int kMode = R::RT || (PRE && NS > 14 && R::LPR == 2)         ? kLoadAny
-                        : !kGuarded                                       ? (sizeof(T) == 4 && NT == 256) ? kLoadTables
-                                                                                                          : kLoadArith
-                        : R::LPR == 1 && CW == 3 * nP                     ? kLoadRows
-                                                                          : kLoadGuarded;
   // S first: loads complete in issue order, so the first product r = b - S x
   // (and the first exchange) can start while the Pinv chunks are in flight
   if constexpr (BC) {
     load_row<T, NS, kGuarded>(mS, static_cast<const T *>(d.S), kg, row, it.N, it.act_w);
     load_row<T, NS, kGuarded>(mM, static_cast<const T *>(d.Pinv), kg, row, it.N, it.act_u);
+  } else if constexpr (R::RT) {
+    load_chunk<T, nP, CW>(mS, static_cast<const T *>(d.S), kg, row, c != 0, it.N, it.act_w, n);
+    load_chunk<T, nP, CW>(mM, static_cast<const T *>(d.Pinv), kg, row, c != 0, it.N, it.act_u, n);
+  } else if constexpr (R::TILED) {
+    const int r0 = row - it.i / R::LPR;
+    load_tile<T, NS, R::TL, R::TW>(mS, static_cast<const T *>(d.S), kg, r0, it.i, it.N, it.act_w);
+    load_tile<T, NS, R::TL, R::TW>(mM, static_cast<const T *>(d.Pinv), kg, r0, it.i, it.N, it.act_u);
   } else {
-    load_chunk<T, NS, CW, kMode>(mS, static_cast<const T *>(d.S), kg, row, c, it.N, it.act_w, n);
-    load_chunk<T, NS, CW, kMode>(mM, static_cast<const T *>(d.Pinv), kg, row, c, it.N, it.act_u, n);
+    load_fixed<T, NS, NT, CW>(mS, static_cast<const T *>(d.S), kg, row, c, it.N, it.act_w);
+    load_fixed<T, NS, NT, CW>(mM, static_cast<const T *>(d.Pinv), kg, row, c, it.N, it.act_u);
   }
   __syncthreads();
   it.base = ALONE ? 0u : (uint32_t)it.ctl[1];
@@ -1575,7 +1620,7 @@ __device__ __forceinline__ void two_rows_item(const KSys &d, float *lds) {
     it.act = k < N && it.row < n;
     it.second = it.act && it.row + 1 < n;
   }
-  const int kg = it.m - 1, own = (it.m + 1) * nP + it.row;
+  const int kg = it.m - 1;
   const bool fwd = (d.flags & KF_FWD) != 0, adj = (d.flags & KF_ADJ) != 0, rel = (d.flags & KF_REL) != 0;
   for (int i = opaque_tid(); i < total; i += stride) lds[i] = 0.f;
 
@@ -1803,6 +1848,7 @@ __device__ __forceinline__ void reg_item_pair(const KSys &d, uint32_t rank, T *l
   const int t = opaque_tid();
   it.q = t / R::LPR;
   it.c = t % R::LPR;
+  it.i = t & (R::TL - 1);
   if constexpr (BC) {
     it.m = t >> 4;
     it.row = t & 15;
@@ -1880,7 +1926,7 @@ __device__ __forceinline__ void reg_item_pair(const KSys &d, uint32_t rank, T *l
     // lane only), then its Pinv chunk into registers
     {
       T tmp[CW];
-      load_chunk<T, NS, CW, kLoadGuarded>(tmp, static_cast<const T *>(d.S), kg, row, c, it.N, it.act_w);
+      load_fixed<T, NS, NT, CW>(tmp, static_cast<const T *>(d.S), kg, row, c, it.N, it.act_w);
       if (it.act_w) {
         const int si = t - R::LPR * n;
 #pragma unroll
@@ -1888,21 +1934,20 @@ __device__ __forceinline__ void reg_item_pair(const KSys &d, uint32_t rank, T *l
           *reinterpret_cast<double2 *>(slds + ((size_t)(j / 2) * SL + si) * 2) = make_double2(tmp[j], tmp[j + 1]);
       }
     }
-    load_chunk<T, NS, CW, kLoadGuarded>(mM, static_cast<const T *>(d.Pinv), kg, row, c, it.N, it.act_u);
+    load_fixed<T, NS, NT, CW>(mM, static_cast<const T *>(d.Pinv), kg, row, c, it.N, it.act_u);
   } else if constexpr (!PLDS) {
-    constexpr int kPairLoad = R::LPR == 1 && CW == 3 * nP ? kLoadRows : kLoadGuarded;
-    load_chunk<T, NS, CW, kPairLoad>(mM, static_cast<const T *>(d.Pinv), kg, row, c, it.N, it.act_u);
-    load_chunk<T, NS, CW, kPairLoad>(mS, static_cast<const T *>(d.S), kg, row, c, it.N, it.act_w);
+    load_fixed<T, NS, NT, CW>(mM, static_cast<const T *>(d.Pinv), kg, row, c, it.N, it.act_u);
+    load_fixed<T, NS, NT, CW>(mS, static_cast<const T *>(d.S), kg, row, c, it.N, it.act_w);
   } else {
     // this lane's Pinv chunk through registers into its LDS slots (read back by
     // this lane only: no barrier needed between the store and the reads)
     T tmp[CW];
-    load_chunk<T, NS, CW, kLoadGuarded>(tmp, static_cast<const T *>(d.Pinv), kg, row, c, it.N, it.act_u);
+    load_fixed<T, NS, NT, CW>(tmp, static_cast<const T *>(d.Pinv), kg, row, c, it.N, it.act_u);
 #pragma unroll
     for (int j = 0; j < CW; j += 4)
       *reinterpret_cast<float4 *>(plds + ((size_t)(j / 4) * NT + t) * 4) = make_float4(tmp[j], tmp[j + 1], tmp[j + 2],
                                                                                         tmp[j + 3]);
-    load_chunk<T, NS, CW, kLoadGuarded>(mS, static_cast<const T *>(d.S), kg, row, c, it.N, it.act_w);
+    load_fixed<T, NS, NT, CW>(mS, static_cast<const T *>(d.S), kg, row, c, it.N, it.act_w);
   }
   __syncthreads();
   it.base = (uint32_t)it.ctl[1];
@@ -1924,7 +1969,7 @@ __device__ __forceinline__ void reg_item_pair(const KSys &d, uint32_t rank, T *l
   if constexpr (SLDS)
     rA_i = bA - s_mv1<SLDS, SL>(it, mS, slds, it.xv, t);
   else
-    rA_i = bA - row_mv(it, mS, it.xv, it.act_w);
+    rA_i = bA - chunk_mv(it, mS, it.xv, it.act_w);
   T rB_i = bB;
   if (it.owner) {
     rA[own_pos] = rA_i;
@@ -1955,8 +2000,8 @@ __device__ __forceinline__ void reg_item_pair(const KSys &d, uint32_t rank, T *l
     if constexpr (PLDS) {
       pinv_mv2<PLDS>(it, mM, plds, rA, rB, t, uA_i, uB_i);
     } else {
-      uA_i = row_mv(it, mM, rA, it.act_u);
-      uB_i = row_mv(it, mM, rB, it.act_u);
+      uA_i = chunk_mv(it, mM, rA, it.act_u);
+      uB_i = chunk_mv(it, mM, rB, it.act_u);
     }
     if (it.act_u && c == 0) {
       uA[(m + 1) * nP + row] = uA_i;
@@ -1966,8 +2011,8 @@ __device__ __forceinline__ void reg_item_pair(const KSys &d, uint32_t rank, T *l
     if constexpr (SLDS) {
       s_mv2<SLDS, SL>(it, mS, slds, uA, uB, t, wA_i, wB_i);
     } else {
-      wA_i = row_mv(it, mS, uA, it.act_w);
-      wB_i = row_mv(it, mS, uB, it.act_w);
+      wA_i = chunk_mv(it, mS, uA, it.act_w);
+      wB_i = chunk_mv(it, mS, uB, it.act_w);
     }
     it.publish_edge(wA_i, 2);
     it.publish_edge(wB_i, 2, VB);
@@ -2082,8 +2127,8 @@ __device__ __forceinline__ void reg_item_pair(const KSys &d, uint32_t rank, T *l
     if constexpr (PLDS) {
       pinv_mv2<PLDS>(it, mM, plds, rA, rB, t, uA_i, uB_i);
     } else {
-      uA_i = row_mv(it, mM, rA, it.act_u);
-      uB_i = row_mv(it, mM, rB, it.act_u);
+      uA_i = chunk_mv(it, mM, rA, it.act_u);
+      uB_i = chunk_mv(it, mM, rB, it.act_u);
     }
     if (it.act_u && c == 0) {
       uA[(m + 1) * nP + row] = uA_i;
@@ -2093,8 +2138,8 @@ __device__ __forceinline__ void reg_item_pair(const KSys &d, uint32_t rank, T *l
     if constexpr (SLDS) {
       s_mv2<SLDS, SL>(it, mS, slds, uA, uB, t, wA_i, wB_i);
     } else {
-      wA_i = row_mv(it, mS, uA, it.act_w);
-      wB_i = row_mv(it, mS, uB, it.act_w);
+      wA_i = chunk_mv(it, mS, uA, it.act_w);
+      wB_i = chunk_mv(it, mS, uB, it.act_w);
     }
     // both edge blocks every exchange (a stopped side's are stale and unused):
     // the neighbours' gather waits for every slot of the current epoch
