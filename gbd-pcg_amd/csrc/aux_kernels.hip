@@ -197,13 +197,16 @@ __global__ void __launch_bounds__(kAuxThreads) precond_kernel(const T *__restric
 
 template <typename T>
 __device__ __forceinline__ T lane_max(T v) {  // over the wave; v >= 0 or -1 (excluded)
-  v = __builtin_fmax(v, dpp<kDppRowShr1>(v));
-  v = __builtin_fmax(v, dpp<kDppRowShr2>(v));
-  v = __builtin_fmax(v, dpp<kDppRowShr4>(v));
-  v = __builtin_fmax(v, dpp<kDppRowShr8>(v));
-  v = __builtin_fmax(v, dpp<kDppRowBcast15, 0xa>(v));
-  v = __builtin_fmax(v, dpp<kDppRowBcast31, 0xc>(v));
-  return read_lane63(v);
+  T w = v;
+  swap_lanes<32>(v, w);
+  v = w = __builtin_fmax(v, w);
+  swap_lanes<16>(v, w);
+  v = __builtin_fmax(v, w);
+  v = __builtin_fmax(v, dpp<kDppQuadXor1>(v));
+  v = __builtin_fmax(v, dpp<kDppQuadXor2>(v));
+  v = __builtin_fmax(v, dpp<kDppRowRor4>(v));
+  v = __builtin_fmax(v, dpp<kDppRowRor8>(v));
+  return read_lane(v, 0);
 }
 
 template <typename T>

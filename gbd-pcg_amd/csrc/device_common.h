@@ -153,34 +153,62 @@ __device__ __forceinline__ uint32_t payload_word(T v, int q) {
 
 // Cross-lane moves use DPP (a VALU operand modifier, a few cycles) rather than
 // __shfl_xor, which lowers to ds_bpermute and costs an LDS round trip per step.
-// GFX9 DPP controls:
+// Every control used has a source lane for each lane: there is no previous value to
+// set up, and FP32 additions take the move as their operand.  GFX9 DPP controls:
 constexpr int kDppQuadXor1 = 0xB1;  // quad_perm [1,0,3,2]
 constexpr int kDppQuadXor2 = 0x4E;  // quad_perm [2,3,0,1]
-constexpr int kDppRowShr1 = 0x111, kDppRowShr2 = 0x112, kDppRowShr4 = 0x114, kDppRowShr8 = 0x118;
-constexpr int kDppRowBcast15 = 0x142, kDppRowBcast31 = 0x143;
+constexpr int kDppRowRor4 = 0x124, kDppRowRor8 = 0x128;  // rotations of rows of 16 lanes
 
-// Value of `v` from the lane selected by CTRL; 0 where the source lane does not
-// exist or the row is masked off.
-template <int CTRL, int ROW_MASK = 0xf>
+// Value of `v` from the lane selected by CTRL.
+template <int CTRL>
 __device__ __forceinline__ float dpp(float v) {
-  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, ROW_MASK, 0xf, false));
+  return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), CTRL, 0xf, 0xf, true));
 }
-template <int CTRL, int ROW_MASK = 0xf>
+template <int CTRL>
 __device__ __forceinline__ double dpp(double v) {
   const uint64_t b = (uint64_t)__double_as_longlong(v);
-  const int lo = __builtin_amdgcn_update_dpp(0, (int)(uint32_t)b, CTRL, ROW_MASK, 0xf, false);
-  const int hi = __builtin_amdgcn_update_dpp(0, (int)(uint32_t)(b >> 32), CTRL, ROW_MASK, 0xf, false);
+  const int lo = __builtin_amdgcn_mov_dpp((int)(uint32_t)b, CTRL, 0xf, 0xf, true);
+  const int hi = __builtin_amdgcn_mov_dpp((int)(uint32_t)(b >> 32), CTRL, 0xf, 0xf, true);
   return __longlong_as_double((long long)(((uint64_t)(uint32_t)hi << 32) | (uint32_t)lo));
 }
 
-__device__ __forceinline__ float read_lane63(float v) {
-  return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 63));
+// Two values exchanged across halves of the wave (W 32: the upper half of a with
+// the lower of b) or neighbouring rows of 16 lanes (W 16: a's odd rows with b's
+// even ones).  Afterwards a + b holds, in the lower half (in the even rows), the
+// sums of a's halves (rows) and in the others those of b: two values folded into
+// one by one instruction per 32 bits and an addition.
+template <int W>
+__device__ __forceinline__ void swap_lanes(uint32_t &a, uint32_t &b) {
+  if constexpr (W == 32) {
+    const auto r = __builtin_amdgcn_permlane32_swap(a, b, false, false);
+    a = r[0];
+    b = r[1];
+  } else {
+    const auto r = __builtin_amdgcn_permlane16_swap(a, b, false, false);
+    a = r[0];
+    b = r[1];
+  }
 }
-__device__ __forceinline__ double read_lane63(double v) {
-  const uint64_t b = (uint64_t)__double_as_longlong(v);
-  const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)b, 63);
-  const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(b >> 32), 63);
-  return __longlong_as_double((long long)(((uint64_t)hi << 32) | lo));
+template <int W>
+__device__ __forceinline__ void swap_lanes(float &a, float &b) {
+  uint32_t x = __float_as_uint(a), y = __float_as_uint(b);
+  swap_lanes<W>(x, y);
+  a = __uint_as_float(x);
+  b = __uint_as_float(y);
+}
+template <int W>
+__device__ __forceinline__ void swap_lanes(double &a, double &b) {
+  const uint64_t u = (uint64_t)__double_as_longlong(a), v = (uint64_t)__double_as_longlong(b);
+  uint32_t xl = (uint32_t)u, xh = (uint32_t)(u >> 32), yl = (uint32_t)v, yh = (uint32_t)(v >> 32);
+  swap_lanes<W>(xl, yl);
+  swap_lanes<W>(xh, yh);
+  a = __longlong_as_double((long long)(((uint64_t)xh << 32) | xl));
+  b = __longlong_as_double((long long)(((uint64_t)yh << 32) | yl));
+}
+template <int W, typename T>
+__device__ __forceinline__ T fold(T a, T b) {
+  swap_lanes<W>(a, b);
+  return a + b;
 }
 
 // Value of lane l (a constant), uniform.
@@ -194,45 +222,61 @@ __device__ __forceinline__ double read_lane(double v, int l) {
   return __longlong_as_double((long long)(((uint64_t)hi << 32) | lo));
 }
 
-// Sum over the 64 lanes of a wave (all lanes active): inclusive scan inside each
-// row of 16 lanes, then the row totals are folded into lane 63, which is
-// broadcast.  A fixed tree: identical inputs give identical bits in every wave.
+// Sums over each row of 16 lanes, in all of them (not the same bits in each: take
+// the row's first lane).
 template <typename T>
-__device__ __forceinline__ T wave_sum(T v) {
-  v += dpp<kDppRowShr1>(v);
-  v += dpp<kDppRowShr2>(v);
-  v += dpp<kDppRowShr4>(v);
-  v += dpp<kDppRowShr8>(v);
-  v += dpp<kDppRowBcast15, 0xa>(v);
-  v += dpp<kDppRowBcast31, 0xc>(v);
-  return read_lane63(v);
+__device__ __forceinline__ T row_sum(T v) {
+  v += dpp<kDppQuadXor1>(v);
+  v += dpp<kDppQuadXor2>(v);
+  v += dpp<kDppRowRor4>(v);
+  v += dpp<kDppRowRor8>(v);
+  return v;
 }
 
-// Three independent wave sums with their DPP steps interleaved (a DPP read of a
-// value written by the previous VALU op must wait; three chains hide that).
+// Three sums over the 64 lanes of a wave (all lanes active): sum l in lane 16 l.  A
+// fixed tree: identical inputs give identical bits in every wave.  The iteration of
+// FP64 systems of n = 28 is bound by VALU issue, a fifth of which six separate scans
+// took (three instructions per 32 bits and step); folded, six sums take 39
+// instructions instead of 276, three in FP32 11 instead of 57.
+template <typename T>
+__device__ __forceinline__ T wave_sums(T s0, T s1, T s2) {
+  return row_sum(fold<16>(fold<32>(s0, s2), fold<32>(s1, s1)));
+}
+
+// Six such sums: sums 0..3 in lanes 16 l, sum 4 in lane 1, sum 5 in lane 33.
+template <typename T>
+__device__ __forceinline__ T wave_sums(T s0, T s1, T s2, T s3, T s4, T s5) {
+  const T a = fold<16>(fold<32>(s0, s2), fold<32>(s1, s3));
+  const T h = fold<32>(s4, s5), b = fold<16>(h, h);
+  const bool odd = (threadIdx.x & 1) != 0;  // even lanes go on with a, odd ones with b
+  T v = (odd ? b : a) + dpp<kDppQuadXor1>(odd ? a : b);
+  v += dpp<kDppQuadXor2>(v);
+  v += dpp<kDppRowRor4>(v);
+  v += dpp<kDppRowRor8>(v);
+  return v;
+}
+// Index of the sum that this lane holds after wave_sums of COUNT values, or -1.
+template <int COUNT>
+__device__ __forceinline__ int wave_sums_slot() {
+  const int l = (int)threadIdx.x & 63;
+  if constexpr (COUNT == 3) return (l & 15) == 0 && l < 48 ? l >> 4 : -1;
+  return (l & 15) == 0 ? l >> 4 : (l & 31) == 1 ? 4 + (l >> 5) : -1;
+}
+
+// Sum over the 64 lanes of a wave (all lanes active), in every lane.
+template <typename T>
+__device__ __forceinline__ T wave_sum(T v) {
+  v = fold<32>(v, v);
+  return read_lane(row_sum(fold<16>(v, v)), 0);
+}
+
+// Three such sums.
 template <typename T>
 __device__ __forceinline__ void wave_sum3(T &a, T &b, T &c) {
-  a += dpp<kDppRowShr1>(a);
-  b += dpp<kDppRowShr1>(b);
-  c += dpp<kDppRowShr1>(c);
-  a += dpp<kDppRowShr2>(a);
-  b += dpp<kDppRowShr2>(b);
-  c += dpp<kDppRowShr2>(c);
-  a += dpp<kDppRowShr4>(a);
-  b += dpp<kDppRowShr4>(b);
-  c += dpp<kDppRowShr4>(c);
-  a += dpp<kDppRowShr8>(a);
-  b += dpp<kDppRowShr8>(b);
-  c += dpp<kDppRowShr8>(c);
-  a += dpp<kDppRowBcast15, 0xa>(a);
-  b += dpp<kDppRowBcast15, 0xa>(b);
-  c += dpp<kDppRowBcast15, 0xa>(c);
-  a += dpp<kDppRowBcast31, 0xc>(a);
-  b += dpp<kDppRowBcast31, 0xc>(b);
-  c += dpp<kDppRowBcast31, 0xc>(c);
-  a = read_lane63(a);
-  b = read_lane63(b);
-  c = read_lane63(c);
+  const T v = wave_sums(a, b, c);
+  a = read_lane(v, 0);
+  b = read_lane(v, 16);
+  c = read_lane(v, 32);
 }
 
 // Sum over each aligned group of 4 lanes; all 4 lanes get the same bits.

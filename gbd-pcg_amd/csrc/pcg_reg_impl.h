@@ -173,19 +173,15 @@ struct RegItem : StateSize<NS, (LP > 0)> {
   // share one XCD: G * sum(x^2) == sum(x)^2 exactly when all x are equal.
   // ALONE: the waves' sums only, which only_totals adds up.
   __device__ __forceinline__ void reduce_publish(T s0, T s1, T s2, bool placement = false) {
-    wave_sum3(s0, s1, s2);
+    const T sums = wave_sums(s0, s1, s2);
     if constexpr (ALONE && NWAVES == 1) {
-      only[0] = s0;
-      only[1] = s1;
-      only[2] = s2;
+      only[0] = read_lane(sums, 0);
+      only[1] = read_lane(sums, 16);
+      only[2] = read_lane(sums, 32);
       return;
     }
-    const int w = threadIdx.x >> 6;
-    if ((threadIdx.x & 63) == 0) {
-      wsum[w * 3 + 0] = s0;
-      wsum[w * 3 + 1] = s1;
-      wsum[w * 3 + 2] = s2;
-    }
+    const int slot = wave_sums_slot<3>();
+    if (slot >= 0) wsum[(threadIdx.x >> 6) * 3 + slot] = sums;
     if constexpr (ALONE) return;
     __syncthreads();
     // lanes 0..2 of wave 0: scalar l summed over the waves in order, published
@@ -321,12 +317,9 @@ struct RegItem : StateSize<NS, (LP > 0)> {
       acc1 += word_value(w2, 1);
       acc2 += word_value(w2, 2);
     }
-    wave_sum3(acc0, acc1, acc2);
-    if (t == 0) {
-      tot[0] = acc0;
-      tot[1] = acc1;
-      tot[2] = acc2;
-    }
+    const T sums = wave_sums(acc0, acc1, acc2);
+    const int slot = wave_sums_slot<3>();
+    if (slot >= 0) tot[slot] = sums;
     return ok;
   }
 
@@ -368,12 +361,9 @@ struct RegItem : StateSize<NS, (LP > 0)> {
         acc1 += word_value(wv_, 1);
         acc2 += word_value(wv_, 2);
       }
-      wave_sum3(acc0, acc1, acc2);
-      if (t == 0) {
-        tot[0] = acc0;
-        tot[1] = acc1;
-        tot[2] = acc2;
-      }
+      const T sums = wave_sums(acc0, acc1, acc2);
+      const int slot = wave_sums_slot<3>();
+      if (slot >= 0) tot[slot] = sums;
     } else {
       const int en = edge * n * WPV;
       const int nleft = rank > 0 ? en : 0;
@@ -405,17 +395,9 @@ struct RegItem : StateSize<NS, (LP > 0)> {
   // wsum holding 6 per wave.  Lanes 0..5 publish.  placement as in
   // reduce_publish, for scalars 1 and 2.
   __device__ __forceinline__ void reduce_publish6(T s0, T s1, T s2, T s3, T s4, T s5, bool placement = false) {
-    wave_sum3(s0, s1, s2);
-    wave_sum3(s3, s4, s5);
-    const int w = threadIdx.x >> 6;
-    if ((threadIdx.x & 63) == 0) {
-      wsum[w * 6 + 0] = s0;
-      wsum[w * 6 + 1] = s1;
-      wsum[w * 6 + 2] = s2;
-      wsum[w * 6 + 3] = s3;
-      wsum[w * 6 + 4] = s4;
-      wsum[w * 6 + 5] = s5;
-    }
+    const T sums = wave_sums(s0, s1, s2, s3, s4, s5);
+    const int slot = wave_sums_slot<6>();
+    if (slot >= 0) wsum[(threadIdx.x >> 6) * 6 + slot] = sums;
     __syncthreads();
     const int l = threadIdx.x;
     if (l >= 6) return;
@@ -460,12 +442,9 @@ struct RegItem : StateSize<NS, (LP > 0)> {
 #pragma unroll
         for (int l = 0; l < 6; ++l) acc[l] += word_value(wv_, l);
       }
-      wave_sum3(acc[0], acc[1], acc[2]);
-      wave_sum3(acc[3], acc[4], acc[5]);
-      if (t == 0) {
-#pragma unroll
-        for (int l = 0; l < 6; ++l) tot[l] = acc[l];
-      }
+      const T sums = wave_sums(acc[0], acc[1], acc[2], acc[3], acc[4], acc[5]);
+      const int slot = wave_sums_slot<6>();
+      if (slot >= 0) tot[slot] = sums;
     } else {
       const int en = edge * n * WPV;
       const int nleft = rank > 0 ? en : 0;
@@ -1247,7 +1226,7 @@ __device__ __forceinline__ void reg_item(const KSys &d, uint32_t rank, T *lds) {
     T r_i;
     {
       T y = row_mv(it, mS, it.xv, it.act_w);
-      r_i = b_i - y;
+      r_i = it.owner ? b_i - y : (T)0;  // zero on the other lanes for good: only w'u needs a select
     }
     if (it.owner) it.rv[own_pos] = r_i;
     it.publish_edge(r_i, 2);
@@ -1277,8 +1256,8 @@ __device__ __forceinline__ void reg_item(const KSys &d, uint32_t rank, T *lds) {
         it.settle();
         p_i = z_i;
         if (it.act_u && c == 0) it.uv[(m + 1) * nP + row] = p_i;  // uv holds p
-        const T rz = it.owner ? r_i * z_i : (T)0;
-        const T r2 = it.owner ? r_i * r_i : (T)0;
+        const T rz = r_i * z_i;
+        const T r2 = r_i * r_i;
         it.reduce_publish(rz, (T)0, r2);
         T unused;
         if (!it.gather(it.wv, 0, eta, unused, rr)) {
@@ -1342,8 +1321,8 @@ __device__ __forceinline__ void reg_item(const KSys &d, uint32_t rank, T *lds) {
           {
             z_i = row_mv(it, mM, it.rv, it.act_u);
           }
-          const T rz = it.owner ? r_i * z_i : (T)0;
-          const T r2 = it.owner ? r_i * r_i : (T)0;
+          const T rz = r_i * z_i;
+          const T r2 = r_i * r_i;
           it.reduce_publish(rz, (T)0, r2);
           T eta_new, u3;
           if (!it.gather(it.wv, 0, eta_new, u3, rr)) {
@@ -1382,9 +1361,9 @@ __device__ __forceinline__ void reg_item(const KSys &d, uint32_t rank, T *lds) {
         __syncthreads();
         w_i = row_mv(it, mS, it.uv, it.act_w);
         it.publish_edge(w_i, 2);
-        const T rz = it.owner ? r_i * u_i : (T)0;
+        const T rz = r_i * u_i;
         const T wu = it.owner ? w_i * u_i : (T)0;
-        const T r2 = it.owner ? r_i * r_i : (T)0;
+        const T r2 = r_i * r_i;
         it.reduce_publish(rz, wu, r2);
         T delta;
         if (!it.gather(it.wv, 2, eta, delta, rr)) {
@@ -1436,9 +1415,9 @@ __device__ __forceinline__ void reg_item(const KSys &d, uint32_t rank, T *lds) {
           __syncthreads();
           w_i = row_mv(it, mS, it.uv, it.act_w);
           it.publish_edge(w_i, 2);
-          const T rz = it.owner ? r_i * u_i : (T)0;
+          const T rz = r_i * u_i;
           const T wu = it.owner ? w_i * u_i : (T)0;
-          const T r2 = it.owner ? r_i * r_i : (T)0;
+          const T r2 = r_i * r_i;
           it.reduce_publish(rz, wu, r2);
           T eta_new, delta_new;
           if (!it.gather(it.wv, 2, eta_new, delta_new, rr)) {
@@ -1584,13 +1563,9 @@ struct TwoRows {
 
   // Workgroup totals in every wave; the caller has a barrier between two calls.
   __device__ __forceinline__ void totals(float &s0, float &s1, float &s2) const {
-    wave_sum3(s0, s1, s2);
-    const int w = threadIdx.x >> 6;
-    if ((threadIdx.x & 63) == 0) {
-      wsum[w * 3 + 0] = s0;
-      wsum[w * 3 + 1] = s1;
-      wsum[w * 3 + 2] = s2;
-    }
+    const float sums = wave_sums(s0, s1, s2);
+    const int slot = wave_sums_slot<3>();
+    if (slot >= 0) wsum[(threadIdx.x >> 6) * 3 + slot] = sums;
     __syncthreads();
     const int l = (int)threadIdx.x & 3;
     const float v = waves_total<NWAVES, 3>(wsum, l < 3 ? l : 0);
@@ -1970,6 +1945,7 @@ __device__ __forceinline__ void reg_item_pair(const KSys &d, uint32_t rank, T *l
     rA_i = bA - s_mv1<SLDS, SL>(it, mS, slds, it.xv, t);
   else
     rA_i = bA - chunk_mv(it, mS, it.xv, it.act_w);
+  if (!it.owner) rA_i = (T)0;  // and stays so: only w'u needs a select below
   T rB_i = bB;
   if (it.owner) {
     rA[own_pos] = rA_i;
@@ -2016,8 +1992,8 @@ __device__ __forceinline__ void reg_item_pair(const KSys &d, uint32_t rank, T *l
     }
     it.publish_edge(wA_i, 2);
     it.publish_edge(wB_i, 2, VB);
-    it.reduce_publish6(it.owner ? rA_i * uA_i : (T)0, it.owner ? wA_i * uA_i : (T)0, it.owner ? rA_i * rA_i : (T)0,
-                       it.owner ? rB_i * uB_i : (T)0, it.owner ? wB_i * uB_i : (T)0, it.owner ? rB_i * rB_i : (T)0);
+    it.reduce_publish6(rA_i * uA_i, it.owner ? wA_i * uA_i : (T)0, rA_i * rA_i,
+                       rB_i * uB_i, it.owner ? wB_i * uB_i : (T)0, rB_i * rB_i);
     if (!it.gather_pair(wA, wB, 2, tt)) timed_out = true;
   }
   // initial checks of each side (as in reg_item)
@@ -2145,8 +2121,8 @@ __device__ __forceinline__ void reg_item_pair(const KSys &d, uint32_t rank, T *l
     // the neighbours' gather waits for every slot of the current epoch
     it.publish_edge(wA_i, 2);
     it.publish_edge(wB_i, 2, VB);
-    it.reduce_publish6(it.owner ? rA_i * uA_i : (T)0, it.owner ? wA_i * uA_i : (T)0, it.owner ? rA_i * rA_i : (T)0,
-                       it.owner ? rB_i * uB_i : (T)0, it.owner ? wB_i * uB_i : (T)0, it.owner ? rB_i * rB_i : (T)0);
+    it.reduce_publish6(rA_i * uA_i, it.owner ? wA_i * uA_i : (T)0, rA_i * rA_i,
+                       rB_i * uB_i, it.owner ? wB_i * uB_i : (T)0, rB_i * rB_i);
     if (!it.gather_pair(wA, wB, 2, tt)) {
       timed_out = true;
       break;
