@@ -1058,6 +1058,50 @@ __device__ __forceinline__ void write_gS(T *gS, const T *gg, const T *lam, int a
   }
 }
 
+// write_gS for a stateSize known at run time only, V consecutive rows per thread and
+// step (2 for even n).  One workgroup writes a whole system's g_S, so the cost is
+// instructions per element: the place of the next one is stepped, not divided out
+// (FP32 n = 14 N = 64, adjoint alone: 78 -> 63 us).
+template <typename T, int nP, int V>
+__device__ __forceinline__ void write_gS_steps(T *gS, const T *gg, const T *lam, int n, int a, int K, int N,
+                                               int threads) {
+  typedef T vec_t __attribute__((ext_vector_type(V), aligned(sizeof(T))));
+  const int cols = 3 * n, bs = cols * n, step = threads * V;
+  const int dr = step % n, dcol = (step / n) % cols, dk = step / bs;
+  int e = opaque_tid() * V;
+  int k = e / bs, col = (e - k * bs) / n, r = e - k * bs - col * n;
+  for (; e < K * bs; e += step) {
+    const int seg = (col >= n) + (col >= 2 * n), cc = col - seg * n;
+    const int j = a + k - 1 + seg;
+    const int lk = (k + 2) * nP + r, lj = (k + 1 + seg) * nP + cc;
+    const bool in = j >= 0 && j < N;
+    const T lj_v = in ? lam[lj] : (T)0, gj_v = in ? gg[lj] : (T)0;
+    vec_t out;
+#pragma unroll
+    for (int v = 0; v < V; ++v) out[v] = in ? (T)-0.5 * (gg[lk + v] * lj_v + lam[lk + v] * gj_v) : (T)0;
+    *reinterpret_cast<__attribute__((address_space(1))) vec_t *>(gptr(gS) + (size_t)a * bs + e) = out;
+    r += dr;
+    col += dcol;
+    k += dk;
+    if (r >= n) {
+      r -= n;
+      ++col;
+    }
+    if (col >= cols) {
+      col -= cols;
+      ++k;
+    }
+  }
+}
+template <typename T, int nP>
+__device__ __forceinline__ void write_gS_any(T *gS, const T *gg, const T *lam, int n, int a, int K, int N,
+                                             int threads) {
+  if (n & 1)
+    write_gS_steps<T, nP, 1>(gS, gg, lam, n, a, K, N, threads);
+  else
+    write_gS_steps<T, nP, 2>(gS, gg, lam, n, a, K, N, threads);
+}
+
 // PRE: the set-up's HBM reads (initial guess window, first right-hand side)
 // issued together with the matrix chunks, one round trip instead of three (off
 // for the one-pass items of the paired kernel, whose 128-VGPR allocation spills
@@ -1477,7 +1521,9 @@ __device__ __forceinline__ void reg_item(const KSys &d, uint32_t rank, T *lds) {
         break;
       }
     }
-    if (pass == 1) {
+    if (pass == 1 && R::RT) {
+      write_gS_any<T, nP>(static_cast<T *>(d.gS), it.xv, it.lv, n, it.a, K, it.N, stride);
+    } else if (pass == 1) {
       // g_S block rows of the own knots: -1/2 (gg_k lam_j^T + lam_k gg_j^T), j in {k-1,k,k+1}
       // (one element per thread and step: the vectorised write_gS costs this
       // item two VGPRs, and with them the 512-thread FP32 n = 14 instance's
@@ -1747,19 +1793,7 @@ __device__ __forceinline__ void two_rows_item(const KSys &d, float *lds) {
     if (pass == 1) {
       it.put(xv, xa, xb);
       __syncthreads();
-      // g_S block rows, as in reg_item
-      const int bs = 3 * n * n;
-      float *gS = static_cast<float *>(d.gS);
-      for (int e = opaque_tid(); e < N * bs; e += stride) {
-        const int k = e / bs, wq = e - k * bs, col = wq / n, r_ = wq - col * n, seg = col / n, cc = col - seg * n;
-        const int j = k - 1 + seg;
-        float val = 0;
-        if (j >= 0 && j < N) {
-          const int lk = (k + 2) * nP, lj = (j + 2) * nP;
-          val = -0.5f * (xv[lk + r_] * lv[lj + cc] + lv[lk + r_] * xv[lj + cc]);
-        }
-        gptr(gS)[e] = val;
-      }
+      write_gS_any<float, nP>(static_cast<float *>(d.gS), xv, lv, n, 0, N, N, stride);
     }
     __syncthreads();
   }
