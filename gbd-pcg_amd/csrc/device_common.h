@@ -243,6 +243,17 @@ __device__ __forceinline__ T wave_sums(T s0, T s1, T s2) {
   return row_sum(fold<16>(fold<32>(s0, s2), fold<32>(s1, s1)));
 }
 
+// The same for the even and the odd lanes by themselves: sum l of the even lanes in
+// lane 16 l, of the odd ones in lane 16 l + 1.
+template <typename T>
+__device__ __forceinline__ T wave_sums_parity(T s0, T s1, T s2) {
+  T v = fold<16>(fold<32>(s0, s2), fold<32>(s1, s1));
+  v += dpp<kDppQuadXor2>(v);
+  v += dpp<kDppRowRor4>(v);
+  v += dpp<kDppRowRor8>(v);
+  return v;
+}
+
 // Six such sums: sums 0..3 in lanes 16 l, sum 4 in lane 1, sum 5 in lane 33.
 template <typename T>
 __device__ __forceinline__ T wave_sums(T s0, T s1, T s2, T s3, T s4, T s5) {

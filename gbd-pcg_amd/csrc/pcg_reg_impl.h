@@ -398,6 +398,16 @@ struct RegItem : StateSize<NS, (LP > 0)> {
     const T sums = wave_sums(s0, s1, s2, s3, s4, s5);
     const int slot = wave_sums_slot<6>();
     if (slot >= 0) wsum[(threadIdx.x >> 6) * 6 + slot] = sums;
+    publish6(placement);
+  }
+  // The same with side A's partials on even lanes and side B's on odd ones.
+  __device__ __forceinline__ void reduce_publish_sides(T s0, T s1, T s2, bool placement = false) {
+    const T sums = wave_sums_parity(s0, s1, s2);
+    const int l = (int)threadIdx.x & 63;
+    if ((l & 15) < 2 && l < 48) wsum[(threadIdx.x >> 6) * 6 + (l & 1) * 3 + (l >> 4)] = sums;
+    publish6(placement);
+  }
+  __device__ __forceinline__ void publish6(bool placement) {
     __syncthreads();
     const int l = threadIdx.x;
     if (l >= 6) return;
@@ -419,10 +429,21 @@ struct RegItem : StateSize<NS, (LP > 0)> {
   // gather for paired solves: six totals, and the neighbours' `edge` edge knots
   // of vA (first edge block) and vB (second) into their ghost knots.
   __device__ __forceinline__ bool gather_pair(T *vA, T *vB, int edge, T (&tt)[6]) {
+    const bool ok = gather6(vA, vB, edge);
+#pragma unroll
+    for (int l = 0; l < 6; ++l) tt[l] = uniform(tot[l]);
+    return ok;
+  }
+  // The same, each lane taking its side's three totals.
+  __device__ __forceinline__ bool gather_sides(T *vA, T *vB, int edge, int side, T (&tt)[3]) {
+    const bool ok = gather6(vA, vB, edge);
+#pragma unroll
+    for (int l = 0; l < 3; ++l) tt[l] = tot[side * 3 + l];
+    return ok;
+  }
+  __device__ __forceinline__ bool gather6(T *vA, T *vB, int edge) {
     if (G == 1) {
       __syncthreads();
-#pragma unroll
-      for (int l = 0; l < 6; ++l) tt[l] = uniform(tot[l]);
       ++seq;
       return true;
     }
@@ -468,8 +489,6 @@ struct RegItem : StateSize<NS, (LP > 0)> {
     if (!ok) ctl[0] = 1;
     __syncthreads();
     ++seq;
-#pragma unroll
-    for (int l = 0; l < 6; ++l) tt[l] = uniform(tot[l]);
     return __builtin_amdgcn_readfirstlane(ctl[0]) == 0;
   }
 };
@@ -530,7 +549,7 @@ __device__ __forceinline__ void chunk_dot2_lds(const float *__restrict__ plds, i
 // FP64 chunks held in LDS as 16-byte blocks: block b of slot i at double2 index
 // b * SL + i (a wave's reads of one block are contiguous).  Two dot products
 // (the two sides of a paired solve) share each matrix read, each in chunk_dot's
-// order, so the bits are those of chunk_dot; chunk_dot_lds_d is one of them.
+// order, so the bits are those of chunk_dot.
 template <int CW, int SL>
 __device__ __forceinline__ void chunk_dot2_lds_d(const double *__restrict__ mlds, int idx,
                                                  const double *__restrict__ xa, const double *__restrict__ xb,
@@ -555,24 +574,6 @@ __device__ __forceinline__ void chunk_dot2_lds_d(const double *__restrict__ mlds
   }
   ya = (a0 + a1) + (a2 + a3);
   yb = (b0 + b1) + (b2 + b3);
-}
-
-template <int CW, int SL>
-__device__ __forceinline__ double chunk_dot_lds_d(const double *__restrict__ mlds, int idx,
-                                                  const double *__restrict__ x) {
-  double a0 = 0, a1 = 0, a2 = 0, a3 = 0;
-#pragma unroll
-  for (int j = 0; j < CW; j += 4) {
-    const double2 m0 = *reinterpret_cast<const double2 *>(mlds + ((size_t)(j / 2) * SL + idx) * 2);
-    const double2 m1 = *reinterpret_cast<const double2 *>(mlds + ((size_t)(j / 2 + 1) * SL + idx) * 2);
-    const double2 u0 = *reinterpret_cast<const double2 *>(x + j);
-    const double2 u1 = *reinterpret_cast<const double2 *>(x + j + 2);
-    a0 = __builtin_fma(m0.x, u0.x, a0);
-    a1 = __builtin_fma(m0.y, u0.y, a1);
-    a2 = __builtin_fma(m1.x, u1.x, a2);
-    a3 = __builtin_fma(m1.y, u1.y, a3);
-  }
-  return (a0 + a1) + (a2 + a3);
 }
 
 // Sum over the LPR lanes sharing one matrix row; all of them get the same bits.
@@ -949,11 +950,11 @@ __device__ __forceinline__ T row_mv(const RegItem<T, NS, NT, BC, LP, ALONE> &it,
 }
 
 // Whether a paired instance keeps its Pinv chunks in LDS: the FP32 column-chunk
-// instances of n <= 14 at 512 threads, held to 128 VGPRs so that two workgroups
+// instances of 2 < n <= 14 at 512 threads, held to 128 VGPRs so that two workgroups
 // share a CU (with the chunks in registers they spill ~100 B per lane).  The
 // host sizes LDS with the same rule (reg_lds_bytes).
 __host__ __device__ constexpr bool pair_pinv_lds(size_t tsize, int nt, bool bc, int ns) {
-  return tsize == 4 && nt == 512 && !bc && ns <= 14;
+  return tsize == 4 && nt == 512 && !bc && ns > 2 && ns <= 14;
 }
 
 // Whether a paired instance keeps its S chunks in LDS: FP64 rows of n = 28 at
@@ -967,59 +968,31 @@ __host__ __device__ constexpr bool pair_s_lds(size_t tsize, int nt, bool bc, int
 }
 __host__ __device__ constexpr int pair_s_slots(int nt, int ns) { return nt - 2 * 2 * ns; }
 
-// u = Pinv r of both sides of a paired solve: from the register chunk, or from
-// the LDS chunk (PLDS).
-template <bool PLDS, typename T, int NS, int NT, bool BC, int CWR>
-__device__ __forceinline__ void pinv_mv2(const RegItem<T, NS, NT, BC> &it, const T (&mM)[CWR], const T *plds,
-                                         const T *va, const T *vb, int tid, T &ya, T &yb) {
-  using R = RegItem<T, NS, NT, BC>;
-  if constexpr (PLDS) {
-    static_assert(sizeof(T) == 4 && !BC, "LDS-resident Pinv: FP32 column chunks only");
-    T a = 0, b = 0;
-    if (it.act_u) {
-      const int off = it.m * R::nP + it.c * R::CW;
-      chunk_dot2_lds<R::CW, NT>(plds, tid, va + off, vb + off, a, b);
+// A matrix times both sides' vectors (paired items, two lanes per row): each lane's
+// chunk times both windows, from registers or from its slot in LDS (SL > 0: slots of
+// that many lanes, FP32 blocks of four values, FP64 of two); then the pair of lanes
+// swaps halves, which leaves the row's product for side A on the even lane and for
+// side B on the odd one, with the bits of group_sum.
+template <int SL, typename T, int NS, int NT, int CWR>
+__device__ __forceinline__ T sides_mv(const RegItem<T, NS, NT> &it, const T (&mat)[CWR], const T *slot_lds, int slot,
+                                      const T *va, const T *vb, bool act) {
+  using R = RegItem<T, NS, NT>;
+  static_assert(R::LPR == 2, "two lanes per row");
+  T a = 0, b = 0;
+  if (act) {
+    const int off = it.m * R::nP + it.c * R::CW;
+    if constexpr (SL > 0) {
+      if constexpr (sizeof(T) == 4)
+        chunk_dot2_lds<R::CW, SL>(slot_lds, slot, va + off, vb + off, a, b);
+      else
+        chunk_dot2_lds_d<R::CW, SL>(slot_lds, slot, va + off, vb + off, a, b);
+    } else {
+      a = chunk_dot<T, R::CW>(mat, va + off);
+      b = chunk_dot<T, R::CW>(mat, vb + off);
     }
-    ya = group_sum<R::LPR>(a);
-    yb = group_sum<R::LPR>(b);
-  } else {
-    ya = chunk_mv(it, mM, va, it.act_u);
-    yb = chunk_mv(it, mM, vb, it.act_u);
   }
-}
-
-// S times one or two vectors in reg_item_pair: from the register chunk, or
-// from the LDS chunk (SLDS: slot = thread index less the left ghost knot's
-// lanes).
-template <bool SLDS, int SL, typename T, int NS, int NT, bool BC, int CWR>
-__device__ __forceinline__ T s_mv1(const RegItem<T, NS, NT, BC> &it, const T (&mS)[CWR], const T *slds, const T *v,
-                                   int tid) {
-  using R = RegItem<T, NS, NT, BC>;
-  if constexpr (SLDS) {
-    T a = 0;
-    if (it.act_w) a = chunk_dot_lds_d<R::CW, SL>(slds, tid - R::LPR * NS, v + it.m * R::nP + it.c * R::CW);
-    return group_sum<R::LPR>(a);
-  } else {
-    return chunk_mv(it, mS, v, it.act_w);
-  }
-}
-
-template <bool SLDS, int SL, typename T, int NS, int NT, bool BC, int CWR>
-__device__ __forceinline__ void s_mv2(const RegItem<T, NS, NT, BC> &it, const T (&mS)[CWR], const T *slds,
-                                      const T *va, const T *vb, int tid, T &ya, T &yb) {
-  using R = RegItem<T, NS, NT, BC>;
-  if constexpr (SLDS) {
-    T a = 0, b = 0;
-    if (it.act_w) {
-      const int off = it.m * R::nP + it.c * R::CW;
-      chunk_dot2_lds_d<R::CW, SL>(slds, tid - R::LPR * NS, va + off, vb + off, a, b);
-    }
-    ya = group_sum<R::LPR>(a);
-    yb = group_sum<R::LPR>(b);
-  } else {
-    ya = chunk_mv(it, mS, va, it.act_w);
-    yb = chunk_mv(it, mS, vb, it.act_w);
-  }
+  const bool odd = it.c != 0;
+  return (odd ? b : a) + dpp<kDppQuadXor1>(odd ? a : b);
 }
 
 // g_S block rows of a rank's owned knots a..a+K-1 (paired items): -1/2 (gg_k lam_j^T +
@@ -1823,23 +1796,6 @@ template <typename T, int NS, int NT, bool BC>
 __device__ __forceinline__ void reg_item_pair(const KSys &d, uint32_t rank, T *lds) {
   using R = RegItem<T, NS, NT, BC>;
   constexpr int n = R::n, nP = R::nP, CW = R::CW;
-  // Pinv chunks in LDS (the first NT * CW values) for the instances held to
-  // 128 VGPRs; the vectors follow
-  constexpr bool PLDS = pair_pinv_lds(sizeof(T), NT, BC, NS);
-  T *plds = nullptr;
-  if constexpr (PLDS) {
-    plds = lds;
-    lds += (size_t)NT * CW;
-  }
-  // S chunks in LDS (the first pair_s_slots * CW values) for the FP64 n = 28
-  // instance at 512 threads; its vectors need only 8 values of read-ahead
-  constexpr bool SLDS = pair_s_lds(sizeof(T), NT, BC, NS);
-  constexpr int SL = SLDS ? pair_s_slots(NT, NS) : 1;
-  T *slds = nullptr;
-  if constexpr (SLDS) {
-    slds = lds;
-    lds += (size_t)SL * CW;
-  }
   R it;
   it.N = (int)d.N;
   it.G = (int)d.G;
@@ -1848,7 +1804,7 @@ __device__ __forceinline__ void reg_item_pair(const KSys &d, uint32_t rank, T *l
   it.b = (int)knot_begin(rank + 1, d.G, d.N);
   it.K = it.b - it.a;
   const int K = it.K;
-  it.VL = (K + 4) * nP + (BC ? 16 : SLDS ? 8 : R::LPR * CW);
+  it.VL = (K + 4) * nP + (BC ? 16 : R::LPR * CW);
   it.slots = d.slots;
   it.tol = d.tol;
   it.rel = (d.flags & KF_REL) != 0;
@@ -1926,36 +1882,12 @@ __device__ __forceinline__ void reg_item_pair(const KSys &d, uint32_t rank, T *l
     }
   }
 
-  T mM[PLDS ? 1 : CW], mS[SLDS ? 1 : CW];
+  T mM[CW], mS[CW];
   if constexpr (BC) {
     load_row<T, NS, true>(mM, static_cast<const T *>(d.Pinv), kg, row, it.N, it.act_u);
     load_row<T, NS, true>(mS, static_cast<const T *>(d.S), kg, row, it.N, it.act_w);
-  } else if constexpr (SLDS) {
-    // this lane's S chunk through registers into its LDS slot (read back by this
-    // lane only), then its Pinv chunk into registers
-    {
-      T tmp[CW];
-      load_fixed<T, NS, NT, CW>(tmp, static_cast<const T *>(d.S), kg, row, c, it.N, it.act_w);
-      if (it.act_w) {
-        const int si = t - R::LPR * n;
-#pragma unroll
-        for (int j = 0; j < CW; j += 2)
-          *reinterpret_cast<double2 *>(slds + ((size_t)(j / 2) * SL + si) * 2) = make_double2(tmp[j], tmp[j + 1]);
-      }
-    }
-    load_fixed<T, NS, NT, CW>(mM, static_cast<const T *>(d.Pinv), kg, row, c, it.N, it.act_u);
-  } else if constexpr (!PLDS) {
-    load_fixed<T, NS, NT, CW>(mM, static_cast<const T *>(d.Pinv), kg, row, c, it.N, it.act_u);
-    load_fixed<T, NS, NT, CW>(mS, static_cast<const T *>(d.S), kg, row, c, it.N, it.act_w);
   } else {
-    // this lane's Pinv chunk through registers into its LDS slots (read back by
-    // this lane only: no barrier needed between the store and the reads)
-    T tmp[CW];
-    load_fixed<T, NS, NT, CW>(tmp, static_cast<const T *>(d.Pinv), kg, row, c, it.N, it.act_u);
-#pragma unroll
-    for (int j = 0; j < CW; j += 4)
-      *reinterpret_cast<float4 *>(plds + ((size_t)(j / 4) * NT + t) * 4) = make_float4(tmp[j], tmp[j + 1], tmp[j + 2],
-                                                                                        tmp[j + 3]);
+    load_fixed<T, NS, NT, CW>(mM, static_cast<const T *>(d.Pinv), kg, row, c, it.N, it.act_u);
     load_fixed<T, NS, NT, CW>(mS, static_cast<const T *>(d.S), kg, row, c, it.N, it.act_w);
   }
   __syncthreads();
@@ -1975,10 +1907,7 @@ __device__ __forceinline__ void reg_item_pair(const KSys &d, uint32_t rank, T *l
   if (it.owner) xA = it.xv[own_pos];
   // r = rhs - S x (B starts from x = 0: r = g_lambda)
   T rA_i;
-  if constexpr (SLDS)
-    rA_i = bA - s_mv1<SLDS, SL>(it, mS, slds, it.xv, t);
-  else
-    rA_i = bA - chunk_mv(it, mS, it.xv, it.act_w);
+  rA_i = bA - chunk_mv(it, mS, it.xv, it.act_w);
   if (!it.owner) rA_i = (T)0;  // and stays so: only w'u needs a select below
   T rB_i = bB;
   if (it.owner) {
@@ -2007,23 +1936,15 @@ __device__ __forceinline__ void reg_item_pair(const KSys &d, uint32_t rank, T *l
     rgA = it.ghost ? rA[it.gpos] : (T)0;
     rgB = it.ghost ? rB[it.gpos] : (T)0;
     // first u = Pinv r, w = S u of both sides
-    if constexpr (PLDS) {
-      pinv_mv2<PLDS>(it, mM, plds, rA, rB, t, uA_i, uB_i);
-    } else {
-      uA_i = chunk_mv(it, mM, rA, it.act_u);
-      uB_i = chunk_mv(it, mM, rB, it.act_u);
-    }
+    uA_i = chunk_mv(it, mM, rA, it.act_u);
+    uB_i = chunk_mv(it, mM, rB, it.act_u);
     if (it.act_u && c == 0) {
       uA[(m + 1) * nP + row] = uA_i;
       uB[(m + 1) * nP + row] = uB_i;
     }
     __syncthreads();
-    if constexpr (SLDS) {
-      s_mv2<SLDS, SL>(it, mS, slds, uA, uB, t, wA_i, wB_i);
-    } else {
-      wA_i = chunk_mv(it, mS, uA, it.act_w);
-      wB_i = chunk_mv(it, mS, uB, it.act_w);
-    }
+    wA_i = chunk_mv(it, mS, uA, it.act_w);
+    wB_i = chunk_mv(it, mS, uB, it.act_w);
     it.publish_edge(wA_i, 2);
     it.publish_edge(wB_i, 2, VB);
     it.reduce_publish6(rA_i * uA_i, it.owner ? wA_i * uA_i : (T)0, rA_i * rA_i,
@@ -2134,23 +2055,15 @@ __device__ __forceinline__ void reg_item_pair(const KSys &d, uint32_t rank, T *l
       rB[it.gpos] = rgB;
     }
     __syncthreads();
-    if constexpr (PLDS) {
-      pinv_mv2<PLDS>(it, mM, plds, rA, rB, t, uA_i, uB_i);
-    } else {
-      uA_i = chunk_mv(it, mM, rA, it.act_u);
-      uB_i = chunk_mv(it, mM, rB, it.act_u);
-    }
+    uA_i = chunk_mv(it, mM, rA, it.act_u);
+    uB_i = chunk_mv(it, mM, rB, it.act_u);
     if (it.act_u && c == 0) {
       uA[(m + 1) * nP + row] = uA_i;
       uB[(m + 1) * nP + row] = uB_i;
     }
     __syncthreads();
-    if constexpr (SLDS) {
-      s_mv2<SLDS, SL>(it, mS, slds, uA, uB, t, wA_i, wB_i);
-    } else {
-      wA_i = chunk_mv(it, mS, uA, it.act_w);
-      wB_i = chunk_mv(it, mS, uB, it.act_w);
-    }
+    wA_i = chunk_mv(it, mS, uA, it.act_w);
+    wB_i = chunk_mv(it, mS, uB, it.act_w);
     // both edge blocks every exchange (a stopped side's are stale and unused):
     // the neighbours' gather waits for every slot of the current epoch
     it.publish_edge(wA_i, 2);
@@ -2208,6 +2121,279 @@ __device__ __forceinline__ void reg_item_pair(const KSys &d, uint32_t rank, T *l
     res.adj_eta = ao.eta;
     res.adj_rr = ao.rr;
     *d.result = res;
+  }
+  if (timed_out && t == 0 && d.err != nullptr)
+    __hip_atomic_store(d.err, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+// The same for two lanes per row: the even lane of a row works for side A, the odd
+// one for side B.  Both hold a chunk of the row and form their part of both sides'
+// products (sides_mv); everything else of an iteration, which VALU issue bounds,
+// is one instruction stream for the two sides: the vector updates, the reductions
+// (three sums over the lanes of one parity each), the divisions and exit tests.
+// Each side performs the operations of its own solve, in the same order.  Against
+// both sides in every lane, per iteration: 64 systems of n = 14 N = 128 FP32 2.59 us
+// (3.00), FP64 5.58 (6.53), one knot range of n = 28 FP64 without exchange 2.66
+// (3.20), all rounds of 32 systems of n = 28 N = 512 60.8 (65.6).
+template <typename T, int NS, int NT>
+__device__ __forceinline__ void reg_item_sides(const KSys &d, uint32_t rank, T *lds) {
+  using R = RegItem<T, NS, NT>;
+  constexpr int n = R::n, nP = R::nP, CW = R::CW;
+  // matrix chunks in LDS ahead of the vectors: Pinv for the instances held to 128
+  // VGPRs, S for the FP64 n = 28 instance at 512 threads (whose vectors need only 8
+  // values of read-ahead)
+  constexpr bool PLDS = pair_pinv_lds(sizeof(T), NT, false, NS), SLDS = pair_s_lds(sizeof(T), NT, false, NS);
+  constexpr int SLP = PLDS ? NT : 0, SLS = SLDS ? pair_s_slots(NT, NS) : 0;
+  T *mlds = lds;
+  lds += (size_t)(SLP + SLS) * CW;
+  R it;
+  it.N = (int)d.N;
+  it.G = (int)d.G;
+  it.rank = (int)rank;
+  it.a = (int)knot_begin(rank, d.G, d.N);
+  it.b = (int)knot_begin(rank + 1, d.G, d.N);
+  it.K = it.b - it.a;
+  const int K = it.K;
+  it.VL = (K + 4) * nP + (SLDS ? 8 : R::LPR * CW);
+  it.slots = d.slots;
+  it.tol = d.tol;
+  it.rel = (d.flags & KF_REL) != 0;
+  it.xcd = false;
+  it.xcd_ok = (d.flags & KF_NOXCD) == 0;
+  const int t = opaque_tid();
+  it.q = t / R::LPR;
+  it.c = t % R::LPR;
+  it.m = it.q / n;
+  it.row = it.q - it.m * n;
+  it.kg = it.a - 1 + it.m;
+  it.act_u = it.m < K + 2;
+  it.act_w = it.m >= 1 && it.m <= K;
+  it.owner = it.act_w;
+  it.ghost = it.q < 4 * n;
+  it.set_edge_slots();
+  {
+    const int gk = it.q / n, gr = it.q - (it.q / n) * n;
+    const int gj = gk < 2 ? gk : K + gk;
+    it.gpos = gj * nP + gr;
+  }
+  // LDS: r, u, w of each side, lambda and g_gamma windows, 6 partials per wave
+  T *rA = lds, *uA = rA + it.VL, *wA = uA + it.VL;
+  const int vb = 3 * it.VL;  // from a vector of side A to that of side B
+  it.xv = rA + 2 * vb;       // lambda0 window, later g_gamma with ghosts
+  it.lv = it.xv + it.VL;     // lambda with ghosts (for g_S)
+  it.wsum = it.lv + it.VL;
+  it.tot = it.wsum + 6 * R::NWAVES;
+  it.ctl = reinterpret_cast<int *>(it.tot + 8);
+  const int total = (int)(it.tot + 8 - lds);
+
+  const int m = it.m, row = it.row, c = it.c, kg = it.kg;
+  const int own_pos = (m + 1) * nP + row;
+  const int edge_off = c * 4 * n;  // this side's edge block
+  T *rv = rA + c * vb, *uv = uA + c * vb, *wv = wA + c * vb;
+
+  if (t == 0) {
+    const uint32_t ea = (uint32_t)(xload(it.rec(0, it.rank)) >> 32);
+    const uint32_t eb = (uint32_t)(xload(it.rec(1, it.rank)) >> 32);
+    uint32_t base = (ea > eb ? ea : eb) + 1u;
+    if (base > 0xFFF00000u) base = 1u;
+    it.ctl[0] = 0;
+    it.ctl[1] = (int)base;
+  }
+  for (int i = opaque_tid(); i < total; i += NT) lds[i] = (T)0;
+
+  // the set-up's vector reads (initial guess window: (K + 2) n <= NT values, one
+  // per thread; the side's right-hand side) issued with the matrix chunks
+  const T *lam0 = static_cast<const T *>(d.lambda);
+  const int wl = (K + 2) * n;
+  T lam_pre = 0, b_i = 0;
+  int lam_pos = -1;
+  {
+    const int i = opaque_tid();
+    if (i < wl) {
+      const int jj = i / n, e = i - jj * n;
+      const int k = it.a - 1 + jj;
+      if (k >= 0 && k < it.N) {
+        lam_pre = gptr(lam0)[(size_t)k * n + e];
+        lam_pos = (jj + 1) * nP + e;
+      }
+    }
+    if (it.owner) b_i = gptr(static_cast<const T *>(c ? d.glambda : d.gamma))[(size_t)kg * n + row];
+  }
+
+  // a matrix kept in LDS goes there through registers (no barrier: a lane reads its
+  // own chunk only)
+  const int sslot = t - R::LPR * n;  // S: no slots for the ghost knots' lanes
+  T mM[PLDS ? 1 : CW], mS[SLDS ? 1 : CW];
+  if constexpr (SLDS) {
+    T tmp[CW];
+    load_fixed<T, NS, NT, CW>(tmp, static_cast<const T *>(d.S), kg, row, c, it.N, it.act_w);
+    if (it.act_w) {
+#pragma unroll
+      for (int j = 0; j < CW; j += 2)
+        *reinterpret_cast<double2 *>(mlds + ((size_t)(j / 2) * SLS + sslot) * 2) = make_double2(tmp[j], tmp[j + 1]);
+    }
+  }
+  if constexpr (PLDS) {
+    T tmp[CW];
+    load_fixed<T, NS, NT, CW>(tmp, static_cast<const T *>(d.Pinv), kg, row, c, it.N, it.act_u);
+#pragma unroll
+    for (int j = 0; j < CW; j += 4)
+      *reinterpret_cast<float4 *>(mlds + ((size_t)(j / 4) * NT + t) * 4) =
+        make_float4(tmp[j], tmp[j + 1], tmp[j + 2], tmp[j + 3]);
+  } else {
+    load_fixed<T, NS, NT, CW>(mM, static_cast<const T *>(d.Pinv), kg, row, c, it.N, it.act_u);
+  }
+  if constexpr (!SLDS) load_fixed<T, NS, NT, CW>(mS, static_cast<const T *>(d.S), kg, row, c, it.N, it.act_w);
+  __syncthreads();
+  it.base = (uint32_t)it.ctl[1];
+  it.seq = 0;
+  if (lam_pos >= 0) it.xv[lam_pos] = lam_pre;
+  for (int i = opaque_tid() + NT; i < wl; i += NT) {
+    const int jj = i / n, e = i - jj * n;
+    const int k = it.a - 1 + jj;
+    if (k >= 0 && k < it.N) it.xv[(jj + 1) * nP + e] = gptr(lam0)[(size_t)k * n + e];
+  }
+  __syncthreads();
+
+  RegOut out{0, GBDPCG_MAX_ITER, 0.0, 0.0};
+  bool timed_out = false, run = true;
+  T x_i = it.owner && c == 0 ? it.xv[own_pos] : (T)0;
+  // r = rhs - S x (side B starts from x = 0: r = g_lambda); zero on lanes without an
+  // own row, where it stays zero: only w'u needs a select below
+  T r_i;
+  {
+    const T y = sides_mv<SLS>(it, mS, mlds, sslot, it.xv, it.xv, it.act_w);
+    r_i = !it.owner ? (T)0 : c ? b_i : b_i - y;
+  }
+  if (it.owner) rv[own_pos] = r_i;
+  it.publish_edge(r_i, 2, edge_off);
+  it.reduce_publish_sides(it.owner ? b_i * b_i : (T)0, (T)0, (T)0, true);
+  T tt[3];
+  double thr = 0.0;
+  T r_g = 0, p_i = 0, s_i = 0, s_g = 0, eta = 0, alpha = 0, u_i = 0, w_i = 0;
+  T last_eta = 0, last_rr = 0;
+  uint32_t iter = 0;
+  const uint32_t max_iter = d.max_iter;
+  if (!it.gather_sides(rA, rA + vb, 2, c, tt)) {
+    timed_out = true;
+  } else {
+    // placement sums: side A's second and third
+    const double sx = (double)uniform(it.tot[1]), sxx = (double)uniform(it.tot[2]);
+    it.xcd = __builtin_amdgcn_readfirstlane((int)(it.xcd_ok && it.G > 1 && sx * sx == (double)it.G * sxx)) != 0;
+    thr = it.rel ? it.tol * it.tol * (double)tt[0] : it.tol;
+    r_g = it.ghost ? rv[it.gpos] : (T)0;
+    u_i = sides_mv<SLP>(it, mM, mlds, t, rA, rA + vb, it.act_u);
+    if (it.act_u) uv[own_pos] = u_i;
+    __syncthreads();
+    w_i = sides_mv<SLS>(it, mS, mlds, sslot, uA, uA + vb, it.act_w);
+    it.publish_edge(w_i, 2, edge_off);
+    it.reduce_publish_sides(r_i * u_i, it.owner ? w_i * u_i : (T)0, r_i * r_i);
+    if (!it.gather_sides(wA, wA + vb, 2, c, tt)) timed_out = true;
+  }
+  if (!timed_out) {
+    // initial checks (as in reg_item)
+    const T delta = tt[1], rr = tt[2];
+    eta = tt[0];
+    p_i = u_i;
+    s_i = w_i;
+    s_g = it.ghost ? wv[it.gpos] : (T)0;
+    alpha = delta != (T)0 ? eta / delta : (T)0;
+    last_eta = eta;
+    last_rr = rr;
+    if (!finite_d((double)eta) || !finite_d((double)rr)) {
+      out.status = GBDPCG_NONFINITE;
+      run = false;
+    } else if (eta == (T)0) {
+      out.status = rr == (T)0 ? GBDPCG_CONVERGED : GBDPCG_BREAKDOWN;
+      run = false;
+    } else if (delta == (T)0 || !finite_d((double)alpha)) {
+      out.status = GBDPCG_BREAKDOWN;
+      run = false;
+    }
+    if (max_iter == 0) run = false;
+  } else {
+    run = false;
+  }
+  // A stopped side's lanes hold their state and go on forming (unused) products for
+  // the exchange.  Every wave has lanes of both sides, so all of them, and all ranks,
+  // leave the loop together.
+  while (__builtin_amdgcn_ballot_w64(run) != 0) {
+    if (run) {
+      if (it.owner) {
+        x_i = fmaT(alpha, p_i, x_i);
+        r_i = fmaT(-alpha, s_i, r_i);
+      }
+      if (it.ghost) r_g = fmaT(-alpha, s_g, r_g);
+    }
+    if (it.owner) rv[own_pos] = r_i;
+    if (it.ghost) rv[it.gpos] = r_g;
+    __syncthreads();
+    u_i = sides_mv<SLP>(it, mM, mlds, t, rA, rA + vb, it.act_u);
+    if (it.act_u) uv[own_pos] = u_i;
+    __syncthreads();
+    w_i = sides_mv<SLS>(it, mS, mlds, sslot, uA, uA + vb, it.act_w);
+    // a stopped side's edges are stale and unused: the neighbours' gather waits for
+    // every slot of the current epoch
+    it.publish_edge(w_i, 2, edge_off);
+    it.reduce_publish_sides(r_i * u_i, it.owner ? w_i * u_i : (T)0, r_i * r_i);
+    if (!it.gather_sides(wA, wA + vb, 2, c, tt)) {
+      timed_out = true;
+      break;
+    }
+    const T w_g = it.ghost ? wv[it.gpos] : (T)0;
+    // as in reg_item: stop tests and next coefficients first, then one branch
+    const T eta_new = tt[0], rr = tt[2];
+    const bool conv = it.rel ? ((double)rr <= thr) : (__builtin_fabs((double)eta_new) < thr);
+    const bool nonfin = !finite_t(eta_new);
+    const T beta = qdiv(eta_new, eta);
+    const T den = tt[1] - beta * qdiv(eta_new, alpha);
+    const bool brk = den == (T)0 || !finite_t(den);
+    const T alpha_new = qdiv(eta_new, den);
+    if (run) {
+      ++iter;
+      last_eta = eta_new;
+      last_rr = rr;
+      if (conv || nonfin || brk) {
+        out.status = conv ? GBDPCG_CONVERGED : nonfin ? GBDPCG_NONFINITE : GBDPCG_BREAKDOWN;
+        run = false;
+      } else {
+        alpha = alpha_new;
+        eta = eta_new;
+        p_i = fmaT(beta, p_i, u_i);
+        s_i = fmaT(beta, s_i, w_i);
+        s_g = fmaT(beta, s_g, w_g);
+        run = iter < max_iter;
+      }
+    }
+  }
+  if (!timed_out) {
+    // lambda and g_gamma to HBM and, with one ghost knot each side, to LDS
+    if (it.owner) {
+      gptr(static_cast<T *>(c ? d.ggamma : d.lambda))[(size_t)kg * n + row] = x_i;
+      (c ? it.xv : it.lv)[own_pos] = x_i;
+    }
+    it.publish_edge(x_i, 1, c ? 0 : 4 * n);
+    it.reduce_publish_sides((T)0, (T)0, (T)0);
+    if (!it.gather_sides(it.xv, it.lv, 1, c, tt))
+      timed_out = true;
+    else
+      write_gS<T, NS, NT>(static_cast<T *>(d.gS), it.xv, it.lv, it.a, K, it.N);
+  }
+  if (timed_out) out.status = GBDPCG_TIMED_OUT;
+  __syncthreads();
+  if (t < 64) {
+    // side A's outcome is in lane 0, side B's in lane 1
+    const int status = out.status, iters = (int)iter;
+    gbdpcg_result res;
+    res.iters = __builtin_amdgcn_readlane(iters, 0);
+    res.status = __builtin_amdgcn_readlane(status, 0);
+    res.adj_iters = __builtin_amdgcn_readlane(iters, 1);
+    res.adj_status = __builtin_amdgcn_readlane(status, 1);
+    res.eta = (double)read_lane(last_eta, 0);
+    res.rr = (double)read_lane(last_rr, 0);
+    res.adj_eta = (double)read_lane(last_eta, 1);
+    res.adj_rr = (double)read_lane(last_rr, 1);
+    if (rank == 0 && t == 0 && d.result != nullptr) *d.result = res;
   }
   if (timed_out && t == 0 && d.err != nullptr)
     __hip_atomic_store(d.err, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
@@ -2289,11 +2475,14 @@ __global__ void __launch_bounds__(NT) pcg_rowcast_kernel(KSys one, const KSys *_
 }
 
 // Paired forward + adjoint items (fused recurrence, both flags set) go to
-// reg_item_pair, every other item to reg_item.
+// reg_item_sides or reg_item_pair, every other item to reg_item.
 template <typename T, int NS, int NT, bool BC>
 __device__ __forceinline__ void pair_item(const KSys &d, uint32_t rank, T *lds) {
   if ((d.flags & (KF_FWD | KF_ADJ)) == (KF_FWD | KF_ADJ) && (d.flags & KF_FUSED)) {
-    reg_item_pair<T, NS, NT, BC>(d, rank, lds);
+    if constexpr (!BC && RegItem<T, NS, NT>::LPR == 2)
+      reg_item_sides<T, NS, NT>(d, rank, lds);
+    else
+      reg_item_pair<T, NS, NT, BC>(d, rank, lds);
   } else if constexpr (pair_s_lds(sizeof(T), NT, BC, NS)) {
     // instances with S in LDS run paired items only (plans route no other item
     // to them): flag the launch rather than skip the item silently
