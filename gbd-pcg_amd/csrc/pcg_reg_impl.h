@@ -546,36 +546,6 @@ __device__ __forceinline__ void chunk_dot2_lds(const float *__restrict__ plds, i
   yb = (b0 + b1) + (b2 + b3);
 }
 
-// FP64 chunks held in LDS as 16-byte blocks: block b of slot i at double2 index
-// b * SL + i (a wave's reads of one block are contiguous).  Two dot products
-// (the two sides of a paired solve) share each matrix read, each in chunk_dot's
-// order, so the bits are those of chunk_dot.
-template <int CW, int SL>
-__device__ __forceinline__ void chunk_dot2_lds_d(const double *__restrict__ mlds, int idx,
-                                                 const double *__restrict__ xa, const double *__restrict__ xb,
-                                                 double &ya, double &yb) {
-  double a0 = 0, a1 = 0, a2 = 0, a3 = 0, b0 = 0, b1 = 0, b2 = 0, b3 = 0;
-#pragma unroll
-  for (int j = 0; j < CW; j += 4) {
-    const double2 m0 = *reinterpret_cast<const double2 *>(mlds + ((size_t)(j / 2) * SL + idx) * 2);
-    const double2 m1 = *reinterpret_cast<const double2 *>(mlds + ((size_t)(j / 2 + 1) * SL + idx) * 2);
-    const double2 u0 = *reinterpret_cast<const double2 *>(xa + j);
-    const double2 u1 = *reinterpret_cast<const double2 *>(xa + j + 2);
-    const double2 v0 = *reinterpret_cast<const double2 *>(xb + j);
-    const double2 v1 = *reinterpret_cast<const double2 *>(xb + j + 2);
-    a0 = __builtin_fma(m0.x, u0.x, a0);
-    a1 = __builtin_fma(m0.y, u0.y, a1);
-    a2 = __builtin_fma(m1.x, u1.x, a2);
-    a3 = __builtin_fma(m1.y, u1.y, a3);
-    b0 = __builtin_fma(m0.x, v0.x, b0);
-    b1 = __builtin_fma(m0.y, v0.y, b1);
-    b2 = __builtin_fma(m1.x, v1.x, b2);
-    b3 = __builtin_fma(m1.y, v1.y, b3);
-  }
-  ya = (a0 + a1) + (a2 + a3);
-  yb = (b0 + b1) + (b2 + b3);
-}
-
 // Sum over the LPR lanes sharing one matrix row; all of them get the same bits.
 template <int LPR, typename T>
 __device__ __forceinline__ T group_sum(T v) {
@@ -968,31 +938,117 @@ __host__ __device__ constexpr bool pair_s_lds(size_t tsize, int nt, bool bc, int
 }
 __host__ __device__ constexpr int pair_s_slots(int nt, int ns) { return nt - 2 * 2 * ns; }
 
-// A matrix times both sides' vectors (paired items, two lanes per row): each lane's
-// chunk times both windows, from registers or from its slot in LDS (SL > 0: slots of
-// that many lanes, FP32 blocks of four values, FP64 of two); then the pair of lanes
-// swaps halves, which leaves the row's product for side A on the even lane and for
-// side B on the odd one, with the bits of group_sum.
-template <int SL, typename T, int NS, int NT, int CWR>
-__device__ __forceinline__ T sides_mv(const RegItem<T, NS, NT> &it, const T (&mat)[CWR], const T *slot_lds, int slot,
-                                      const T *va, const T *vb, bool act) {
-  using R = RegItem<T, NS, NT>;
-  static_assert(R::LPR == 2, "two lanes per row");
-  T a = 0, b = 0;
-  if (act) {
-    const int off = it.m * R::nP + it.c * R::CW;
-    if constexpr (SL > 0) {
-      if constexpr (sizeof(T) == 4)
-        chunk_dot2_lds<R::CW, SL>(slot_lds, slot, va + off, vb + off, a, b);
-      else
-        chunk_dot2_lds_d<R::CW, SL>(slot_lds, slot, va + off, vb + off, a, b);
+// Paired items on two lanes per row: a quad holds two rows, each lane W columns of the
+// padded row (a quarter, rounded up to an even number) of both, value 2 j + r being
+// row r, column j.  So a lane reads a quarter of each side's window and not half:
+// those reads bound the iteration once VALU issue does not.  Per iteration, against a
+// chunk of its own row per lane: FP64 n = 28, one knot range without exchange, 2.50 us
+// (2.67), FP64 n = 12 N = 100 x100 7.68 (8.53), FP32 n = 14 N = 128 x64 2.46 (2.57).  Where a
+// lane's columns are not whole 16-byte reads (FP32 n = 6 and 12) the chunks stay: n = 12
+// N = 100 x100 4.65 us, 4.80 in quads.
+template <int NS>
+constexpr int quad_cols() {
+  return 2 * ((3 * (int)padded_n(NS) + 7) / 8);
+}
+template <typename T, int NS>
+constexpr bool in_quads() {
+  return quad_cols<NS>() * (int)sizeof(T) % 16 == 0;
+}
+
+// Loads them, both rows (r0, r0 + 1: adjacent in memory) at once; lane i of the quad.
+// Guarded loads for n = 28, as load_guarded, branch-free otherwise.
+template <typename T, int NS>
+__device__ __forceinline__ void load_quad(T (&dst)[2 * quad_cols<NS>()], const T *__restrict__ A, int kg, int r0,
+                                          int i, int N, bool active) {
+  typedef T pair_t __attribute__((ext_vector_type(2), aligned(sizeof(T))));
+  constexpr int n = NS, nP = (int)padded_n(NS), W = quad_cols<NS>();
+  int il = i, rl = r0;
+  asm volatile("" : "+v"(il), "+v"(rl));
+  const bool rowok = active && kg >= 0 && kg < N;
+  const uint32_t base = rowok ? (uint32_t)kg * (uint32_t)(3 * n * n) + (uint32_t)rl : 0u;
+#pragma unroll
+  for (int j = 0; j < W; ++j) {
+    const int col = il * W + j, seg = col / nP, cc = col - seg * nP;
+    const bool ok = rowok && seg < 3 && cc < n && !(kg == 0 && seg == 0) && !(kg == N - 1 && seg == 2);
+    pair_t v = {0, 0};
+    if constexpr (NS > 14) {
+      if (ok) v = load_at<pair_t>(A, 0u, base + (uint32_t)((seg * n + cc) * n));
+      dst[2 * j] = v.x;
+      dst[2 * j + 1] = v.y;
     } else {
-      a = chunk_dot<T, R::CW>(mat, va + off);
-      b = chunk_dot<T, R::CW>(mat, vb + off);
+      v = load_at<pair_t>(A, 0u, ok ? base + (uint32_t)((seg * n + cc) * n) : 0u);
+      dst[2 * j] = ok ? v.x : (T)0;
+      dst[2 * j + 1] = ok ? v.y : (T)0;
     }
   }
+}
+
+// A lane's columns of both rows times both sides' windows (xa, xb: its first column),
+// from registers or from its slot `idx` in LDS (SL > 0: 16-byte block b at block index
+// b * SL + idx, so a wave's reads of one block are contiguous): ya, yb are the partial
+// products of rows 0 and 1.
+template <int SL, typename T, int W, int MW>
+__device__ __forceinline__ void quad_dot2(const T (&mat)[MW], const T *__restrict__ lds, int idx,
+                                          const T *__restrict__ xa, const T *__restrict__ xb, T (&ya)[2], T (&yb)[2]) {
+  constexpr int V = 16 / (int)sizeof(T);
+  static_assert(W % V == 0, "whole 16-byte reads");
+  typedef T block_t __attribute__((ext_vector_type(V)));
+  T a[2][2] = {{0, 0}, {0, 0}}, b[2][2] = {{0, 0}, {0, 0}};
+  block_t mv = {};
+#pragma unroll
+  for (int j0 = 0; j0 < W; j0 += V) {
+    const block_t u = *reinterpret_cast<const block_t *>(xa + j0), v = *reinterpret_cast<const block_t *>(xb + j0);
+#pragma unroll
+    for (int jj = 0; jj < V; ++jj) {
+      const int j = j0 + jj;
+      if constexpr (SL > 0) {
+        if (2 * j % V == 0) mv = *reinterpret_cast<const block_t *>(lds + ((size_t)(2 * j / V) * SL + idx) * V);
+      }
+#pragma unroll
+      for (int r = 0; r < 2; ++r) {
+        T e;
+        if constexpr (SL > 0) e = mv[2 * j % V + r]; else e = mat[2 * j + r];
+        a[r][j % 2] = fmaT(e, u[jj], a[r][j % 2]);
+        b[r][j % 2] = fmaT(e, v[jj], b[r][j % 2]);
+      }
+    }
+  }
+#pragma unroll
+  for (int r = 0; r < 2; ++r) {
+    ya[r] = a[r][0] + a[r][1];
+    yb[r] = b[r][0] + b[r][1];
+  }
+}
+
+// A matrix times both sides' vectors: partial products of the lanes that share a row (a
+// quad: two rows) added up by DPP, so that the even lane of each row ends with its
+// product for side A and the odd one for side B.
+template <int SL, typename T, int NS, int NT, int MW>
+__device__ __forceinline__ T sides_mv(const RegItem<T, NS, NT> &it, const T (&mat)[MW], const T *lds, int idx,
+                                      const T *va, const T *vb, bool act) {
+  using R = RegItem<T, NS, NT>;
+  static_assert(R::LPR == 2 && NS % 2 == 0, "two lanes per row, rows in pairs");
+  T a[2] = {0, 0}, b[2] = {0, 0};
+  if constexpr (!in_quads<T, NS>()) {
+    if (act) {
+      const int off = it.m * R::nP + it.c * R::CW;
+      if constexpr (SL > 0) {
+        chunk_dot2_lds<R::CW, SL>(lds, idx, va + off, vb + off, a[0], b[0]);
+      } else {
+        a[0] = chunk_dot<T, R::CW>(mat, va + off);
+        b[0] = chunk_dot<T, R::CW>(mat, vb + off);
+      }
+    }
+  } else if (act) {
+    const int off = it.m * R::nP + it.i * quad_cols<NS>();
+    quad_dot2<SL, T, quad_cols<NS>()>(mat, lds, idx, va + off, vb + off, a, b);
+  }
   const bool odd = it.c != 0;
-  return (odd ? b : a) + dpp<kDppQuadXor1>(odd ? a : b);
+  if constexpr (!in_quads<T, NS>()) return (odd ? b[0] : a[0]) + dpp<kDppQuadXor1>(odd ? a[0] : b[0]);
+  const bool upper = it.i >= 2;
+  const T pa = (upper ? a[1] : a[0]) + dpp<kDppQuadXor2>(upper ? a[0] : a[1]);
+  const T pb = (upper ? b[1] : b[0]) + dpp<kDppQuadXor2>(upper ? b[0] : b[1]);
+  return (odd ? pb : pa) + dpp<kDppQuadXor1>(odd ? pa : pb);
 }
 
 // g_S block rows of a rank's owned knots a..a+K-1 (paired items): -1/2 (gg_k lam_j^T +
@@ -2127,8 +2183,7 @@ __device__ __forceinline__ void reg_item_pair(const KSys &d, uint32_t rank, T *l
 }
 
 // The same for two lanes per row: the even lane of a row works for side A, the odd
-// one for side B.  Both hold a chunk of the row and form their part of both sides'
-// products (sides_mv); everything else of an iteration, which VALU issue bounds,
+// one for side B.  Both take part in both sides' products (sides_mv); everything else of an iteration, which VALU issue bounds,
 // is one instruction stream for the two sides: the vector updates, the reductions
 // (three sums over the lanes of one parity each), the divisions and exit tests.
 // Each side performs the operations of its own solve, in the same order.  Against
@@ -2163,6 +2218,7 @@ __device__ __forceinline__ void reg_item_sides(const KSys &d, uint32_t rank, T *
   const int t = opaque_tid();
   it.q = t / R::LPR;
   it.c = t % R::LPR;
+  it.i = t & 3;
   it.m = it.q / n;
   it.row = it.q - it.m * n;
   it.kg = it.a - 1 + it.m;
@@ -2221,29 +2277,40 @@ __device__ __forceinline__ void reg_item_sides(const KSys &d, uint32_t rank, T *
   }
 
   // a matrix kept in LDS goes there through registers (no barrier: a lane reads its
-  // own chunk only)
+  // own values only)
+  constexpr int MW = in_quads<T, NS>() ? 2 * quad_cols<NS>() : CW, V = 16 / (int)sizeof(T);
+  static_assert(MW <= CW && MW % V == 0, "LDS slots of CW values, whole blocks");
+  typedef T block_t __attribute__((ext_vector_type(V)));
   const int sslot = t - R::LPR * n;  // S: no slots for the ghost knots' lanes
-  T mM[PLDS ? 1 : CW], mS[SLDS ? 1 : CW];
-  if constexpr (SLDS) {
-    T tmp[CW];
-    load_fixed<T, NS, NT, CW>(tmp, static_cast<const T *>(d.S), kg, row, c, it.N, it.act_w);
-    if (it.act_w) {
+  T mM[PLDS ? 1 : MW], mS[SLDS ? 1 : MW];
+  auto to_lds = [&](const T(&v)[MW], int slots, int slot) {
 #pragma unroll
-      for (int j = 0; j < CW; j += 2)
-        *reinterpret_cast<double2 *>(mlds + ((size_t)(j / 2) * SLS + sslot) * 2) = make_double2(tmp[j], tmp[j + 1]);
+    for (int j = 0; j < MW; j += V) {
+      block_t e;
+#pragma unroll
+      for (int k = 0; k < V; ++k) e[k] = v[j + k];
+      *reinterpret_cast<block_t *>(mlds + ((size_t)(j / V) * slots + slot) * V) = e;
     }
+  };
+  auto load = [&](T(&v)[MW], const void *mat, bool active) {
+    if constexpr (in_quads<T, NS>())
+      load_quad<T, NS>(v, static_cast<const T *>(mat), kg, row - (it.i >> 1), it.i, it.N, active);
+    else
+      load_fixed<T, NS, NT, CW>(v, static_cast<const T *>(mat), kg, row, c, it.N, active);
+  };
+  if constexpr (SLDS) {
+    T tmp[MW];
+    load(tmp, d.S, it.act_w);
+    if (it.act_w) to_lds(tmp, SLS, sslot);
   }
   if constexpr (PLDS) {
-    T tmp[CW];
-    load_fixed<T, NS, NT, CW>(tmp, static_cast<const T *>(d.Pinv), kg, row, c, it.N, it.act_u);
-#pragma unroll
-    for (int j = 0; j < CW; j += 4)
-      *reinterpret_cast<float4 *>(mlds + ((size_t)(j / 4) * NT + t) * 4) =
-        make_float4(tmp[j], tmp[j + 1], tmp[j + 2], tmp[j + 3]);
+    T tmp[MW];
+    load(tmp, d.Pinv, it.act_u);
+    to_lds(tmp, SLP, t);
   } else {
-    load_fixed<T, NS, NT, CW>(mM, static_cast<const T *>(d.Pinv), kg, row, c, it.N, it.act_u);
+    load(mM, d.Pinv, it.act_u);
   }
-  if constexpr (!SLDS) load_fixed<T, NS, NT, CW>(mS, static_cast<const T *>(d.S), kg, row, c, it.N, it.act_w);
+  if constexpr (!SLDS) load(mS, d.S, it.act_w);
   __syncthreads();
   it.base = (uint32_t)it.ctl[1];
   it.seq = 0;
