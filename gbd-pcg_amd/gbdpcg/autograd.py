@@ -47,8 +47,9 @@ class PCGSolve(torch.autograd.Function):
     def backward(ctx, glam):
         S_, P_, lam = ctx.saved_tensors
         n, N, tol, max_iter, exit_mode, recurrence = ctx.cfg
-        gg = torch.zeros_like(lam)
-        gS = torch.zeros_like(S_)
+        # written whole by the adjoint solve (padding blocks of gS included)
+        gg = torch.empty_like(lam)
+        gS = torch.empty_like(S_)
         res = adjoint(S_, None, lam, glam.contiguous(), gg, gS, n, N, P_, forward=False, tol=tol,
                       max_iter=max_iter, exit_mode=exit_mode, recurrence=recurrence)
         _require_converged("adjoint", res.adj_status, res.adj_iters)
