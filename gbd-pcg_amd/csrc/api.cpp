@@ -340,11 +340,20 @@ static int finish_reg_layout(int dtype, uint32_t n, uint32_t N, Layout *c) {
 // threads (one wave per SIMD: every wave runs the uniform scalar work, so fewer
 // waves cost less) with up to 8 knots per workgroup; 512 threads when the knots
 // need it, or when only then do all workgroups fit one XCD (shared L2: XCD-local
-// exchanges).  any: the instances for any stateSize up to 32 instead of the fixed
-// sizes.  Returns GBDPCG_ERR_UNSUPPORTED when the shape does not suit this kernel.
+// exchanges).  Then, where that means fewer workgroups, more knots each: in the row
+// broadcast all that fit, as its waves cost the same with all their rows in use (FP64
+// n = 14 N = 256 1.81 us per iteration, with 8 knots each 2.03; N = 400 2.03, 2.46; n = 12
+// N = 200 reference form 2.55, 2.78), else until there is a workgroup per CU of one XCD
+// (n = 2 N = 510 FP64 1.59 us, 2.87; n = 4 N = 500 FP32 1.28, 1.65; n = 8 N = 300 FP64
+// reference form 2.70, 3.59).  any: the instances for any stateSize up to 32 instead
+// of the fixed sizes.  Returns GBDPCG_ERR_UNSUPPORTED when the shape does not suit
+// this kernel.
 static int plan_single_reg(int dtype, uint32_t n, uint32_t N, uint32_t want_G, uint32_t kcap, Layout *L,
                            int only_nt = 0, bool fused = true, bool bc = false, bool pair = false, bool any = false) {
   if (any ? n > 32 : !reg_supported((int)n, bc) || N < 4) return GBDPCG_ERR_UNSUPPORTED;
+  DeviceInfo di;
+  const int drc = device_info(cur_dev(), &di);
+  if (drc < 0) return drc;
   Layout spread;  // first layout found whose workgroups span several XCDs
   bool have_spread = false;
   for (int nt : {256, 512, 64}) {
@@ -373,6 +382,13 @@ static int plan_single_reg(int dtype, uint32_t n, uint32_t N, uint32_t want_G, u
     const int rc = finish_reg_layout(dtype, n, N, &c);
     if (rc == GBDPCG_ERR_UNSUPPORTED) continue;
     if (rc < 0) return rc;
+    if (!want_G && !kcap) {  // more knots each, as above; which systems are taken is decided by 8
+      const uint32_t one_xcd = std::max(8u, ceil_div(N, (uint32_t)(di.cus / kXcds)));
+      Layout more = c;
+      more.G = std::min(G, ceil_div(N, bc ? kmax : std::min(kmax, one_xcd)));
+      more.stride = 0;
+      if (more.G < G && N / more.G >= 2 && finish_reg_layout(dtype, n, N, &more) == GBDPCG_OK) c = more;
+    }
     if (c.stride == (uint32_t)kXcds) {
       *L = c;
       return GBDPCG_OK;
