@@ -330,7 +330,11 @@ static int finish_reg_layout(int dtype, uint32_t n, uint32_t N, Layout *c) {
                                                                    : alone_lanes(n, N, lpr, nt, (uint32_t)tsize(dtype)) * N * lpr;
     c->block = (int)std::min<uint32_t>((uint32_t)c->nt, ceil_div(lanes, 64) * 64);
   }
-  if (!c->stride) c->stride = c->G <= per_xcd ? (uint32_t)kXcds : 1u;
+  // one XCD up to two and a half workgroups per CU, also where the registers admit
+  // more: beyond, sharing the CUs costs more than exchanging across XCDs (FP32
+  // reference form, one XCD / all: n = 13 N = 512, 74 ranks, 3.6 / 4.3 us per iteration;
+  // n = 28 N = 192, 96 ranks, 4.9 / 4.4; n = 12 N = 1000, 125 ranks, 8.6 / 4.6)
+  if (!c->stride) c->stride = c->G <= std::min(per_xcd, (uint32_t)(di.cus / kXcds) * 5 / 2) ? (uint32_t)kXcds : 1u;
   c->grid = c->G * c->stride;
   return GBDPCG_OK;
 }
@@ -354,7 +358,7 @@ static int plan_single_reg(int dtype, uint32_t n, uint32_t N, uint32_t want_G, u
   DeviceInfo di;
   const int drc = device_info(cur_dev(), &di);
   if (drc < 0) return drc;
-  Layout spread;  // first layout found whose workgroups span several XCDs
+  Layout spread;  // first layout found that does not suit one XCD
   bool have_spread = false;
   for (int nt : {256, 512, 64}) {
     if (only_nt && nt != only_nt) continue;
@@ -389,7 +393,9 @@ static int plan_single_reg(int dtype, uint32_t n, uint32_t N, uint32_t want_G, u
       more.stride = 0;
       if (more.G < G && N / more.G >= 2 && finish_reg_layout(dtype, n, N, &more) == GBDPCG_OK) c = more;
     }
-    if (c.stride == (uint32_t)kXcds) {
+    // one XCD, but not with more than two workgroups to a CU where 512 threads need
+    // fewer (n = 28 N = 160 FP32: 80 ranks 2.6 us per iteration, 20 ranks 2.0)
+    if (c.stride == (uint32_t)kXcds && c.G <= 2 * (uint32_t)(di.cus / kXcds)) {
       *L = c;
       return GBDPCG_OK;
     }

@@ -1,0 +1,64 @@
+"""What the planners choose, by the times of whole calls: a choice that another
+request of the same call beats by a margin is a fault of the planner.
+
+Every call runs a fixed number of iterations (tolerance 0) and is the fastest of
+several timed runs; the margins (10 % where both sides are the same kind of call)
+are several times the spread of such minima and well below the faults they guard
+against (1.2 to 1.7 times)."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def _fastest_us(call, reps=10, tries=7):
+    import torch
+    for _ in range(3):
+        call()
+    best = float("inf")
+    for _ in range(tries):
+        a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+        a.record()
+        for _ in range(reps):
+            call()
+        b.record()
+        b.synchronize()
+        best = min(best, a.elapsed_time(b) / reps * 1e3)
+    return best
+
+
+def _system(n, N, dtype):
+    """Block-tridiagonal, diagonally dominant S and its block-Jacobi preconditioner."""
+    import torch
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(100 * n + N)
+    S = torch.randn(N, 3, n, n, generator=gen, device="cuda", dtype=torch.float64) / (4 * n)
+    S[:, 1] = (S[:, 1] + S[:, 1].mT) / 2 + torch.eye(n, device="cuda", dtype=torch.float64)
+    S[1:, 0] = S[:-1, 2].mT
+    P = torch.zeros_like(S)
+    P[:, 1] = torch.eye(n, device="cuda", dtype=torch.float64)
+    g = torch.randn(N * n, generator=gen, device="cuda", dtype=torch.float64)
+    T = torch.float64 if dtype == np.float64 else torch.float32
+    return S.reshape(-1).to(T), P.reshape(-1).to(T), g.to(T)
+
+
+def _solve_us(n, N, dtype, recurrence, **kw):
+    import torch
+    import gbdpcg
+    S, P, g = _system(n, N, dtype)
+    lam = torch.zeros_like(g)
+
+    def call():
+        lam.zero_()
+        gbdpcg.solve_async(S, g, lam, n, N, P, tol=0.0, max_iter=20, exit_mode=gbdpcg.EXIT_REL_RESID,
+                           recurrence=recurrence, **kw)
+    return _fastest_us(call)
+
+
+@pytest.mark.parametrize("n,N,longer,recurrence", [(28, 160, 220, 1), (28, 192, 220, 1), (12, 850, 1500, 0),
+                                                   (12, 1000, 1500, 1), (14, 550, 900, 1)])
+def test_longer_horizons_are_no_faster(gpu, n, N, longer, recurrence):
+    """FP32: an iteration on `longer` knots does all that one on N knots does.  (Four
+    workgroups of one solve sharing each CU of an XCD made the shorter one slower.)"""
+    short, full = (_solve_us(n, k, np.float32, recurrence) for k in (N, longer))
+    assert short <= 1.1 * full, (short, full)
