@@ -349,8 +349,11 @@ static int finish_reg_layout(int dtype, uint32_t n, uint32_t N, Layout *c) {
 // n = 14 N = 256 1.81 us per iteration, with 8 knots each 2.03; N = 400 2.03, 2.46; n = 12
 // N = 200 reference form 2.55, 2.78), else until there is a workgroup per CU of one XCD
 // (n = 2 N = 510 FP64 1.59 us, 2.87; n = 4 N = 500 FP32 1.28, 1.65; n = 8 N = 300 FP64
-// reference form 2.70, 3.59).  any: the instances for any stateSize up to 32 instead
-// of the fixed sizes.  Returns GBDPCG_ERR_UNSUPPORTED when the shape does not suit
+// reference form 2.70, 3.59).  What suits no single XCD takes the layout of the fewest
+// workgroups, as an exchange costs by its ranks (FP32, 256 / 512 threads: n = 24 N = 1200
+// reference form 12.7 / 4.2 us, n = 28 N = 900 7.3 / 2.8; but FP64 fused n = 29 N = 200
+// 3.9 / 4.5: the 32-column class spills at 512 threads).  any: the instances for any
+// stateSize up to 32 instead of the fixed sizes.  Returns GBDPCG_ERR_UNSUPPORTED when the shape does not suit
 // this kernel.
 static int plan_single_reg(int dtype, uint32_t n, uint32_t N, uint32_t want_G, uint32_t kcap, Layout *L,
                            int only_nt = 0, bool fused = true, bool bc = false, bool pair = false, bool any = false) {
@@ -358,7 +361,7 @@ static int plan_single_reg(int dtype, uint32_t n, uint32_t N, uint32_t want_G, u
   DeviceInfo di;
   const int drc = device_info(cur_dev(), &di);
   if (drc < 0) return drc;
-  Layout spread;  // first layout found that does not suit one XCD
+  Layout spread;  // layout of the fewest workgroups among those that do not suit one XCD
   bool have_spread = false;
   for (int nt : {256, 512, 64}) {
     if (only_nt && nt != only_nt) continue;
@@ -383,23 +386,27 @@ static int plan_single_reg(int dtype, uint32_t n, uint32_t N, uint32_t want_G, u
     if (G < 1 || N / G < 2 || ceil_div(N, G) > kmax || G > (uint32_t)kMaxWgsPerSystem) continue;
     c.G = G;
     c.stride = 0;
-    const int rc = finish_reg_layout(dtype, n, N, &c);
-    if (rc == GBDPCG_ERR_UNSUPPORTED) continue;
-    if (rc < 0) return rc;
-    if (!want_G && !kcap) {  // more knots each, as above; which systems are taken is decided by 8
+    int rc = finish_reg_layout(dtype, n, N, &c);
+    if (rc < 0 && rc != GBDPCG_ERR_UNSUPPORTED) return rc;
+    if (rc < 0 && !any) continue;
+    if (!want_G && !kcap) {  // more knots each, as above; which systems a fixed size takes is decided by 8
       const uint32_t one_xcd = std::max(8u, ceil_div(N, (uint32_t)(di.cus / kXcds)));
       Layout more = c;
       more.G = std::min(G, ceil_div(N, bc ? kmax : std::min(kmax, one_xcd)));
       more.stride = 0;
-      if (more.G < G && N / more.G >= 2 && finish_reg_layout(dtype, n, N, &more) == GBDPCG_OK) c = more;
+      if (more.G < G && N / more.G >= 2 && finish_reg_layout(dtype, n, N, &more) == GBDPCG_OK) {
+        c = more;
+        rc = GBDPCG_OK;
+      }
     }
+    if (rc < 0) continue;
     // one XCD, but not with more than two workgroups to a CU where 512 threads need
     // fewer (n = 28 N = 160 FP32: 80 ranks 2.6 us per iteration, 20 ranks 2.0)
     if (c.stride == (uint32_t)kXcds && c.G <= 2 * (uint32_t)(di.cus / kXcds)) {
       *L = c;
       return GBDPCG_OK;
     }
-    if (!have_spread) {
+    if (!have_spread || (c.G < spread.G && !(any && dtype == GBDPCG_F64 && fused && n > 28))) {
       spread = c;
       have_spread = true;
     }

@@ -62,3 +62,15 @@ def test_longer_horizons_are_no_faster(gpu, n, N, longer, recurrence):
     workgroups of one solve sharing each CU of an XCD made the shorter one slower.)"""
     short, full = (_solve_us(n, k, np.float32, recurrence) for k in (N, longer))
     assert short <= 1.1 * full, (short, full)
+
+
+@pytest.mark.parametrize("dtype,n,N", [(np.float32, 15, 3000), (np.float32, 16, 3000), (np.float32, 24, 1200),
+                                       (np.float32, 20, 2000), (np.float32, 31, 700), (np.float64, 10, 3000),
+                                       (np.float64, 13, 3000), (np.float64, 15, 2000)])
+def test_long_horizons_of_any_size_keep_up_with_lds(gpu, dtype, n, N):
+    """Sizes without instances of their own, more workgroups than one XCD holds,
+    reference recurrence (two exchanges per iteration over all ranks): not slower
+    than the LDS-resident kernel, which has fewer ranks."""
+    import gbdpcg
+    auto, lds = _solve_us(n, N, dtype, 0), _solve_us(n, N, dtype, 0, kernel=gbdpcg.KERNEL_LDS)
+    assert auto <= lds, (auto, lds)
