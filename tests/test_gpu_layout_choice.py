@@ -74,3 +74,10 @@ def test_long_horizons_of_any_size_keep_up_with_lds(gpu, dtype, n, N):
     import gbdpcg
     auto, lds = _solve_us(n, N, dtype, 0), _solve_us(n, N, dtype, 0, kernel=gbdpcg.KERNEL_LDS)
     assert auto <= lds, (auto, lds)
+
+
+@pytest.mark.parametrize("N,recurrence", [(850, 0), (890, 1)])
+def test_row_broadcast_does_not_crowd_one_xcd(gpu, N, recurrence):
+    """FP64 n = 12 in the row broadcast, about 62 workgroups: as above."""
+    short, full = (_solve_us(12, k, np.float64, recurrence) for k in (N, 1000))
+    assert short <= 1.1 * full, (short, full)
