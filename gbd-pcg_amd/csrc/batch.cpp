@@ -226,8 +226,7 @@ int plan_launch(int dtype, const gbdpcg_system_desc *systems, const std::vector<
     set_error("no workgroup fits at %zu B LDS", lds);
     return GBDPCG_ERR_TOO_LARGE;
   }
-  const uint32_t grid = (uint32_t)prop.multiProcessorCount * (uint32_t)occ;
-  const uint32_t per_xcd = grid / kXcds;
+  uint32_t grid = (uint32_t)prop.multiProcessorCount * (uint32_t)occ;
   for (uint32_t i : idx) {
     if (G[i] > grid) {
       set_error("system %u needs %u co-resident workgroups (capacity %u)", i, G[i], grid);
@@ -241,55 +240,80 @@ int plan_launch(int dtype, const gbdpcg_system_desc *systems, const std::vector<
   std::vector<uint32_t> order(idx.size());
   std::iota(order.begin(), order.end(), 0u);
   std::stable_sort(order.begin(), order.end(), [&](uint32_t a, uint32_t b) { return cost[a] > cost[b]; });
-  std::vector<double> free_at(grid, 0.0);
   struct Item {
     double start;
     uint32_t sys, rank;
   };
-  std::vector<std::vector<Item>> lists(grid);
-  std::vector<uint32_t> cand;
+  std::vector<std::vector<Item>> lists;
   double makespan = 0.0;
-  for (uint32_t q : order) {
-    const uint32_t s = idx[q];
-    const uint32_t g = G[s];
-    std::vector<uint32_t> chosen;
-    double start = 0.0;
-    if (g <= per_xcd) {
-      double best = 1e300;
-      for (int x = 0; x < kXcds; ++x) {
-        cand.clear();
-        for (uint32_t j = 0; j < per_xcd; ++j) cand.push_back((uint32_t)x + (uint32_t)kXcds * j);
-        std::stable_sort(cand.begin(), cand.end(), [&](uint32_t a, uint32_t b) { return free_at[a] < free_at[b]; });
-        const double st = free_at[cand[g - 1]];
-        if (st < best) {
-          best = st;
-          chosen.assign(cand.begin(), cand.begin() + g);
+  auto schedule = [&]() {  // on `grid` workgroups; returns the rounds
+    const uint32_t per_xcd = grid / kXcds;
+    std::vector<double> free_at(grid, 0.0);
+    std::vector<uint32_t> cand;
+    lists.assign(grid, {});
+    makespan = 0.0;
+    for (uint32_t q : order) {
+      const uint32_t s = idx[q];
+      const uint32_t g = G[s];
+      std::vector<uint32_t> chosen;
+      double start = 0.0;
+      if (g <= per_xcd) {
+        double best = 1e300;
+        for (int x = 0; x < kXcds; ++x) {
+          cand.clear();
+          for (uint32_t j = 0; j < per_xcd; ++j) cand.push_back((uint32_t)x + (uint32_t)kXcds * j);
+          std::stable_sort(cand.begin(), cand.end(), [&](uint32_t a, uint32_t b) { return free_at[a] < free_at[b]; });
+          const double st = free_at[cand[g - 1]];
+          if (st < best) {
+            best = st;
+            chosen.assign(cand.begin(), cand.begin() + g);
+          }
         }
+        start = best;
+      } else {
+        cand.resize(grid);
+        std::iota(cand.begin(), cand.end(), 0u);
+        std::stable_sort(cand.begin(), cand.end(), [&](uint32_t a, uint32_t b) { return free_at[a] < free_at[b]; });
+        chosen.assign(cand.begin(), cand.begin() + g);
+        start = free_at[cand[g - 1]];
       }
-      start = best;
-    } else {
-      cand.resize(grid);
-      std::iota(cand.begin(), cand.end(), 0u);
-      std::stable_sort(cand.begin(), cand.end(), [&](uint32_t a, uint32_t b) { return free_at[a] < free_at[b]; });
-      chosen.assign(cand.begin(), cand.begin() + g);
-      start = free_at[cand[g - 1]];
+      // ranks in increasing workgroup index (neighbouring ranks stay close)
+      std::sort(chosen.begin(), chosen.end());
+      for (uint32_t r = 0; r < g; ++r) {
+        lists[chosen[r]].push_back({start, s, r});
+        free_at[chosen[r]] = start + cost[q];
+      }
+      makespan = std::max(makespan, start + cost[q]);
     }
-    // ranks in increasing workgroup index (neighbouring ranks stay close)
-    std::sort(chosen.begin(), chosen.end());
-    for (uint32_t r = 0; r < g; ++r) {
-      lists[chosen[r]].push_back({start, s, r});
-      free_at[chosen[r]] = start + cost[q];
-    }
-    makespan = std::max(makespan, start + cost[q]);
+    size_t rounds = 0;
+    for (const auto &l : lists) rounds = std::max(rounds, l.size());
+    return (uint32_t)rounds;
+  };
+  // A workgroup per CU as long as that takes one round and leaves every system its
+  // XCD: the list above fills an XCD before it takes the next, and two workgroups
+  // sharing a CU with others idle cost (FP64, 100 systems of n = 2 N = 33: 50.3 us
+  // with two per CU, 45.0 with one).
+  uint32_t rounds = 0, total_items = 0, widest = 0;
+  const uint32_t cus = (uint32_t)prop.multiProcessorCount;
+  for (uint32_t i : idx) {
+    total_items += G[i];
+    widest = std::max(widest, G[i]);
   }
-  uint32_t rounds = 0, total_items = 0;
-  for (auto &l : lists) {
+  if (L.reg && occ > 1 && total_items <= cus && widest <= cus / kXcds) {
+    grid = cus;
+    rounds = schedule();
+    if (rounds > 1) {
+      grid = cus * (uint32_t)occ;
+      rounds = 0;
+    } else {
+      occ = 1;
+    }
+  }
+  if (rounds == 0) rounds = schedule();
+  for (auto &l : lists)
     std::stable_sort(l.begin(), l.end(), [](const Item &a, const Item &b) {
       return a.start < b.start || (a.start == b.start && a.sys < b.sys);
     });
-    rounds = std::max<uint32_t>(rounds, (uint32_t)l.size());
-    total_items += (uint32_t)l.size();
-  }
   L.item_off = items.size();
   items.resize(items.size() + (size_t)rounds * grid, kNoItem);
   for (uint32_t b = 0; b < grid; ++b)

@@ -81,3 +81,24 @@ def test_row_broadcast_does_not_crowd_one_xcd(gpu, N, recurrence):
     """FP64 n = 12 in the row broadcast, about 62 workgroups: as above."""
     short, full = (_solve_us(12, k, np.float64, recurrence) for k in (N, 1000))
     assert short <= 1.1 * full, (short, full)
+
+
+def test_batches_spread_over_idle_cus(gpu):
+    """100 one-workgroup systems on 256 CUs take no longer than 12 of them (they shared
+    CUs two by two while others were idle)."""
+    import torch
+    import gbdpcg
+    n, N = 2, 33
+    S, P, g = _system(n, N, np.float64)
+
+    def us(count):
+        lam = torch.zeros(count, n * N, device="cuda", dtype=torch.float64)
+        b = gbdpcg.Batch([dict(S=S, Pinv=P, gamma=g, lam=lam[i], n=n, N=N) for i in range(count)], tol=0.0,
+                         max_iter=30, exit_mode=gbdpcg.EXIT_REL_RESID, recurrence=gbdpcg.RECUR_FUSED)
+
+        def call():
+            lam.zero_()
+            b.run()
+        return _fastest_us(call)
+    few, many = us(12), us(100)
+    assert many <= 1.1 * few, (many, few)
