@@ -333,14 +333,16 @@ static int finish_reg_layout(int dtype, uint32_t n, uint32_t N, Layout *c) {
   // one XCD up to two and a half workgroups per CU, also where the registers admit
   // more: beyond, sharing the CUs costs more than exchanging across XCDs (FP32
   // reference form, one XCD / all: n = 28 N = 160, 80 ranks, 4.5 / 4.8 us per iteration;
-  // n = 28 N = 192, 96 ranks, 4.9 / 4.4; n = 12 N = 1000, 125 ranks, 8.6 / 4.6).  Row
-  // broadcast, its waves bound by FP64 issue: little beyond one (n = 12 N = 512, 37 ranks,
+  // n = 28 N = 192, 96 ranks, 4.9 / 4.4; n = 12 N = 1000, 125 ranks, 8.6 / 4.6).  FP64
+  // row broadcast, bound by FP64 issue: little beyond one (n = 12 N = 512, 37 ranks,
   // 3.6 / 3.8; N = 550, 40 ranks, 4.3 / 3.8; N = 850, 61 ranks, 6.6 / 4.1).
   // The any-size instances and rows of n <= 8 share a CU better (n = 13 N = 600, 86 ranks,
   // 4.4 / 4.8; n = 15 N = 550, 92 ranks, 4.8 / 4.9; n = 6 N = 2000, 106 ranks, 5.0 / 4.7),
   // one-wave workgroups (64 threads) best: wherever they fit.
   const uint32_t one_xcd = (uint32_t)(di.cus / kXcds);
-  const uint32_t crowd = c->nt == 64 ? per_xcd : c->bc ? one_xcd * 6 / 5 : one_xcd * (c->any || n <= 8 ? 23 : 20) / 8;
+  const uint32_t crowd = c->nt == 64                      ? per_xcd
+                         : c->bc && dtype == GBDPCG_F64 ? one_xcd * 6 / 5
+                                                        : one_xcd * (c->any || n <= 8 ? 23 : 20) / 8;
   if (!c->stride) c->stride = c->G <= std::min(per_xcd, crowd) ? (uint32_t)kXcds : 1u;
   c->grid = c->G * c->stride;
   return GBDPCG_OK;
