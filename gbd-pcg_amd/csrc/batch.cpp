@@ -511,8 +511,21 @@ int gbdpcg_batch_create(gbdpcg_batch **out, int dtype, const gbdpcg_system_desc 
     // What the LDS-resident kernel takes (its plan decides what is refused and
     // which recurrence a system runs) goes to the register kernel for any
     // stateSize when that holds every system of the launch with the recurrence
-    // asked for: rows in registers, several times the LDS kernel's rate.
-    if (!launches[li].reg) instead(kAnyAll, 512, [](const BatchLaunch &) { return true; });
+    // asked for: rows in registers, several times the LDS kernel's rate.  Not where
+    // small workgroups that exchange (a cap on their knots) then need twice the rounds: up
+    // to 1,500 values per matrix, three of the LDS kernel's share a CU and cost little more
+    // than a register item each (FP64 reference form, 150 systems of n = 2 N = 16, four
+    // knots each: 137 us in one round, 184 in two; n = 6 N = 40, ten knots each, 165 and 205;
+    // but n = 12 N = 16, four knots each, 264 and 225).
+    if (!launches[li].reg) {
+      const uint32_t rounds = launches[li].rounds;
+      bool small = true;
+      for (uint32_t i : mem)
+        small = small && (systems[i].N + G[i] - 1) / G[i] * systems[i].n * 3 * padded_n(systems[i].n) <= 1500;
+      auto keep = [&](const BatchLaunch &R) { return !small || R.rounds < 2 * rounds || R.items == R.systems; };
+      instead(kAnyAll, 512, keep);
+      if (!launches[li].reg && narrow && cfg->threads != 512) instead(kAnyRows, 256, keep);
+    }
     if (!launches[li].reg || !narrow) continue;
     // Systems of one workgroup each have no exchange: worth a change of layout
     // (100 systems of n = 12, N 10..40, FP32: 69 against 99 us on several).

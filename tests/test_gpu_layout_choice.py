@@ -83,22 +83,33 @@ def test_row_broadcast_does_not_crowd_one_xcd(gpu, N, recurrence):
     assert short <= 1.1 * full, (short, full)
 
 
+def _batch_us(n, N, count, dtype, recurrence, **kw):
+    import torch
+    import gbdpcg
+    S, P, g = _system(n, N, dtype)
+    lam = torch.zeros(count, n * N, device="cuda", dtype=g.dtype)
+    b = gbdpcg.Batch([dict(S=S, Pinv=P, gamma=g, lam=lam[i], n=n, N=N) for i in range(count)], tol=0.0, max_iter=30,
+                     exit_mode=gbdpcg.EXIT_REL_RESID, recurrence=recurrence, **kw)
+
+    def call():
+        lam.zero_()
+        b.run()
+    return _fastest_us(call)
+
+
 def test_batches_spread_over_idle_cus(gpu):
     """100 one-workgroup systems on 256 CUs take no longer than 12 of them (they shared
     CUs two by two while others were idle)."""
-    import torch
-    import gbdpcg
-    n, N = 2, 33
-    S, P, g = _system(n, N, np.float64)
-
-    def us(count):
-        lam = torch.zeros(count, n * N, device="cuda", dtype=torch.float64)
-        b = gbdpcg.Batch([dict(S=S, Pinv=P, gamma=g, lam=lam[i], n=n, N=N) for i in range(count)], tol=0.0,
-                         max_iter=30, exit_mode=gbdpcg.EXIT_REL_RESID, recurrence=gbdpcg.RECUR_FUSED)
-
-        def call():
-            lam.zero_()
-            b.run()
-        return _fastest_us(call)
-    few, many = us(12), us(100)
+    few, many = (_batch_us(2, 33, count, np.float64, 1) for count in (12, 100))
     assert many <= 1.1 * few, (many, few)
+
+
+@pytest.mark.parametrize("n,N,cap", [(2, 16, 4), (6, 40, 12)])
+def test_capped_batches_keep_up_with_lds(gpu, n, N, cap):
+    """FP64, reference recurrence, a cap on the knots of a workgroup: the automatic
+    choice is not slower than the LDS-resident kernel under the same cap."""
+    import gbdpcg
+    kw = dict(knots_per_wg=cap)
+    auto, lds = _batch_us(n, N, 150, np.float64, 0, **kw), _batch_us(n, N, 150, np.float64, 0,
+                                                                    kernel=gbdpcg.KERNEL_LDS, **kw)
+    assert auto <= 1.1 * lds, (auto, lds)
