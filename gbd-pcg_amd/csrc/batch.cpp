@@ -539,9 +539,15 @@ int gbdpcg_batch_create(gbdpcg_batch **out, int dtype, const gbdpcg_system_desc 
     // us against 570 (one 512-thread workgroup per CU) and 624 (two of two lanes
     // per row), FP64 1,659 against 2,446; reference form 581 / 782 and 2,272 /
     // 3,821.  With one round the fewer, larger workgroups win (60 systems: 105
-    // against 113, FP64 218 against 292).
+    // against 113, FP64 218 against 292), and so they do where systems that they hold
+    // alone would have to exchange here (1,000 systems of n = 2 N = 254 FP32: 88 us, 215; 600
+    // of n = 14 N = 35 reference form 141, 282): unless they run in one round, the planner's
+    // estimates decide, which are good to a tenth (600 of four sizes n <= 13, N 5..20,
+    // reference form: estimated 8 % slower, 87 us, 106).
     if (launches[li].rounds > 1 && cfg->threads != 512)
-      instead(kAnyRows, 256, [](const BatchLaunch &) { return true; });
+      instead(kAnyRows, 256, [&](const BatchLaunch &R) {
+        return R.rounds == 1 || R.makespan <= 1.1 * launches[li].makespan;
+      });
   }
 
   // device state

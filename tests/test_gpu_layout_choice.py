@@ -113,3 +113,12 @@ def test_capped_batches_keep_up_with_lds(gpu, n, N, cap):
     auto, lds = _batch_us(n, N, 150, np.float64, 0, **kw), _batch_us(n, N, 150, np.float64, 0,
                                                                     kernel=gbdpcg.KERNEL_LDS, **kw)
     assert auto <= 1.1 * lds, (auto, lds)
+
+
+@pytest.mark.parametrize("dtype,n,N,count,recurrence", [(np.float32, 2, 254, 1000, 1), (np.float64, 2, 180, 600, 1),
+                                                        (np.float32, 16, 30, 400, 0), (np.float32, 14, 35, 600, 0)])
+def test_batches_of_several_rounds_keep_up_with_512_threads(gpu, dtype, n, N, count, recurrence):
+    """Systems that one workgroup of 512 threads holds and one of 256 does not: the
+    automatic choice is not slower than the larger workgroups."""
+    auto, wide = (_batch_us(n, N, count, dtype, recurrence, threads=t) for t in (0, 512))
+    assert auto <= 1.1 * wide, (auto, wide)
