@@ -570,7 +570,11 @@ static int choose_layout(int dev, int dtype, uint32_t n, uint32_t N, bool fused,
                          Layout *L, bool pair = false, bool as_pair = false) {
   if (cfg->grid[0] == 0 && cfg->knots_per_wg == 0 && cfg->kernel == GBDPCG_KERNEL_AUTO && cfg->threads == 0) {
     TuneChoice c;
-    if (tune_lookup(single_key(dev, dtype, n, N, fused, cfg->exit_mode), &c) &&
+    // choices are timed on forward solves: an instance for any size, which would run
+    // forward and adjoint one after the other, is none for a paired solve of a size whose
+    // own instances iterate both together (FP32 n = 14 N = 64, 30 iterations: 83 us, 114)
+    const bool together = pair && reg_supported((int)n) && N >= 4;
+    if (tune_lookup(single_key(dev, dtype, n, N, fused, cfg->exit_mode), &c) && !(together && c.a >= kKindAny) &&
         layout_from(dtype, n, N, c.a, (int)c.b, c.c, c.d, L, fused, pair) == GBDPCG_OK)
       return GBDPCG_OK;
   }
