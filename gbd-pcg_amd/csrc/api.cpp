@@ -433,15 +433,13 @@ static int plan_single_reg(int dtype, uint32_t n, uint32_t N, uint32_t want_G, u
 // 1.75 / 2.67, n = 2 N = 30 on one wave 0.19 / 1.13 and 0.23 / 1.99; FP64: n = 6
 // N = 40 0.90 / 1.75 and 1.21 / 2.92, n = 32 N = 8 2.07 / 3.91 reference form).
 // GBDPCG_ERR_UNSUPPORTED when no workgroup holds it.
-// as_pair: a solve whose sums are to be those of the paired forward + adjoint solve
-// of the same system (adjoint-only in FP64): that solve's layout.
-static int plan_one_workgroup(int dtype, uint32_t n, uint32_t N, bool fused, bool pair, bool as_pair, Layout *L) {
+static int plan_one_workgroup(int dtype, uint32_t n, uint32_t N, bool fused, bool pair, Layout *L) {
   if (n > 32 || (fused && N < 2)) return GBDPCG_ERR_UNSUPPORTED;
-  const bool both = (pair || as_pair) && fused && n <= 14 && reg_supported((int)n) && N >= 4;
+  const bool both = pair && fused && n <= 14 && reg_supported((int)n) && N >= 4;
   for (const int set : {(int)kAnyTiny, (int)kAnyRows, (int)kAnyAll, (int)kAnyLong}) {
     const int nt = set == kAnyTiny ? 64 : set == kAnyRows ? 256 : 512;
     Layout c;
-    c.pair = both && pair;
+    c.pair = both;
     // FP64 rows of n = 12 and 14 broadcast by DPP up to N = 14: 1.14 us per fused
     // iteration at N = 14, 1.31 on kAnyRows (reference form 1.46, 1.53)
     c.bc = nt == 256 && dtype == GBDPCG_F64 && N >= 4 && reg_supported((int)n, true) &&
@@ -450,9 +448,7 @@ static int plan_one_workgroup(int dtype, uint32_t n, uint32_t N, bool fused, boo
     c.fused = fused;
     c.nt = nt;
     if (c.any ? !any_supported(n, nt, c.any) : nt == 64) continue;
-    RegVariant v = c.variant();
-    v.pair = both;
-    if (N > reg_max_knots(dtype, n, nt, v, true)) continue;
+    if (N > reg_max_knots(dtype, n, nt, c.variant(), true)) continue;
     // FP64 rows that must be packed (alone_lanes) gain nothing in the fused form:
     // n = 14 N = 36 2.14 us per iteration, 2.04 on several ranks
     if (set == kAnyLong && dtype == GBDPCG_F64 && fused && n > 12 && n < 16 && 16 * N > (uint32_t)nt) continue;
@@ -480,6 +476,19 @@ static uint32_t kind_of(const Layout &L) {
   if (!L.reg) return kKindLds;
   if (L.any) return L.any == kAnyRows ? kKindRows : L.any == kAnyLong ? kKindLong : kKindAny;
   return L.bc ? kKindRowcast : kKindReg;
+}
+
+// Whether the paired forward + adjoint solve of a system runs the row broadcast: FP64
+// rows of n = 12 and 14, on one workgroup (alone) up to 14 knots, on several beyond what
+// one holds in column chunks.  An adjoint solve by itself (as_pair) then takes the same
+// ranks, which gives it that solve's bits (tests/test_gpu_adjoint.py holds them to 1e-12);
+// one workgroup without exchange would be faster up to the 32 or 42 knots it holds (30
+// iterations, with the host's part: n = 12 N = 20 61 us against 82, n = 14 N = 32 80, 85).
+static bool pairs_by_rowcast(int dtype, uint32_t n, uint32_t N, bool fused, bool *alone) {
+  *alone = false;
+  if (dtype != GBDPCG_F64 || !fused || N < 4 || !reg_supported((int)n, true)) return false;
+  *alone = N <= reg_max_knots(dtype, n, 256, RegVariant{true, true});
+  return *alone || N > reg_max_knots(dtype, n, 512, RegVariant{true, false, true}, true);
 }
 
 // Rebuilds a layout from its (kind, threads, workgroups, stride); checks that it
@@ -545,8 +554,10 @@ static int untuned_layout(int dtype, uint32_t n, uint32_t N, bool fused, const g
     if (rc < 0) return rc;
   }
   int rc = GBDPCG_ERR_UNSUPPORTED;
-  if (cfg->kernel == GBDPCG_KERNEL_AUTO && open && req_nt == 0)
-    rc = plan_one_workgroup(dtype, n, N, fused, pair, as_pair, L);
+  bool alone;
+  const bool ranks = as_pair && pairs_by_rowcast(dtype, n, N, fused, &alone) && !alone;
+  if (cfg->kernel == GBDPCG_KERNEL_AUTO && open && req_nt == 0 && !ranks)
+    rc = plan_one_workgroup(dtype, n, N, fused, pair, L);
   if (rc == GBDPCG_ERR_UNSUPPORTED &&
       ((cfg->kernel == GBDPCG_KERNEL_AUTO && dtype == GBDPCG_F64) || cfg->kernel == GBDPCG_KERNEL_ROWCAST))
     rc = plan_single_reg(dtype, n, N, cfg->grid[0], cfg->knots_per_wg, L, req_nt, fused, true, pair);
@@ -572,8 +583,11 @@ static int choose_layout(int dev, int dtype, uint32_t n, uint32_t N, bool fused,
     TuneChoice c;
     // choices are timed on forward solves: an instance for any size, which would run
     // forward and adjoint one after the other, is none for a paired solve of a size whose
-    // own instances iterate both together (FP32 n = 14 N = 64, 30 iterations: 83 us, 114)
-    const bool together = pair && reg_supported((int)n) && N >= 4;
+    // own instances iterate both together (FP32 n = 14 N = 64, 30 iterations: 83 us, 114),
+    // nor for an adjoint solve that goes with one
+    bool alone;
+    const bool together = (pair && reg_supported((int)n) && N >= 4) ||
+                          (as_pair && pairs_by_rowcast(dtype, n, N, fused, &alone));
     if (tune_lookup(single_key(dev, dtype, n, N, fused, cfg->exit_mode), &c) && !(together && c.a >= kKindAny) &&
         layout_from(dtype, n, N, c.a, (int)c.b, c.c, c.d, L, fused, pair) == GBDPCG_OK)
       return GBDPCG_OK;
@@ -712,7 +726,7 @@ static int solve_locked(Workspace *ws, int dtype, uint32_t n, uint32_t N, const 
   if (fused && N < 2) fused = false;  // one knot: the reference recurrence
   // forward + adjoint on a register kernel (n <= 14): both solves in one loop
   bool pair = fused && (flags & KF_FWD) && (flags & KF_ADJ) && n <= 14;
-  // adjoint alone in FP64: the sums, to the last bits, of the paired solve
+  // adjoint alone in FP64: where the row broadcast runs it, the ranks of the paired solve
   const bool as_pair = dtype == GBDPCG_F64 && (flags & (KF_FWD | KF_ADJ)) == KF_ADJ;
   Layout L;
   int rc = cached_layout(ws, dtype, n, N, fused, cfg, &L, pair, as_pair);
