@@ -1210,11 +1210,11 @@ int gbdpcg_tune_single(int dtype, uint32_t n, uint32_t N, const void *d_S, const
     c.knots_per_wg = c.threads = 0;
     rc = untuned_layout(dtype, n, N, fused, &c, &def, false, false);
     if (rc == GBDPCG_ERR_TOO_LARGE && fused && lds_fused_unfit(dtype, n, N)) {
-      // solves of this config run the reference iteration (solve_locked): tune
-      // those layouts, cached under that recurrence's key, which they look up
+      // solves of this config run the reference iteration (solve_locked): the
+      // LDS-resident kernel's layouts of that form are tuned against their untuned one
       fused = false;
       unfit = true;
-      rc = plan_single(dtype, n, N, false, 0, 0, &def);
+      rc = untuned_layout(dtype, n, N, false, &c, &def, false, false);
     }
     if (rc < 0) return rc;
     add(def);
@@ -1223,11 +1223,13 @@ int gbdpcg_tune_single(int dtype, uint32_t n, uint32_t N, const void *d_S, const
   // the config leaves the kernel and the threads per workgroup open (looked up
   // under the recurrence the default plan settled on)
   const bool open_cfg = cfg->kernel == GBDPCG_KERNEL_AUTO && cfg->threads == 0;
-  // a choice already made for this shape (this process, or the cache file) is kept
+  // a choice already made for this shape (this process, or the cache file) is kept.
+  // unfit: what solves look up (the reference form's key), else what was found last time
+  const std::string key = single_key(dev, dtype, n, N, fused, cfg->exit_mode), unfit_key = "unfit-" + key;
   if (open_cfg) {
     TuneChoice c;
     Layout L;
-    if (tune_lookup(single_key(dev, dtype, n, N, fused, cfg->exit_mode), &c) &&
+    if ((tune_lookup(key, &c) || (unfit && tune_lookup(unfit_key, &c))) &&
         layout_from(dtype, n, N, c.a, (int)c.b, c.c, c.d, &L, fused) == GBDPCG_OK) {
       if (report) {
         gbdpcg_tune_report r{};
@@ -1357,20 +1359,24 @@ int gbdpcg_tune_single(int dtype, uint32_t n, uint32_t N, const void *d_S, const
     ++timed;
     const double us = total / trials;
     if (ci == 0) default_us = us;
-    if (us < best_us) {
+    if (us < best_us && !(unfit && L.reg && cands.size() > 1)) {
       best_us = us;
       best = ci;
     }
   }
   cleanup();
-  if (timed == 0) {
+  if (best_us >= 1e300) {
     set_error("gbdpcg_tune_single: no candidate layout completed");
     return GBDPCG_ERR_TIMEOUT;
   }
   const Layout &B = cands[best];
-  if (open_cfg)
-    tune_store(single_key(dev, dtype, n, N, fused, cfg->exit_mode),
-               TuneChoice{kind_of(B), (uint32_t)B.nt, B.G, B.stride});
+  if (open_cfg) {
+    // unfit: solves (plain reference ones share the key) change layout only where that
+    // is faster than the one they take by themselves
+    const TuneChoice c{kind_of(B), (uint32_t)B.nt, B.G, B.stride};
+    if (unfit) tune_store(unfit_key, c);
+    if (!unfit || default_us < 0 || best_us < default_us) tune_store(key, c);
+  }
   if (report) {
     gbdpcg_tune_report r{};
     r.candidates = timed;

@@ -345,7 +345,9 @@ typedef struct gbdpcg_tune_report {
   uint32_t knots_per_wg;   /* chosen cap on knots per workgroup                        */
   uint32_t threads;        /* chosen threads per workgroup                             */
   uint32_t wgs;            /* single solve: chosen workgroups; batch: launch grid      */
-  uint32_t kernel;         /* GBDPCG_KERNEL_LDS, _REGISTER or _ROWCAST                 */
+  uint32_t kernel;         /* GBDPCG_KERNEL_LDS, _REGISTER or _ROWCAST; _REGISTER also for
+                              the instances for any stateSize, which only automatic
+                              solves run                                            */
   double best_us;          /* mean time of one solve / one batch run, chosen layout    */
   double default_us;       /* same for the untuned default layout                      */
 } gbdpcg_tune_report;
@@ -357,7 +359,10 @@ typedef struct gbdpcg_tune_report {
  * threads and kernel automatic.  A choice already cached for the shape is
  * returned without timing (report->from_cache = 1).  With cfg->kernel or
  * cfg->threads set, only the matching candidates are timed and the cache is
- * neither read nor written.  trials = timed runs per candidate (0 = 5). */
+ * neither read nor written.  A fused request that runs the reference iteration (see
+ * GBDPCG_RECUR_FUSED) times the LDS-resident kernel's layouts against the untuned
+ * one: the report names the best of them, and solves take it only where it is the
+ * faster (best_us < default_us).  trials = timed runs per candidate (0 = 5). */
 int gbdpcg_tune_single(int dtype, uint32_t stateSize, uint32_t knotPoints, const void *d_S, const void *d_Pinv,
                        const void *d_gamma, const gbdpcg_config *cfg, uint32_t trials,
                        gbdpcg_tune_report *report);

@@ -122,3 +122,25 @@ def test_batches_of_several_rounds_keep_up_with_512_threads(gpu, dtype, n, N, co
     automatic choice is not slower than the larger workgroups."""
     auto, wide = (_batch_us(n, N, count, dtype, recurrence, threads=t) for t in (0, 512))
     assert auto <= 1.1 * wide, (auto, wide)
+
+
+@pytest.mark.parametrize("n,N", [(29, 25), (27, 9)])
+def test_tuning_a_fused_request_without_a_fused_layout_costs_nothing(gpu, n, N):
+    """FP64 at odd N from n = 25 on runs the reference iteration: after tuning the fused
+    request, it and a plain reference solve take the untuned layout, bit for bit, unless
+    a faster one was found, and neither is slower than before."""
+    import torch
+    import gbdpcg
+    S, P, g = _system(n, N, np.float64)
+    kw = dict(tol=0.0, max_iter=20, exit_mode=gbdpcg.EXIT_REL_RESID)
+
+    def solution(recurrence):
+        lam = torch.zeros_like(g)
+        gbdpcg.solve(S, g, lam, n, N, P, recurrence=recurrence, **kw)
+        return lam
+    before = [(solution(r), _solve_us(n, N, np.float64, r)) for r in (0, 1)]
+    rep = gbdpcg.tune_single(S, g, n, N, P, recurrence=gbdpcg.RECUR_FUSED, **kw)
+    after = [(solution(r), _solve_us(n, N, np.float64, r)) for r in (0, 1)]
+    for (lam0, us0), (lam1, us1) in zip(before, after):
+        assert us1 <= 1.1 * us0, (us1, us0)
+        assert rep["best_us"] < rep["default_us"] or torch.equal(lam0, lam1)
