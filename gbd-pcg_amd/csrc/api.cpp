@@ -426,9 +426,12 @@ static int plan_single_reg(int dtype, uint32_t n, uint32_t N, uint32_t want_G, u
 }
 
 // One workgroup for the whole system, the smallest that holds it: no exchange at
-// all, which is more than the smaller matvecs of several workgroups save at every
-// size that fits (microseconds per iteration, one workgroup against the best of
-// several, fused and reference form; FP32: n = 14 N = 36 1.05 / 1.47 and 1.27 /
+// all, which is more than the smaller matvecs of several workgroups save (17 sizes from
+// n = 2 to 32, five horizons each up to the largest, both precisions and forms, against
+// the layouts of several workgroups: two thirds of their time at the median.  Slower,
+// and taken all the same: FP64 n = 28 up to N = 7, 2 to 4 us per solve against that size's
+// own instance on one workgroup of 256 threads.  Microseconds per iteration, one
+// workgroup against the best of several, fused and reference form; FP32: n = 14 N = 36 1.05 / 1.47 and 1.27 /
 // 2.35, n = 12 N = 42 0.89 / 1.34 and 1.14 / 2.20, n = 32 N = 16 1.51 / 1.89 and
 // 1.75 / 2.67, n = 2 N = 30 on one wave 0.19 / 1.13 and 0.23 / 1.99; FP64: n = 6
 // N = 40 0.90 / 1.75 and 1.21 / 2.92, n = 32 N = 8 2.07 / 3.91 reference form).

@@ -363,14 +363,17 @@ int gbdpcg_batch_create(gbdpcg_batch **out, int dtype, const gbdpcg_system_desc 
   const size_t max_lds = prop.sharedMemPerBlock;
   const size_t budget = lds_budget_bytes ? std::min<size_t>(lds_budget_bytes, max_lds) : max_lds;
 
-  // Kernel choice.  Register-resident rows take the fused recurrence, the
-  // specialised stateSizes and N >= 4; the LDS-resident kernel takes the rest.
-  // By default a plan is one persistent launch: the register kernel when every
-  // system suits it (the runtime-n instance when stateSizes differ), else the
-  // LDS kernel for all.  cfg->batch_split asks for one launch per kernel class
-  // present instead: rows of n <= 14 (their runtime-n instance then needs the
-  // registers of those sizes only: two 512-thread workgroups per CU), rows of
-  // n = 28, and the LDS kernel for systems the register kernels do not take.
+  // Kernel choice.  The fixed sizes' register kernels take the fused recurrence and
+  // N >= 4; the LDS-resident kernel is planned for the rest.  By default a plan is one
+  // persistent launch: those register kernels when every system suits them, else one
+  // for all.  cfg->batch_split asks for one launch per kernel class present instead:
+  // rows of n <= 14, rows of n = 28, and the rest.  An automatic plan then changes
+  // kernel where another is the better one (after plan_launch, below): FP32 mixes of
+  // sizes and whatever the LDS-resident kernel was planned for go to the any-size
+  // instances of one lane per row (kAnyAll), systems of one workgroup each and plans
+  // of several rounds to those of whichever workgroup suits them (kAnyAll, kAnyRows).
+  // Forward + adjoint plans of fixed sizes stay on the paired kernels (FP64 mixes of
+  // n <= 14 on their runtime-n instance).
   const bool reg_cfg = fused_cfg && cfg->kernel != GBDPCG_KERNEL_LDS;
   const bool split = cfg->batch_split != 0;
   std::vector<uint32_t> small, wide, lds_sys;

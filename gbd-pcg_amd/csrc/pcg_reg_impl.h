@@ -1,7 +1,8 @@
 // Register-resident PCG kernels for gfx950: the latency path (templates,
 // instantiated in pcg_reg_kernel.hip (fused recurrence, column chunks),
 // pcg_reg_ref_kernel.hip (reference recurrence), pcg_rowcast_kernel.hip (row
-// broadcast) and pcg_pair_kernel_f32/_f64.hip (forward + adjoint together)).
+// broadcast), pcg_pair_kernel_f32/_f64.hip (forward + adjoint together) and
+// pcg_any_*.hip (any stateSize up to 32, systems of one workgroup)).
 //
 // Same method and exchange protocol as pcg_kernel.hip, with every block row a
 // workgroup owns held in registers instead of LDS.  FUSED: the single-reduction
@@ -1136,8 +1137,9 @@ __device__ __forceinline__ void write_gS_any(T *gS, const T *gg, const T *lam, i
 // for the one-pass items of the paired kernel, whose 128-VGPR allocation spills
 // differently, and runs its batches slower, with it; the paired item issues its
 // own set-up reads together).
-// BF: the matrix chunks loaded branch-free (load_chunk), for the fixed-size
-// instances; the runtime-n instances keep the guarded loads.
+// BF: row broadcast of n <= 14 loads its rows branch-free (load_row); the runtime-n
+// instances, short of registers, keep the guarded loads there.  Column chunks are
+// loaded branch-free in any case, but for n = 28 at 512 threads (load_fixed).
 // LP: lanes per row of the runtime-stateSize items, ALONE: a system's only rank
 // (RegItem).
 template <typename T, int NS, int NT, bool FUSED, bool BC = false, bool PRE = true, bool BF = PRE, int LP = 0,
@@ -1176,7 +1178,8 @@ __device__ __forceinline__ void reg_item(const KSys &d, uint32_t rank, T *lds) {
     const int ln = ALONE ? (int)alone_lanes((uint32_t)n, d.N, R::LPR, NT, sizeof(T)) : n;
     it.m = it.q / ln;
     it.row = it.q - it.m * ln;
-    // no neighbours: no lanes for ghost rows, so it holds two knots more
+    // no neighbours: no lanes for ghost rows (a lone item of an any-size instance so
+    // holds two knots more; the planner gives a fixed size no more than with neighbours)
     if (ALONE || (!R::RT && it.G == 1)) ++it.m;
   }
   it.kg = it.a - 1 + it.m;
@@ -1844,10 +1847,11 @@ __device__ __forceinline__ void two_rows_item(const KSys &d, float *lds) {
 // both flags set).  The two solves share S and Pinv and are independent until
 // g_S is formed, so each iteration runs the two right-hand sides (A: gamma,
 // from lambda0; B: g_lambda, from 0) through the same resident matrices and one
-// exchange carrying both sets of scalars and edges.  Each side performs exactly
-// the operations of its own solve in reg_item, in the same order, and stops on
-// its own exit test; once one side has stopped, the other runs alone (its
-// matvecs and updates are skipped, the exchange continues for the other).
+// exchange carrying both sets of scalars and edges.  Each side performs the
+// operations of its own solve in reg_item, in the row broadcast in the same order (the
+// same bits); chunks and lone items of reg_item group the lanes of a sum otherwise.  A
+// side stops on its own exit test; the other then goes on with both sides' products
+// formed and the stopped one's discarded.
 template <typename T, int NS, int NT, bool BC>
 __device__ __forceinline__ void reg_item_pair(const KSys &d, uint32_t rank, T *lds) {
   using R = RegItem<T, NS, NT, BC>;
@@ -2183,13 +2187,14 @@ __device__ __forceinline__ void reg_item_pair(const KSys &d, uint32_t rank, T *l
 }
 
 // The same for two lanes per row: the even lane of a row works for side A, the odd
-// one for side B.  Both take part in both sides' products (sides_mv); everything else of an iteration, which VALU issue bounds,
-// is one instruction stream for the two sides: the vector updates, the reductions
-// (three sums over the lanes of one parity each), the divisions and exit tests.
-// Each side performs the operations of its own solve, in the same order.  Against
-// both sides in every lane, per iteration: 64 systems of n = 14 N = 128 FP32 2.59 us
-// (3.00), FP64 5.58 (6.53), one knot range of n = 28 FP64 without exchange 2.66
-// (3.20), all rounds of 32 systems of n = 28 N = 512 60.8 (65.6).
+// one for side B.  Both take part in both sides' products (sides_mv); everything else
+// of an iteration, which VALU issue bounds, is one instruction stream for the two
+// sides: the vector updates, the reductions (three sums over the lanes of one parity
+// each), the divisions and exit tests.  Each side runs the recurrence of its own
+// solve; the sums of a row (quads) and of a wave come together in another order than
+// reg_item's.  Against both sides in every lane, per iteration: 64 systems of n = 14
+// N = 128 FP32 2.59 us (3.00), FP64 5.58 (6.53), one knot range of n = 28 FP64 without
+// exchange 2.66 (3.20), all rounds of 32 systems of n = 28 N = 512 60.8 (65.6).
 template <typename T, int NS, int NT>
 __device__ __forceinline__ void reg_item_sides(const KSys &d, uint32_t rank, T *lds) {
   using R = RegItem<T, NS, NT>;
@@ -2515,12 +2520,11 @@ __device__ __forceinline__ void reg_entry(const KSys &one, const KSys *__restric
 }
 
 // Waves per SIMD the column-chunk kernel is compiled for: the FP32 instances
-// for rows of n <= 14 at 512 threads (the specialised ones and the runtime-n
-// one, NS = -1) are held to 128 VGPRs, so that two workgroups share a CU in
-// batch plans and long single solves (the planners count on it).
+// for rows of n <= 14 at 512 threads are held to 128 VGPRs, so that two workgroups
+// share a CU in batch plans and long single solves (the planners count on it).
 template <typename T, int NS, int NT>
 constexpr int reg_waves_per_eu() {
-  return (sizeof(T) == 4 && NT == 512 && NS != 0 && NS <= 14) ? 4 : 1;
+  return (sizeof(T) == 4 && NT == 512 && NS <= 14) ? 4 : 1;
 }
 
 // Register-resident rows, reg_lpr(n) lanes per row, column chunks.
@@ -2619,10 +2623,10 @@ pcg_pair_kernel(KSys one, const KSys *__restrict__ systems,
 // rounded up to 4), any_lpr lanes per row.  Bound by the same chain of on-chip
 // latencies as the fixed sizes; a class costs the multiply-adds and registers of
 // its padding only.  Against the LDS-resident kernel, which ran these sizes (one
-// solve, microseconds per iteration): n = 13 N = 50 FP32 reference form 2.35
+// solve on several workgroups, microseconds per iteration): n = 13 N = 50 FP32 reference form 2.35
 // (4.1), fused 1.61 (2.9), FP64 3.31 (4.2) and 2.15 (3.2); n = 24 N = 60 FP32
 // 2.65 (4.1) and 1.78 (3.5); a batch of 96 systems of ten sizes n <= 31, FP32
-// reference form, 168 us (1,081).  SET names the classes one kernel
+// reference form, 135 us (1,081).  SET names the classes one kernel
 // holds and with them its registers: the tiny and narrow ones serve systems of
 // n <= 8 and n <= 16, the wide one larger ones, kAnyAll batches of mixed sizes.
 template <typename T, int NT, bool FUSED, int SET, bool ALONE>
