@@ -136,6 +136,7 @@ struct Layout {
   bool fused = true;   // its recurrence (the LDS kernel takes it from the flags)
   int nt = 256;        // threads per workgroup
   int block = 0;       // ... of which launched (0: all)
+  uint32_t asked = 0;  // workgroups that the no-allocation scratch is asked for (0: G)
   RegVariant variant() const { return RegVariant{fused, bc, pair, any}; }
 };
 
@@ -372,6 +373,7 @@ static int plan_single_reg(int dtype, uint32_t n, uint32_t N, uint32_t want_G, u
   if (drc < 0) return drc;
   Layout spread;  // layout of the fewest workgroups among those that do not suit one XCD
   bool have_spread = false;
+  uint32_t asked = 0;
   for (int nt : {256, 512, 64}) {
     if (only_nt && nt != only_nt) continue;
     if (nt == 64 && (!bc || !only_nt)) continue;  // one-wave ranks: on request (or tuned)
@@ -398,6 +400,7 @@ static int plan_single_reg(int dtype, uint32_t n, uint32_t N, uint32_t want_G, u
     int rc = finish_reg_layout(dtype, n, N, &c);
     if (rc < 0 && rc != GBDPCG_ERR_UNSUPPORTED) return rc;
     if (rc < 0 && !any) continue;
+    const bool by_eight = rc == GBDPCG_OK;
     if (!want_G && !kcap) {  // more knots each, as above; which systems a fixed size takes is decided by 8
       const uint32_t one_xcd = std::max(8u, ceil_div(N, (uint32_t)(di.cus / kXcds)));
       Layout more = c;
@@ -415,6 +418,13 @@ static int plan_single_reg(int dtype, uint32_t n, uint32_t N, uint32_t want_G, u
       *L = c;
       return GBDPCG_OK;
     }
+    // what the no-allocation scratch takes does not follow the choice made here: it is
+    // asked for the records of the first layout found, a fixed size's also with eight
+    // knots each where that is less
+    if (!have_spread)
+      asked = by_eight ? c.G : (uint32_t)kMaxWgsPerSystem;
+    else if (!any)
+      asked = std::min(asked, G);
     if (!have_spread || (c.G < spread.G && !(any && dtype == GBDPCG_F64 && fused && n > 28))) {
       spread = c;
       have_spread = true;
@@ -422,6 +432,7 @@ static int plan_single_reg(int dtype, uint32_t n, uint32_t N, uint32_t want_G, u
   }
   if (!have_spread) return GBDPCG_ERR_UNSUPPORTED;
   *L = spread;
+  L->asked = std::max(asked, spread.G);
   return GBDPCG_OK;
 }
 
@@ -888,16 +899,21 @@ int solve_on_scratch(int dtype, uint32_t n, uint32_t N, const void *S, const voi
     rc = choose_layout(dev, dtype, n, N, false, cfg, &L, false);
   }
   if (rc < 0) return rc;
-  size_t words = 2 * (size_t)L.G * rec_words(n, (uint32_t)(tsize(dtype) / 4));
-  if (L.any && words > scratch_words - kScratchHeaderWords) {
-    // long horizons: the LDS-resident kernel takes fewer workgroups, hence records
-    rc = plan_single(dtype, n, N, fused, cfg->grid[0], cfg->knots_per_wg, &(L = Layout()));
+  const size_t held = scratch_words - kScratchHeaderWords, per_wg = 2 * rec_words(n, (uint32_t)(tsize(dtype) / 4));
+  uint32_t asked = std::max(L.G, L.asked);
+  if (L.any && asked * per_wg > held) {
+    // long horizons: accepted where the LDS-resident kernel's records fit, on that
+    // kernel if only those do
+    Layout lds;
+    rc = plan_single(dtype, n, N, fused, cfg->grid[0], cfg->knots_per_wg, &lds);
     if (rc < 0) return rc;
-    words = 2 * (size_t)L.G * rec_words(n, (uint32_t)(tsize(dtype) / 4));
+    asked = lds.G;
+    if (L.G * per_wg > held) L = lds;
   }
-  if (words > scratch_words - kScratchHeaderWords) {
+  const size_t words = L.G * per_wg;
+  if (asked * per_wg > held) {
     set_error("n=%u N=%u needs %zu words of exchange records on %u workgroups; the no-allocation scratch holds "
-              "%zu", n, N, words, L.G, scratch_words - kScratchHeaderWords);
+              "%zu", n, N, asked * per_wg, asked, held);
     return GBDPCG_ERR_TOO_LARGE;
   }
   hipStream_t stream = static_cast<hipStream_t>(cfg->stream);

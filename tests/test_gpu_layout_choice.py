@@ -144,3 +144,25 @@ def test_tuning_a_fused_request_without_a_fused_layout_costs_nothing(gpu, n, N):
     for (lam0, us0), (lam1, us1) in zip(before, after):
         assert us1 <= 1.1 * us0, (us1, us0)
         assert rep["best_us"] < rep["default_us"] or torch.equal(lam0, lam1)
+
+
+@pytest.mark.parametrize("n,N,dtype,fits", [
+    (14, 3300, np.float32, True), (14, 3800, np.float32, True), (14, 4000, np.float32, False),
+    (14, 4096, np.float32, False), (28, 900, np.float64, True), (28, 960, np.float64, False),
+    (12, 2000, np.float64, True), (20, 3000, np.float32, True), (24, 480, np.float64, False)])
+def test_what_the_scratch_takes(gpu, n, N, dtype, fits):
+    """The no-allocation solve takes the horizons that its documentation names (n = 14 FP32
+    up to about 3800, n = 28 FP64 up to about 900) and refuses those beyond, whatever
+    layout the planner runs; what it takes has the bits of the ordinary call."""
+    import torch
+    import gbdpcg
+    S, P, g = _system(n, N, dtype)
+    kw = dict(tol=0.0, max_iter=5, exit_mode=gbdpcg.EXIT_REL_RESID, recurrence=gbdpcg.RECUR_FUSED)
+    lam, ref = torch.zeros_like(g), torch.zeros_like(g)
+    if not fits:
+        with pytest.raises(gbdpcg.GbdpcgError, match="scratch"):
+            gbdpcg.solve_noalloc(S, g, lam, n, N, P, **kw)
+        return
+    gbdpcg.solve_noalloc(S, g, lam, n, N, P, **kw)
+    gbdpcg.solve(S, g, ref, n, N, P, **kw)
+    assert torch.equal(lam, ref)
