@@ -136,7 +136,8 @@ struct Layout {
   bool fused = true;   // its recurrence (the LDS kernel takes it from the flags)
   int nt = 256;        // threads per workgroup
   int block = 0;       // ... of which launched (0: all)
-  uint32_t asked = 0;  // workgroups that the no-allocation scratch is asked for (0: G)
+  uint32_t asked = 0;  // workgroups whose records the no-allocation scratch is asked for (0: G;
+                       // kMaxWgsPerSystem: the LDS-resident kernel's)
   RegVariant variant() const { return RegVariant{fused, bc, pair, any}; }
 };
 
@@ -418,13 +419,10 @@ static int plan_single_reg(int dtype, uint32_t n, uint32_t N, uint32_t want_G, u
       *L = c;
       return GBDPCG_OK;
     }
-    // what the no-allocation scratch takes does not follow the choice made here: it is
-    // asked for the records of the first layout found, a fixed size's also with eight
-    // knots each where that is less
-    if (!have_spread)
-      asked = by_eight ? c.G : (uint32_t)kMaxWgsPerSystem;
-    else if (!any)
-      asked = std::min(asked, G);
+    // what the no-allocation scratch takes does not follow the choice made here, nor how
+    // many workgroups the registers let share a CU: it is asked for the records of the
+    // first threads per workgroup whose eight knots each two to a CU hold
+    if (!asked && by_eight && (any || G <= 2 * (uint32_t)di.cus)) asked = have_spread ? G : c.G;
     if (!have_spread || (c.G < spread.G && !(any && dtype == GBDPCG_F64 && fused && n > 28))) {
       spread = c;
       have_spread = true;
@@ -432,7 +430,7 @@ static int plan_single_reg(int dtype, uint32_t n, uint32_t N, uint32_t want_G, u
   }
   if (!have_spread) return GBDPCG_ERR_UNSUPPORTED;
   *L = spread;
-  L->asked = std::max(asked, spread.G);
+  L->asked = asked ? asked : (uint32_t)kMaxWgsPerSystem;
   return GBDPCG_OK;
 }
 
@@ -901,7 +899,7 @@ int solve_on_scratch(int dtype, uint32_t n, uint32_t N, const void *S, const voi
   if (rc < 0) return rc;
   const size_t held = scratch_words - kScratchHeaderWords, per_wg = 2 * rec_words(n, (uint32_t)(tsize(dtype) / 4));
   uint32_t asked = std::max(L.G, L.asked);
-  if (L.any && asked * per_wg > held) {
+  if (asked * per_wg > held && (L.any || L.asked == (uint32_t)kMaxWgsPerSystem)) {
     // long horizons: accepted where the LDS-resident kernel's records fit, on that
     // kernel if only those do
     Layout lds;

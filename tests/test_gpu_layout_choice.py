@@ -149,11 +149,14 @@ def test_tuning_a_fused_request_without_a_fused_layout_costs_nothing(gpu, n, N):
 @pytest.mark.parametrize("n,N,dtype,fits", [
     (14, 3300, np.float32, True), (14, 3800, np.float32, True), (14, 4000, np.float32, False),
     (14, 4096, np.float32, False), (28, 900, np.float64, True), (28, 960, np.float64, False),
-    (12, 2000, np.float64, True), (20, 3000, np.float32, True), (24, 480, np.float64, False)])
+    (12, 2000, np.float64, True), (20, 3000, np.float32, True), (24, 480, np.float64, False),
+    (14, 5166, np.float32, True), (12, 7306, np.float32, True), (28, 1292, np.float32, True)])
 def test_what_the_scratch_takes(gpu, n, N, dtype, fits):
     """The no-allocation solve takes the horizons that its documentation names (n = 14 FP32
     up to about 3800, n = 28 FP64 up to about 900) and refuses those beyond, whatever
-    layout the planner runs; what it takes has the bits of the ordinary call."""
+    layout the planner runs; horizons of which two workgroups to a CU do not hold eight
+    knots each are the LDS-resident kernel's, whose records fit again.  What it takes has
+    the bits of the ordinary call, or of that kernel's where only its records fit."""
     import torch
     import gbdpcg
     S, P, g = _system(n, N, dtype)
@@ -164,5 +167,6 @@ def test_what_the_scratch_takes(gpu, n, N, dtype, fits):
             gbdpcg.solve_noalloc(S, g, lam, n, N, P, **kw)
         return
     gbdpcg.solve_noalloc(S, g, lam, n, N, P, **kw)
-    gbdpcg.solve(S, g, ref, n, N, P, **kw)
+    kernel = gbdpcg.KERNEL_LDS if (n, N) in ((14, 5166), (12, 7306)) else gbdpcg.KERNEL_AUTO
+    gbdpcg.solve(S, g, ref, n, N, P, kernel=kernel, **kw)
     assert torch.equal(lam, ref)
