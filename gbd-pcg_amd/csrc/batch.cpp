@@ -128,8 +128,6 @@ double system_cost(const gbdpcg_system_desc &d, uint32_t G, bool fused, size_t t
   return passes * (iters * (exch + mv) + 2 * exch) + load + 3000.0;
 }
 
-// Paired instances for rows of n = 28 (one lane per row): FP32 at 512 threads,
-// FP64 at 256.
 // Paired instances for rows of n = 28: FP32 at 512 threads; FP64 at 256 (one
 // lane per row) and, for launches whose systems are all forward + adjoint, at
 // 512 (S in LDS; that instance runs paired items only).
